@@ -24,6 +24,7 @@
 
 #include "common.hpp"
 #include "exact.hpp"
+#include "flat_half.hpp"
 #include "select.hpp"
 
 namespace qvh {
@@ -1626,44 +1627,45 @@ __global__ void pack_rows_kernel(const float* __restrict__ src, float* __restric
 /// products and sums while they stay below 2^24).
 __device__ __forceinline__ bool small_integer(float v) { return v == rintf(v) && fabsf(v) <= 16777216.0f; }
 
-/// Squared norm of one padded row (fused chain over dp / 4 float4 chunks) and whether all of its
-/// values are small integers.
-__device__ __forceinline__ float padded_norm(const float* row, uint32_t dp, bool& integral) {
-  const f32x4* p = reinterpret_cast<const f32x4*>(row);
-  float s = 0.0f;
-  bool ok = true;
-  for (uint32_t c = 0; c < dp / 4; ++c) {
-    const f32x4 v = p[c];
-    ok = ok && small_integer(v[0]) && small_integer(v[1]) && small_integer(v[2]) && small_integer(v[3]);
-    s = fmaf(v[0], v[0], s);
-    s = fmaf(v[1], v[1], s);
-    s = fmaf(v[2], v[2], s);
-    s = fmaf(v[3], v[3], s);
-  }
-  integral = ok;
-  return s;
-}
-
-/// out[r] = sum of squares of row r (any order: only the GEMM-form screening uses it). With
-/// `meta`, also folds the rows into the store's bound data: meta[0] = largest squared norm (as
-/// float bits; non-negative floats order like their bits), meta[1] != 0 once a row holds a value
-/// that is not a small integer. One atomic per wave.
-__global__ void row_norms_kernel(const float* __restrict__ rows, float* __restrict__ out, uint64_t n,
-                                 uint32_t dp, uint32_t* __restrict__ meta) {
-  const uint64_t r = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+/// out[r] = sum of squares of row r, summed in double and rounded once (any order: only the GEMM-form
+/// screening uses it), eight lanes per row so that a wave reads whole lines. Folds the rows into the
+/// store's bound data: meta[0] = largest squared norm (as float bits; non-negative floats order
+/// like their bits), meta[1] != 0 once a row holds a value that is not a small integer, meta[2] =
+/// largest magnitude (float bits). One atomic per wave and word.
+__global__ void __launch_bounds__(256) row_norms_kernel(const float* __restrict__ rows, float* __restrict__ out,
+                                                        uint64_t n, uint32_t dp, uint32_t* __restrict__ meta) {
+  const uint64_t r = (static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x) / 8;
+  const uint32_t l = threadIdx.x & 7u;
   bool integral = true;
-  float s = 0.0f;
+  double s = 0.0;
+  float largest = 0.0f;
   if (r < n) {
-    s = padded_norm(rows + r * dp, dp, integral);
-    out[r] = s;
-  }
-  if (meta == nullptr) return;
-  uint32_t top = __float_as_uint(s == s ? s : __builtin_huge_valf());
+    const f32x4* p = reinterpret_cast<const f32x4*>(rows + r * dp);
+    for (uint32_t c = l; c < dp / 4; c += 8) {
+      const f32x4 v = p[c];
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) top = max(top, static_cast<uint32_t>(__shfl_xor(top, off, 64)));
+      for (int i = 0; i < 4; ++i) {
+        integral = integral && small_integer(v[i]);
+        largest = fmaxf(largest, fabsf(v[i]));
+        s = fma(static_cast<double>(v[i]), static_cast<double>(v[i]), s);
+      }
+    }
+  }
+#pragma unroll
+  for (int off = 4; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+  const float n2 = static_cast<float>(s);
+  if (r < n && l == 0) out[r] = n2;
+  uint32_t top = __float_as_uint(n2 == n2 ? n2 : __builtin_huge_valf());
+  uint32_t mag = __float_as_uint(largest);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), off, 64)));
+    mag = max(mag, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mag), off, 64)));
+  }
   const bool all_integral = __ballot(!integral) == 0;
   if ((threadIdx.x & 63) == 0) {
     atomicMax(&meta[0], top);
+    atomicMax(&meta[2], mag);
     if (!all_integral) atomicOr(&meta[1], 1u);
   }
 }
@@ -1684,10 +1686,27 @@ __global__ void row_norms_kernel(const float* __restrict__ rows, float* __restri
 /// and every stored row are small integers and (P + R)^2 <= 2^24: every product, partial sum and
 /// difference of either form is then an integer below 2^24, so both forms are exact.
 /// *any_delta (nullable) is raised when some query's delta is not 0.
+///
+/// With `half` (the scan on the 16-bit matrix unit, flat_half.hip; thr is then set), also the query's
+/// scale into word kHalfScaleWord of its thr words, and a bound of that scan's own. Its value of a
+/// row differs from the true distance by at most, in units of u (P + R)^2 (L2; u (1 + P R) for the
+/// inner product):
+///   2 + 6      the norms (summed in double, rounded once) and the split operands: |lo| <= 2^-11 |x|,
+///              so dropping lo.lo and rounding lo cost 3 x 2^-22 sum |q_i x_i| = 12 u P R, at most
+///              6 u (P + R)^2 doubled; halves below the fp16 range add less than 2;
+///   n/16 + 1   matrix steps on the sum proper, each within 18 u of the sum of its magnitudes (17
+///              addends each truncated at 2^-24 of the largest, one rounding; the steps of the small
+///              products come first and count 2^-10 of that): 1.125 n + 18;
+///   2          the value's way back to a distance;
+/// and the reference's own sum, which adds every term through at most n/32 + 15 roundings
+/// (src/simd/kernels_avx2.cc:35-83: four 8-lane chains, a tree, a tail of up to 7), two of them in
+/// the difference: n/32 + 18. Together below 1.16 n + 50; delta uses 1.25 n + 64. It is 0 under the
+/// condition above if also no stored or query value exceeds 2048 in magnitude: hi then holds every
+/// value, lo is 0, and the sums are exact.
 __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restrict__ src, float* __restrict__ qp,
                                                            uint64_t nq, uint32_t dim, uint32_t dp,
                                                            float* __restrict__ qn, const uint32_t* __restrict__ meta,
-                                                           int l2, float* __restrict__ delta,
+                                                           int l2, int half, float* __restrict__ delta,
                                                            uint32_t* __restrict__ any_delta, uint32_t* __restrict__ fb,
                                                            uint32_t* __restrict__ thr, uint32_t thr_stride) {
   const uint64_t q = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
@@ -1695,28 +1714,42 @@ __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restri
   const uint32_t lane = threadIdx.x & 63u;
   // The search's words for the kernels after this one: the query's shared prune bounds to +inf
   // (ordered bits) and the fallback count to zero.
-  if (thr != nullptr && lane < thr_stride) thr[q * thr_stride + lane] = 0xFF800000u;
+  if (thr != nullptr && lane < thr_stride && !(half && lane == kHalfScaleWord)) {
+    thr[q * thr_stride + lane] = 0xFF800000u;
+  }
   if (fb != nullptr && q == 0 && lane == 0) fb[0] = 0u;
-  float s = 0.0f;
+  double s = 0.0;
+  float largest = 0.0f;
   bool ok = true;
   for (uint32_t c = lane; c < dp; c += 64) {
     const float v = c < dim ? src[q * dim + c] : 0.0f;
     qp[q * dp + c] = v;
-    s = fmaf(v, v, s);
+    s = fma(static_cast<double>(v), static_cast<double>(v), s);
+    largest = fmaxf(largest, fabsf(v));
     ok = ok && small_integer(v);
   }
   if (qn == nullptr) return;
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+  for (int off = 32; off >= 1; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    largest = fmaxf(largest, __shfl_xor(largest, off, 64));
+  }
   const bool integral = __builtin_amdgcn_ballot_w64(!ok) == 0;
   if (lane != 0) return;
-  qn[q] = s;
-  const double P = sqrt(static_cast<double>(s));
+  const float n2 = static_cast<float>(s);
+  qn[q] = n2;
+  if (half) {
+    // L2: the norm step's weight 2^8 s_q / s_x stays within fp16.
+    const float sx = half_scale(__uint_as_float(meta[0])), sq = half_scale(n2);
+    thr[q * thr_stride + kHalfScaleWord] = __float_as_uint(l2 && sq > 128.0f * sx ? 128.0f * sx : sq);
+  }
+  const double P = sqrt(static_cast<double>(n2));
   const double R = sqrt(static_cast<double>(__uint_as_float(meta[0])));
   const double u = 1.0 / 16777216.0;
-  const double coef = (4.0 * dp + 16.0) * u;
+  const double coef = (half ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;
   double d;
-  if (integral && meta[1] == 0 && (P + R) * (P + R) * (1.0 + 1e-12) <= 16777216.0) {
+  if (integral && meta[1] == 0 && (P + R) * (P + R) * (1.0 + 1e-12) <= 16777216.0 &&
+      (!half || (largest <= 2048.0f && __uint_as_float(meta[2]) <= 2048.0f))) {
     d = 0.0;
   } else if (l2) {
     d = coef * (P + R) * (P + R);
@@ -2513,6 +2546,9 @@ int shared_list_length(uint32_t k) {
   return need <= 16 ? 16 : need <= 32 ? 32 : 0;
 }
 
+/// Keys the wide merge takes over all lists.
+uint32_t wide_selection(uint32_t k) { return k + std::max<uint32_t>(16, k / 2); }
+
 /// List length for a batch whose GEMM-form distances are all exact (every query's delta is 0:
 /// small-integer queries against a store of small integers), which needs no margin over k; 0 when
 /// none applies. 1M x 128 integer mixture, k = 10: scan 22.30 -> 21.53 ms, merge 82 -> 65 us (12
@@ -2541,17 +2577,6 @@ void launch_scan_kl(bool l2, int mode, dim3 grid, const ScanArgs& a, hipStream_t
     } else {
       hipLaunchKernelGGL((flat_scan_kernel<DP, KL, false, 0>), grid, dim3(kThreads), 0, s, a);
     }
-  }
-}
-
-template <int DP>
-void launch_scan_dp(int kl, bool l2, int mode, dim3 grid, const ScanArgs& a, hipStream_t s) {
-  if (kl == 10) {
-    launch_scan_kl<DP, 10>(l2, mode, grid, a, s);
-  } else if (kl == 16) {
-    launch_scan_kl<DP, 16>(l2, mode, grid, a, s);
-  } else {
-    launch_scan_kl<DP, 32>(l2, mode, grid, a, s);
   }
 }
 
@@ -2587,21 +2612,21 @@ void launch_scan(uint32_t dp, int kl, dim3 grid, const ScanArgs& a, hipStream_t 
     return;
   }
   switch (dp) {
-    case 16: launch_scan_dp<16>(kl, l2, filter, grid, a, s); break;
-    case 24: launch_scan_dp<24>(kl, l2, filter, grid, a, s); break;
-    case 32: launch_scan_dp<32>(kl, l2, filter, grid, a, s); break;
-    case 40: launch_scan_dp<40>(kl, l2, filter, grid, a, s); break;
-    case 48: launch_scan_dp<48>(kl, l2, filter, grid, a, s); break;
-    case 56: launch_scan_dp<56>(kl, l2, filter, grid, a, s); break;
-    case 64: launch_scan_dp<64>(kl, l2, filter, grid, a, s); break;
-    case 72: launch_scan_dp<72>(kl, l2, filter, grid, a, s); break;
-    case 80: launch_scan_dp<80>(kl, l2, filter, grid, a, s); break;
-    case 88: launch_scan_dp<88>(kl, l2, filter, grid, a, s); break;
-    case 96: launch_scan_dp<96>(kl, l2, filter, grid, a, s); break;
-    case 104: launch_scan_dp<104>(kl, l2, filter, grid, a, s); break;
-    case 112: launch_scan_dp<112>(kl, l2, filter, grid, a, s); break;
-    case 120: launch_scan_dp<120>(kl, l2, filter, grid, a, s); break;
-    case 128: launch_scan_dp<128>(kl, l2, filter, grid, a, s); break;
+    case 16: launch_scan_kl<16, 32>(l2, filter, grid, a, s); break;
+    case 24: launch_scan_kl<24, 32>(l2, filter, grid, a, s); break;
+    case 32: launch_scan_kl<32, 32>(l2, filter, grid, a, s); break;
+    case 40: launch_scan_kl<40, 32>(l2, filter, grid, a, s); break;
+    case 48: launch_scan_kl<48, 32>(l2, filter, grid, a, s); break;
+    case 56: launch_scan_kl<56, 32>(l2, filter, grid, a, s); break;
+    case 64: launch_scan_kl<64, 32>(l2, filter, grid, a, s); break;
+    case 72: launch_scan_kl<72, 32>(l2, filter, grid, a, s); break;
+    case 80: launch_scan_kl<80, 32>(l2, filter, grid, a, s); break;
+    case 88: launch_scan_kl<88, 32>(l2, filter, grid, a, s); break;
+    case 96: launch_scan_kl<96, 32>(l2, filter, grid, a, s); break;
+    case 104: launch_scan_kl<104, 32>(l2, filter, grid, a, s); break;
+    case 112: launch_scan_kl<112, 32>(l2, filter, grid, a, s); break;
+    case 120: launch_scan_kl<120, 32>(l2, filter, grid, a, s); break;
+    case 128: launch_scan_kl<128, 32>(l2, filter, grid, a, s); break;
     default: throw Failure(QVH_EUNSUPPORTED, "flat scan: unsupported padded dimension");
   }
 }
@@ -2646,12 +2671,15 @@ struct qvh_flat {
   uint64_t n = 0, cap = 0;
   DeviceBuffer rows, norms;
   // meta[0]: largest stored squared norm (float bits), meta[1]: nonzero once a stored value is not a
-  // small integer (row_norms_kernel); the inputs of the re-score certificate's bound.
+  // small integer, meta[2]: largest magnitude (row_norms_kernel); the inputs of the re-score
+  // certificate's bound.
   DeviceBuffer meta;
   // Host copy of meta after the last append: every stored value a small integer and every stored
-  // squared norm at most 2^24, so that integer queries re-score with delta = 0.
+  // squared norm at most 2^24, so that integer queries re-score with delta = 0 (on the 16-bit matrix
+  // unit if also no magnitude exceeds 2048).
   bool integral_rows = true;
-  uint32_t h_meta[2] = {0, 0};
+  bool half_integral_rows = true;
+  uint32_t h_meta[4] = {0, 0, 0, 0};
   hipStream_t stream = nullptr;
   std::mutex mu;
   // per-call workspace (grown on demand, serialized by mu)
@@ -2701,6 +2729,10 @@ struct FlatPlan {
   enum Path { kFew, kSplit, kExactOnly, kMfma, kSorted } path = kMfma;
   bool wide = false;
   bool ring = false;  // kMfma: the ring scan (one 32-query group, unfiltered) instead of the MFMA scan
+  // kMfma: the scan on the 16-bit matrix unit (rows up to kHalfMaxDp, up to kHalfMaxSel groups a query).
+  bool half = false;
+  bool pair = false;       // its list layout: two lanes per query
+  uint32_t row_waves = 1;  // and waves per query group
   int kl = 16;
   // List length when every query's distances turn out exact (exact_list_length), or 0: the scan
   // and merge are then launched for both lengths, and the device runs the one that applies.
@@ -2743,6 +2775,34 @@ struct FlatBuffers {
   float* cx = nullptr;
   float* cn = nullptr;
 };
+
+/// Row splits for `qblocks` query blocks over `tiles` row tiles: one work-group per CU at a time, so
+/// the count (1 to 7, or a multiple of 8 for the XCD mapping) is the smallest whose work-groups fill
+/// whole rounds of the CUs to 97%: longer splits start fewer lists and exchange bounds with fewer
+/// others. When no count fills 97% of its rounds, the best fill weighted by parallelism (at least
+/// four rounds when the rows allow) decides, fewer splits on ties. A split keeps at least four
+/// tiles: with fewer rows per split the per-split lists take in most rows.
+uint64_t choose_splits(uint64_t qblocks, uint64_t tiles, uint64_t max_splits, int cus) {
+  const uint64_t cap = std::max<uint64_t>(1, std::min<uint64_t>(tiles / 4, max_splits));
+  uint64_t pick = 1;
+  double best = -1.0;
+  for (uint64_t c = 1; c <= cap; c = c < 8 ? c + 1 : c + 8) {
+    const uint64_t total = qblocks * c;
+    const uint64_t rounds = ceil_div(total, static_cast<uint64_t>(cus));
+    if (static_cast<double>(total) / static_cast<double>(rounds * cus) >= 0.97) return c;
+  }
+  for (uint64_t c = 1; c <= cap; c = c < 8 ? c + 1 : c + 8) {
+    const uint64_t total = qblocks * c;
+    const uint64_t rounds = ceil_div(total, static_cast<uint64_t>(cus));
+    const double fill = static_cast<double>(total) / static_cast<double>(rounds * cus);
+    const double score = fill * std::min(1.0, static_cast<double>(total) / (4.0 * cus));
+    if (score > best + 1e-9) {
+      best = score;
+      pick = c;
+    }
+  }
+  return pick;
+}
 
 /// d_idx (listed admitted rows) is in use when n_idx > 0 or `indexed`.
 FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool indexed, bool filtered, uint64_t n_idx,
@@ -2813,9 +2873,11 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
   p.qn = nq * sizeof(float);
   p.delta = nq * sizeof(float);
   p.kl = p.wide ? 32 : shared_list_length(k);
+  p.half = !ring && f->dp <= kHalfMaxDp && (!p.wide || wide_selection(k) <= kHalfMaxSel);
   // The ring scan takes the margin's lists for integer stores too (exact distances certify with any
   // list length): a second, gated launch of its scan and merge would cost more than it saves.
-  p.kl_exact = !p.wide && !ring && f->integral_rows ? exact_list_length(k) : 0;
+  p.kl_exact =
+      !p.wide && !ring && (p.half ? f->half_integral_rows : f->integral_rows) ? exact_list_length(k) : 0;
   p.qblocks = static_cast<uint32_t>(ceil_div(nq, kQueriesPerBlock));
   p.scan_rows = indexed ? n_idx : f->n;
   if (ring) {
@@ -2828,44 +2890,11 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
     p.nsplit = ceil_div(p.scan_rows, p.rows_per_split);
   } else {
     const uint64_t tiles = std::max<uint64_t>(1, ceil_div(p.scan_rows, kTileRows));
-    // One workgroup per CU at a time: the split count (1 to 7, or a multiple of 8 for the XCD
-    // mapping) is the smallest whose workgroups fill whole rounds of the CUs to 97%: longer splits
-    // start fewer lists and exchange bounds with fewer others. 1M x 128, scan at k = 10 (the earlier
-    // choice, which preferred four rounds, without bound slots above 64 splits -> this one): 512
-    // queries 256 -> 128 splits 1.33 -> 1.18 ms, 1,024 queries 256 -> 64 splits 2.46 -> 2.14 ms,
-    // 2,048 queries 128 -> 32 splits 4.71 -> 4.12 ms, 8,192 queries 32 -> 8 splits 16.04 -> 15.97 ms;
-    // 10,000 queries keep 32 (24 splits: 21.27 ms, 32: 20.22, 40: 22.35). When no count fills 97%
-    // of its rounds, the best fill weighted by parallelism (at least four rounds when the rows
-    // allow) decides, fewer splits on ties. A split keeps at least four tiles: with fewer
-    // rows per split the per-split top-k lists take in most rows (1.18M x 100 cosine with 0.5% of
-    // the ids allowed: 32 splits 0.47 ms, 16 splits 0.37 ms).
-    {
-      const uint64_t cap = std::max<uint64_t>(1, std::min<uint64_t>(tiles / 4, kMaxSplits));
-      double best = -1.0;
-      bool full = false;
-      for (uint64_t c = 1; c <= cap && !full; c = c < 8 ? c + 1 : c + 8) {
-        if (c >= 8 && c % 8) continue;
-        const uint64_t total = p.qblocks * c;
-        const uint64_t rounds = ceil_div(total, static_cast<uint64_t>(cus));
-        const double fill = static_cast<double>(total) / static_cast<double>(rounds * cus);
-        if (fill >= 0.97) {
-          p.nsplit = c;
-          full = true;
-        }
-      }
-      for (uint64_t c = 1; c <= cap && !full; c = c < 8 ? c + 1 : c + 8) {
-        if (c >= 8 && c % 8) continue;
-        const uint64_t total = p.qblocks * c;
-        const uint64_t rounds = ceil_div(total, static_cast<uint64_t>(cus));
-        const double fill = static_cast<double>(total) / static_cast<double>(rounds * cus);
-        const double par = std::min(1.0, static_cast<double>(total) / (4.0 * cus));
-        const double score = fill * par;
-        if (score > best + 1e-9) {
-          best = score;
-          p.nsplit = c;
-        }
-      }
-    }
+    // 1M x 128, scan at k = 10 on the fp32 matrix unit (a choice that preferred four rounds -> this
+    // one): 512 queries 256 -> 128 splits 1.33 -> 1.18 ms, 1,024 queries 256 -> 64 splits 2.46 -> 2.14
+    // ms, 2,048 queries 128 -> 32 splits 4.71 -> 4.12 ms; 10,000 queries keep 32 (24 splits: 21.27 ms,
+    // 32: 20.22, 40: 22.35).
+    p.nsplit = choose_splits(p.qblocks, tiles, kMaxSplits, cus);
     p.rows_per_split = ceil_div(tiles, p.nsplit) * kTileRows;
   }
   const size_t parts = static_cast<size_t>(nq) * 2 * p.nsplit * p.kl;
@@ -2873,6 +2902,20 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
   p.pr = parts * sizeof(uint32_t);
   p.thr = nq * (p.ring ? kRingBoundStride : kScanBoundStride) * sizeof(uint32_t);
   p.fb = (nq + 2) * sizeof(uint32_t);  // count, listed queries, then the launch gate word
+  if (p.half) {
+    // 512 queries per work-group (64 per wave) share a tile's conversion and LDS reads; fewer, two
+    // waves take the halves of each tile for the same queries, up to 128 in 32-query groups (more
+    // waves at work). Lists of 32 leave registers for 32 queries per wave. The partial lists stay
+    // within the size computed above.
+    p.pair = p.kl == 32 || nq <= 128;
+    p.row_waves = nq <= (p.pair ? 128u : 256u) ? 2 : 1;
+    const uint64_t lists = half_lists_per_split(p.pair);
+    const uint64_t tiles = std::max<uint64_t>(1, ceil_div(p.scan_rows, kHalfTileRows));
+    const uint64_t max_splits = std::min<uint64_t>(kHalfMaxLists / lists, 2 * p.nsplit / lists);
+    p.qblocks = static_cast<uint32_t>(ceil_div(nq, half_queries_per_block(p.pair, p.row_waves)));
+    p.nsplit = choose_splits(p.qblocks, tiles, max_splits, cus);
+    p.rows_per_split = ceil_div(tiles, p.nsplit) * kHalfTileRows;
+  }
   // Listed rows are gathered once into a contiguous copy: the scan reads every row once per query
   // block, and through the list each of those reads would be a scattered gather (1.18M x 100
   // cosine, 10% listed, 10,000 queries: 2.97 ms through the list, 2.86 ms on the copy).
@@ -2911,7 +2954,8 @@ FlatBuffers handle_buffers(qvh_flat* f, const FlatPlan& p) {
 /// beforehand) is set when some query's bound is not 0. With thr, also the MFMA scan's words:
 /// thr_stride prune bounds per query in thr and the fallback count in b.fb.
 void flat_prep_queries(qvh_flat* f, const FlatBuffers& b, const float* d_raw, uint64_t nq, hipStream_t s,
-                       uint32_t* any_delta = nullptr, uint32_t* thr = nullptr, uint32_t thr_stride = 0) {
+                       bool half = false, uint32_t* any_delta = nullptr, uint32_t* thr = nullptr,
+                       uint32_t thr_stride = 0) {
   const float* qs = d_raw;
   if (f->metric == QVH_METRIC_COSINE) {  // normalized in a copy
     if (b.stage != d_raw) {
@@ -2921,8 +2965,8 @@ void flat_prep_queries(qvh_flat* f, const FlatBuffers& b, const float* d_raw, ui
     qs = b.stage;
   }
   hipLaunchKernelGGL(prep_queries_kernel, dim3(static_cast<unsigned>(ceil_div(nq, 4))), dim3(256), 0, s, qs, b.q, nq,
-                     f->dim, f->dp, b.qn, f->meta.as<uint32_t>(), f->metric == QVH_METRIC_L2 ? 1 : 0, b.delta,
-                     any_delta, thr != nullptr ? b.fb : nullptr, thr, thr_stride);
+                     f->dim, f->dp, b.qn, f->meta.as<uint32_t>(), f->metric == QVH_METRIC_L2 ? 1 : 0, half ? 1 : 0,
+                     b.delta, any_delta, thr != nullptr ? b.fb : nullptr, thr, thr_stride);
   QVH_HIP(hipGetLastError());
 }
 
@@ -2941,7 +2985,7 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   // prep (its shared bounds, strided for the ring scan, and the fallback count).
   if (gate) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, gate, 1, 0u);
   if (p.path == FlatPlan::kMfma) {
-    flat_prep_queries(f, b, d_queries, nq, s, gate, b.thr, p.ring ? kRingBoundStride : kScanBoundStride);
+    flat_prep_queries(f, b, d_queries, nq, s, p.half, gate, b.thr, p.ring ? kRingBoundStride : kScanBoundStride);
   } else {
     flat_prep_queries(f, b, d_queries, nq, s);
   }
@@ -3068,9 +3112,9 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   a.part_d = b.pd;
   a.part_r = b.pr;
   a.qthr = b.thr;
-  // The wide merge's R = k + max(16, k / 2) keys: up to R = 64 the register scan shares a bound of
-  // rank ceil(R / 2) (1M x 128 integer mixture, 10k queries, k = 32: 28.9 ms with no shared bound).
-  const uint32_t wide_sel = k + std::max<uint32_t>(16, k / 2);
+  // The wide merge's R keys: up to R = 64 the register scan shares a bound of rank ceil(R / 2) (1M x
+  // 128 integer mixture, 10k queries, k = 32: 28.9 ms with no shared bound).
+  const uint32_t wide_sel = wide_selection(k);
   a.share_rank = p.wide && wide_sel <= 64 && f->dp <= static_cast<uint32_t>(kMaxDp) ? (wide_sel + 1) / 2 : 0;
   a.share = !p.wide || a.share_rank != 0 ? 1 : 0;
   a.dp = f->dp;
@@ -3079,8 +3123,35 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   a.rowsplit = nq <= static_cast<uint64_t>(kQueriesPerBlock / 2) && !d_idx && !d_bitmap && f->dp <= kMaxDp ? 1 : 0;
   a.bound_slots = !p.wide && (!a.rowsplit || p.nsplit <= kScanSlotMaxSplits) ? 1 : 0;
   const dim3 sgrid(static_cast<unsigned>(p.qblocks * p.nsplit));
+  HalfScanArgs ha{};
+  if (p.half) {
+    ha.X = a.X;
+    ha.xnorm = a.xnorm;
+    ha.n = a.n;
+    ha.dp = f->dp;
+    ha.Q = a.Q;
+    ha.qnorm = a.qnorm;
+    ha.nq = a.nq;
+    ha.bitmap = a.bitmap;
+    ha.l2 = a.l2;
+    ha.nsplit = a.nsplit;
+    ha.qblocks = a.qblocks;
+    ha.rows_per_split = a.rows_per_split;
+    ha.row_waves = p.row_waves;
+    ha.part_d = a.part_d;
+    ha.part_r = a.part_r;
+    ha.words = a.qthr;
+    ha.share = a.share;
+    ha.share_rank = a.share_rank;
+    ha.bound_slots = p.wide ? 0 : 1;
+    ha.meta = f->meta.as<uint32_t>();
+  }
   auto scan = [&](int kl) {
-    if (p.ring) {
+    if (p.half) {
+      ha.gate = a.gate;
+      ha.gate_want = a.gate_want;
+      launch_half_scan(kl, gate && kl == p.kl_exact ? 1 : 3, p.pair, sgrid, ha, s);
+    } else if (p.ring) {
       launch_ring(f->dp, kl, sgrid, a, s);
     } else {
       launch_scan(f->dp, kl, sgrid, a, s);
@@ -3120,9 +3191,38 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   m.fallback = fb + 1;
   m.nfallback = fb;
   const dim3 mgrid(static_cast<unsigned>(ceil_div(nq, 4)));
-  if (p.wide) {
-    const uint32_t sel_n = k + std::max<uint32_t>(16, k / 2);
-    hipLaunchKernelGGL(flat_merge_wide_kernel, mgrid, dim3(256), 0, s, m, sel_n);
+  if (p.half) {
+    HalfMergeArgs hm{};
+    hm.X = m.X;
+    hm.dim = m.dim;
+    hm.dp = m.dp;
+    hm.n = a.n;
+    hm.Q = m.Q;
+    hm.nq = m.nq;
+    hm.k = k;
+    hm.l2 = m.l2;
+    hm.nlists = static_cast<uint32_t>(half_lists_per_split(p.pair) * p.nsplit);
+    hm.wide = p.wide ? 1 : 0;
+    hm.part_d = m.part_d;
+    hm.part_r = m.part_r;
+    hm.idx = d_idx;
+    hm.bitmap = a.bitmap;
+    hm.out_rows = d_rows;
+    hm.out_dist = d_dist;
+    hm.delta = b.delta;
+    hm.fallback = m.fallback;
+    hm.nfallback = m.nfallback;
+    if (gate) {
+      hm.gate = gate;
+      hm.gate_want = 0;
+      hm.sel = static_cast<uint32_t>(p.kl_exact);
+      launch_half_merge(p.kl_exact, hm, s);
+      hm.gate_want = 1;
+    }
+    hm.sel = p.wide ? wide_sel : static_cast<uint32_t>(p.kl);
+    launch_half_merge(p.kl, hm, s);
+  } else if (p.wide) {
+    hipLaunchKernelGGL(flat_merge_wide_kernel, mgrid, dim3(256), 0, s, m, wide_sel);
   } else {
     if (gate) {  // the merge of the short lists, or (gate set) of the margin's
       m.gate = gate;
@@ -3148,7 +3248,7 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   // query would read every row alone: 1024-d, 500k rows, three uncertified queries took 112 ms),
   // into the scan's partial lists, which the merge has consumed; the rest one work-group each.
   const uint32_t fsplit = fallback_splits(e.n, device_cus(f->device));
-  const size_t part_entries = static_cast<size_t>(nq) * 2 * p.nsplit * p.kl;
+  const size_t part_entries = p.pd / sizeof(float);
   if (k <= 64 && fsplit >= 8 && static_cast<size_t>(kFallbackSplitQueries) * fsplit * k <= part_entries) {
     ExactArgs es = e;
     es.nsplit = fsplit;
@@ -3229,8 +3329,9 @@ qvh_status qvh_flat_create(uint32_t dim, int metric, qvh_flat** out) {
       throw Failure(QVH_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
     try {
-      f->meta.reserve(2 * sizeof(uint32_t));
-      hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, f->stream, f->meta.as<uint32_t>(), 2, 0u);
+      f->meta.reserve(sizeof(f->h_meta));
+      hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, f->stream, f->meta.as<uint32_t>(),
+                         sizeof(f->h_meta) / sizeof(uint32_t), 0u);
       QVH_HIP(hipGetLastError());
       // Created here rather than on the first call from another stream, so that the search
       // without allocation never creates one.
@@ -3319,7 +3420,7 @@ void flat_append(qvh_flat* f, const float* rows, uint64_t n, float* stored_out, 
   const uint64_t total = n * f->dp;
   hipLaunchKernelGGL(pack_rows_kernel, dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0,
                      f->stream, stage, dst, n, f->dim, f->dp);
-  hipLaunchKernelGGL(row_norms_kernel, dim3(static_cast<unsigned>(ceil_div(n, 256))), dim3(256), 0,
+  hipLaunchKernelGGL(row_norms_kernel, dim3(static_cast<unsigned>(ceil_div(n, 32))), dim3(256), 0,
                      f->stream, dst, f->norms.as<float>() + f->n, n, f->dp, f->meta.as<uint32_t>());
   QVH_HIP(hipGetLastError());
   QVH_HIP(hipMemcpyAsync(f->h_meta, f->meta.ptr, sizeof(f->h_meta), hipMemcpyDeviceToHost, f->stream));
@@ -3329,6 +3430,9 @@ void flat_append(qvh_flat* f, const float* rows, uint64_t n, float* stored_out, 
   float top;  // largest stored squared norm
   std::memcpy(&top, &f->h_meta[0], sizeof(top));
   f->integral_rows = f->h_meta[1] == 0 && top <= 16777216.0f;
+  float largest;
+  std::memcpy(&largest, &f->h_meta[2], sizeof(largest));
+  f->half_integral_rows = f->integral_rows && largest <= 2048.0f;
 }
 
 }  // namespace

@@ -1,0 +1,731 @@
+// Flat exact search for rows of up to 128 dims on the 16-bit matrix unit.
+//
+// The fp32 matrix instructions run at 157 TFLOP/s, the fp16 ones at 2.5 PFLOP/s with fp32
+// accumulation. A float times a power of two splits into two halves, x = hi + lo with |lo| <= 2^-11
+// |x|, and <q, x> = hi.hi + hi.lo + lo.hi up to 3 x 2^-22 of sum |q_i x_i|: three fp16 products give
+// the dot product to about the rounding of an fp32 chain at a third of 16 times its rate. Where
+// every stored value and every query of the batch is an integer of magnitude at most 2048, hi alone
+// is exact and one product does.
+//
+// The scan does not keep rows but groups of 16 consecutive rows: a lane takes the minimum of its 16
+// accumulators (one group of one query), and only that minimum is compared, queued and listed. The
+// merge takes the best groups of a query, scores their rows in the reference's order and stops as
+// soon as the rounding bound shows that no later group can hold a row of the answer. A result row is
+// never decided by the 16-bit scan's value, only excluded by it, and every exclusion is covered by
+// the bound (prep_queries_kernel) or the query goes to the exact kernel.
+//
+// Ranking value. Per query the scan ranks by s_q s_x (||x||^2 / 2 - <q, x>) (L2) or -s_q s_x <q, x>:
+// the distance up to a positive factor and a constant of the query. s_x brings the largest stored
+// norm to (2^10, 2^11], s_q the query's norm, both powers of two, so every half is in range. The
+// norm enters as one more matrix step: three halves of ||x||^2 s_x^2 / 2^9 in the row's padding
+// against (w, w, w), w = 2^8 s_q / s_x.
+#include <type_traits>
+
+#include "common.hpp"
+#include "exact.hpp"
+#include "flat_half.hpp"
+#include "select.hpp"
+
+namespace {
+
+using namespace qvh;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kWaves = 8;  // 2 per SIMD: one's selection runs beside the other's matrix steps
+constexpr int kThreads = kWaves * 64;
+constexpr int kTile = static_cast<int>(kHalfTileRows);
+// Queued groups per lane before a wave-wide flush (a 32-row block queues up to two). The queue arrays
+// also carry the hand-off of two row waves: four query groups' lists, 4 * 64 * KL entries.
+constexpr int queue_cap(int kl) { return kl > 16 ? 16 : 8; }
+
+/// Inserts (d, g) into the sorted list (the caller has checked d <= Ld[KL - 1]); a lane's groups come in
+/// increasing order, so an equal minimum already listed stays ahead. One parallel step: every
+/// entry's new value depends on its own compare and its neighbour's.
+template <int KL>
+__device__ __forceinline__ void group_insert(float (&Ld)[KL], uint32_t (&Lg)[KL], float d, uint32_t g) {
+  bool lt[KL];
+#pragma unroll
+  for (int x = 0; x < KL; ++x) lt[x] = d < Ld[x];
+#pragma unroll
+  for (int x = KL - 1; x > 0; --x) {
+    Ld[x] = lt[x] ? (lt[x - 1] ? Ld[x - 1] : d) : Ld[x];
+    Lg[x] = lt[x] ? (lt[x - 1] ? Lg[x - 1] : g) : Lg[x];
+  }
+  Ld[0] = lt[0] ? d : Ld[0];
+  Lg[0] = lt[0] ? g : Lg[0];
+}
+
+/// The same for groups in any order: equal minima by group.
+template <int KL>
+__device__ __forceinline__ void group_insert_any(float (&Ld)[KL], uint32_t (&Lg)[KL], float d, uint32_t g) {
+  bool lt[KL];
+#pragma unroll
+  for (int x = 0; x < KL; ++x) lt[x] = (d < Ld[x]) | ((d == Ld[x]) & (g < Lg[x]));
+#pragma unroll
+  for (int x = KL - 1; x > 0; --x) {
+    Ld[x] = lt[x] ? (lt[x - 1] ? Ld[x - 1] : d) : Ld[x];
+    Lg[x] = lt[x] ? (lt[x - 1] ? Lg[x - 1] : g) : Lg[x];
+  }
+  Ld[0] = lt[0] ? d : Ld[0];
+  Lg[0] = lt[0] ? g : Lg[0];
+}
+
+/// Sorts N values ascending in registers (a bitonic network).
+template <int N>
+__device__ __forceinline__ void sort_u32(uint32_t (&v)[N]) {
+#pragma unroll
+  for (int size = 2; size <= N; size <<= 1) {
+#pragma unroll
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int l = i ^ stride;
+        if (l > i) {
+          const uint32_t lo = min(v[i], v[l]), hi = max(v[i], v[l]);
+          const bool up = (i & size) == 0;
+          v[i] = up ? lo : hi;
+          v[l] = up ? hi : lo;
+        }
+      }
+    }
+  }
+}
+
+/// The K-th smallest of a query's 32 bound slots.
+template <int K>
+__device__ __forceinline__ uint32_t slots_kth_smallest(const uint32_t* slots) {
+  uint32_t v[32];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const uint64_t w = __hip_atomic_load(reinterpret_cast<const uint64_t*>(slots) + i, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    v[2 * i] = static_cast<uint32_t>(w);
+    v[2 * i + 1] = static_cast<uint32_t>(w >> 32);
+  }
+  if constexpr (K == 32) {
+    uint32_t m = v[0];
+#pragma unroll
+    for (int i = 1; i < 32; ++i) m = max(m, v[i]);
+    return m;
+  } else {
+    sort_u32<32>(v);
+    return v[K - 1];
+  }
+}
+
+/// Minimum of 16 accumulators.
+__device__ __forceinline__ float min16(const f32x16& a) {
+  float m = fminf(fminf(a[0], a[1]), a[2]);
+#pragma unroll
+  for (int r = 3; r + 1 < 16; r += 2) m = fminf(fminf(m, a[r]), a[r + 1]);
+  return fminf(m, a[15]);
+}
+
+// NK: 16-dim matrix steps per row. NP: 1 product (hi.hi) or 3. QG: 32-query column groups per wave.
+// QG = 2: lane l lists query l of the wave's 64 (after one half-wave swap of the minima); QG = 1: the
+// lanes j and j + 32 list the two 16-row halves of every block for query j of 32.
+//
+// Split of the work (1M x 128, 10,000 queries): 512 queries per work-group, so that a tile's
+// conversion and LDS traffic is shared by as many queries as the registers hold (64 per wave: 128
+// VGPRs of query halves at NP = 3), two waves per SIMD.
+template <int NK, int KL, int NP, int QG>
+__global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
+  if (a.gate != nullptr && ((*a.gate != 0u) != (a.gate_want != 0u))) return;  // the same for the whole grid
+  // A row in LDS: 16 NK halves, then 8 halves with the norm's three parts. The stride is 4 mod 8
+  // banks, so 16 rows' 16-byte reads of one column touch every bank once.
+  constexpr int STRIDE = 16 * NK + 8;
+  constexpr int C8 = 2 * NK;  // 8-float chunks per row
+  constexpr int CHUNKS = kTile * C8;
+  constexpr int PER = (CHUNKS + kThreads - 1) / kThreads;
+  __shared__ __attribute__((aligned(16))) _Float16 s_hi[2][kTile * STRIDE];
+  __shared__ __attribute__((aligned(16))) _Float16 s_lo[NP == 3 ? 2 : 1][NP == 3 ? kTile * STRIDE : 8];
+  __shared__ uint64_t s_bits[2];
+  // Queued (minimum, group) per lane, entry-major.
+  constexpr int kCap = queue_cap(KL);
+  static_assert(4 * 64 * KL <= kCap * kThreads, "the row waves' hand-off fits the queue arrays");
+  __shared__ float s_qd[kCap * kThreads];
+  __shared__ uint32_t s_qg[kCap * kThreads];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, h = lane >> 5;
+
+  // Work-group w runs on XCD w % 8; each XCD gets its own row splits, so the work-groups resident on
+  // one XCD at a time stream the same rows through its L2.
+  uint32_t qb, split;
+  const uint32_t wg = blockIdx.x;
+  if (a.nsplit % 8 == 0) {
+    const uint32_t x = wg % 8, li = wg / 8;
+    split = (li / a.qblocks) * 8 + x;
+    qb = li % a.qblocks;
+  } else {
+    split = wg / a.qblocks;
+    qb = wg % a.qblocks;
+  }
+
+  const uint32_t rw = a.row_waves;
+  const uint32_t qwaves = kWaves / rw;
+  const uint32_t qgroup = static_cast<uint32_t>(wave) % qwaves;  // the wave's 32 QG queries
+  const uint32_t rslot = static_cast<uint32_t>(wave) / qwaves;   // its 32-row half (rw = 2)
+  const int blk0 = static_cast<int>(rslot), blk1 = rw == 1 ? 2 : blk0 + 1;
+  const uint32_t q0 = (qb * qwaves + qgroup) * (32 * QG);
+  const bool wave_active = q0 < a.nq;
+  const uint32_t q = q0 + (QG == 2 ? static_cast<uint32_t>(lane) : static_cast<uint32_t>(j));  // the query this lane lists
+  const bool qvalid = q < a.nq;
+  const float sx = half_scale(__uint_as_float(a.meta[0]));
+
+  // Query operands: column j of group g, dims 16 kk + 8 h .. + 7 of step kk, negated and scaled.
+  f16x8 bh[QG][NK], bl[NP == 3 ? QG : 1][NP == 3 ? NK : 1];
+  f16x8 baug[QG];
+#pragma unroll
+  for (int g = 0; g < QG; ++g) {
+    const uint32_t qc = q0 + 32 * g + j;
+    const bool ok = qc < a.nq;
+    const float sq = ok ? __uint_as_float(a.words[static_cast<size_t>(qc) * kHalfWordStride + kHalfScaleWord]) : 0.0f;
+    const float* qp = a.Q + static_cast<size_t>(ok ? qc : 0) * a.dp;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      const uint32_t c = static_cast<uint32_t>(16 * kk + 8 * h);
+      const bool in = ok && c < a.dp;
+      const f32x4 v0 = *reinterpret_cast<const f32x4*>(qp + (in ? c : 0));
+      const f32x4 v1 = *reinterpret_cast<const f32x4*>(qp + (in ? c + 4 : 4));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float v = in ? -sq * (i < 4 ? v0[i & 3] : v1[i & 3]) : 0.0f;
+        const _Float16 hi = static_cast<_Float16>(v);
+        bh[g][kk][i] = hi;
+        if constexpr (NP == 3) bl[g][kk][i] = static_cast<_Float16>(v - static_cast<float>(hi));
+      }
+    }
+    const _Float16 w = static_cast<_Float16>(ok && h == 0 && a.l2 ? 256.0f * sq / sx : 0.0f);
+    baug[g] = f16x8{w, w, w, 0, 0, 0, 0, 0};
+  }
+
+  float Ld[KL];
+  uint32_t Lg[KL];
+#pragma unroll
+  for (int x = 0; x < KL; ++x) {
+    Ld[x] = __builtin_huge_valf();
+    Lg[x] = QVH_EMPTY_ROW;
+  }
+
+  // Prune threshold: the smaller of this list's KL-th minimum and the shared per-query value. Any
+  // list's KL-th bounds the KL-th of the union of all lists, so groups above it can never be among
+  // the query's KL best (equal minima pass: ties are decided by group). Bound slots: every list
+  // publishes its best minimum to one of the query's 32 slots; different slots hold minima of
+  // different groups, so the KL-th smallest slot bounds the query's KL-th best minimum from above.
+  uint32_t* const qw = a.words + static_cast<size_t>(qvalid ? q : 0u) * kHalfWordStride;
+  float pthr = __builtin_huge_valf();
+  if (qvalid && a.share) {
+    pthr = ordered_to_float(__hip_atomic_load(qw, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+  constexpr uint32_t kLists = QG == 2 ? 1u : 2u;  // per split and query
+  const uint32_t list = split * kLists + (QG == 2 ? 0u : static_cast<uint32_t>(h));
+  const uint32_t src = (list * rw + rslot) % kHalfSlots;
+  float published = __builtin_huge_valf();
+  auto share_threshold = [&]() {
+    float t = Ld[KL - 1];
+    if constexpr (QG == 1) {
+      // The lane pair's lists hold disjoint groups: their union has KL at or below
+      // max(own[KL/2-1], other[KL/2-1]) as well as below either list's KL-th.
+      const float oth_k = __shfl_xor(t, 32, 64);
+      const float own_h = Ld[KL / 2 - 1], oth_h = __shfl_xor(own_h, 32, 64);
+      t = fminf(fminf(t, oth_k), fmaxf(own_h, oth_h));
+      if (a.share_rank != 0) {
+        // The merge takes R > KL groups: the pair's union has 2 c >= R groups at or below the larger
+        // of the two lanes' c-th entries.
+        float own_c = Ld[0];
+#pragma unroll
+        for (int x = 1; x < KL; ++x) own_c = static_cast<uint32_t>(x) + 1 == a.share_rank ? Ld[x] : own_c;
+        t = fmaxf(own_c, __shfl_xor(own_c, 32, 64));
+      }
+    }
+    if (qvalid) {
+      const uint32_t g = __hip_atomic_fetch_min(qw, float_to_ordered(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      t = fminf(t, ordered_to_float(g));
+      if (a.bound_slots) {
+        if (Ld[0] < published) {
+          published = Ld[0];
+          __hip_atomic_fetch_min(qw + kHalfSlotBase + src, float_to_ordered(published), __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+        }
+        t = fminf(t, ordered_to_float(slots_kth_smallest<KL>(qw + kHalfSlotBase)));
+      }
+    }
+    pthr = fminf(pthr, t);
+  };
+
+  int qcount = 0;
+  float thr = pthr;
+  auto flush_queue = [&]() {
+    int m = qcount;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
+    for (int e = 0; e < m; ++e) {
+      if (e < qcount) {
+        const float v = s_qd[e * kThreads + tid];
+        if (v < Ld[KL - 1]) group_insert<KL>(Ld, Lg, v, s_qg[e * kThreads + tid]);
+      }
+    }
+    qcount = 0;
+    thr = fminf(pthr, Ld[KL - 1]);
+  };
+
+  const uint64_t r0 = static_cast<uint64_t>(split) * a.rows_per_split;
+  const uint64_t r1 = r0 < a.n ? (a.n < r0 + a.rows_per_split ? a.n : r0 + a.rows_per_split) : r0;
+  const uint32_t ntiles = static_cast<uint32_t>(ceil_div(r1 - r0, kTile));
+  const uint64_t last_row = r1 > r0 ? r1 - 1 : r0;
+
+  f32x4 stage[PER][2];
+  float stage_norm = 0.0f;
+  uint64_t stage_bits = ~0ull;
+  // Unconditional loads (rows past the split repeat its last row, columns past the row its first:
+  // masked later), so none sits under a branch and the next tile stays in flight under this one's
+  // matrix steps.
+  auto load_tile = [&](uint32_t t) {
+    const uint64_t base = r0 + static_cast<uint64_t>(t) * kTile;
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      int c = tid + p * kThreads;
+      if (CHUNKS % kThreads != 0) c = c < CHUNKS ? c : CHUNKS - 1;
+      const uint32_t row = static_cast<uint32_t>(c / C8), col = 8u * static_cast<uint32_t>(c % C8);
+      uint64_t gr = base + row;
+      gr = gr < last_row ? gr : last_row;
+      const float* src_row = a.X + gr * a.dp + (col < a.dp ? col : 0u);
+      stage[p][0] = *reinterpret_cast<const f32x4*>(src_row);
+      stage[p][1] = *reinterpret_cast<const f32x4*>(src_row + 4);
+    }
+    if (a.l2) {
+      uint64_t gn = base + (tid & (kTile - 1));
+      gn = gn < last_row ? gn : last_row;
+      stage_norm = a.xnorm[gn];
+    }
+    if (a.bitmap) stage_bits = a.bitmap[base >> 6];
+  };
+  // Row 16 h + 4 a + b of a 32-row block goes to LDS row 8 a + 4 h + b: accumulator register r of
+  // lane half h is then row 16 h + r, so a lane's 16 accumulators are 16 consecutive rows.
+  auto lds_row = [](uint32_t row) {
+    return (row & 32u) | ((row >> 2 & 3u) << 3) | ((row >> 4 & 1u) << 2) | (row & 3u);
+  };
+  auto store_tile = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int c = tid + p * kThreads;
+      if (CHUNKS % kThreads == 0 || c < CHUNKS) {
+        const uint32_t row = static_cast<uint32_t>(c / C8), col = 8u * static_cast<uint32_t>(c % C8);
+        const float s = col < a.dp ? sx : 0.0f;
+        f16x8 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float v = s * stage[p][i >> 2][i & 3];
+          hi[i] = static_cast<_Float16>(v);
+          if constexpr (NP == 3) lo[i] = static_cast<_Float16>(v - static_cast<float>(hi[i]));
+        }
+        const uint32_t at = lds_row(row) * STRIDE + col;
+        *reinterpret_cast<f16x8*>(&s_hi[buf][at]) = hi;
+        if constexpr (NP == 3) *reinterpret_cast<f16x8*>(&s_lo[buf][at]) = lo;
+      }
+    }
+    if (tid < kTile) {
+      float v = stage_norm * sx * sx * 0x1p-9f;
+      f16x8 n = {};
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        n[i] = static_cast<_Float16>(v);
+        v -= static_cast<float>(n[i]);
+      }
+      *reinterpret_cast<f16x8*>(&s_hi[buf][lds_row(static_cast<uint32_t>(tid)) * STRIDE + 16 * NK]) = n;
+    }
+    if (tid == kTile) s_bits[buf] = stage_bits;
+  };
+
+  if (ntiles > 0) {
+    load_tile(0);
+    store_tile(0);
+  }
+  __syncthreads();
+
+  for (uint32_t t = 0; t < ntiles; ++t) {
+    const int buf = static_cast<int>(t & 1);
+    if (t + 1 < ntiles) load_tile(t + 1);
+    if (wave_active) {
+      const uint64_t tile_row0 = r0 + static_cast<uint64_t>(t) * kTile;
+      const uint64_t left = r1 - tile_row0;
+      uint64_t admit = a.bitmap ? s_bits[buf] : ~0ull;
+      if (left < 64) admit &= (1ull << left) - 1;
+      admit = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(admit >> 32)))) << 32) |
+              static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(admit)));
+      for (int blk = blk0; blk < blk1; ++blk) {
+        const _Float16* ah = &s_hi[buf][(32 * blk + j) * STRIDE + 8 * h];
+        f32x16 acc[QG];
+#pragma unroll
+        for (int g = 0; g < QG; ++g) acc[g] = f32x16{};
+        if constexpr (NP == 3) {
+          // The small products first: their roundings are 2^-11 of the sum's.
+          const _Float16* al = &s_lo[buf][(32 * blk + j) * STRIDE + 8 * h];
+#pragma unroll
+          for (int kk = 0; kk < NK; ++kk) {
+            const f16x8 xh = *reinterpret_cast<const f16x8*>(ah + 16 * kk);
+            const f16x8 xl = *reinterpret_cast<const f16x8*>(al + 16 * kk);
+#pragma unroll
+            for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, bh[g][kk], acc[g], 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, bl[g][kk], acc[g], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+          const f16x8 xh = *reinterpret_cast<const f16x8*>(ah + 16 * kk);
+#pragma unroll
+          for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, bh[g][kk], acc[g], 0, 0, 0);
+        }
+        if (a.l2) {
+          // Every lane reads its row's norm parts; the upper half's weights are zero.
+          const f16x8 xn = *reinterpret_cast<const f16x8*>(&s_hi[buf][(32 * blk + j) * STRIDE + 16 * NK]);
+#pragma unroll
+          for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xn, baug[g], acc[g], 0, 0, 0);
+        }
+        const uint32_t bits = static_cast<uint32_t>(admit >> (32 * blk));
+        if (bits != 0xFFFFFFFFu) {  // wave-uniform: a filter, or the split's last rows
+          const uint32_t lb = bits >> (16 * h);
+#pragma unroll
+          for (int g = 0; g < QG; ++g) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[g][r] = (lb >> r) & 1u ? acc[g][r] : __builtin_huge_valf();
+          }
+        }
+        const uint32_t group0 = static_cast<uint32_t>((tile_row0 + 32 * static_cast<uint32_t>(blk)) / kHalfGroupRows);
+        if constexpr (QG == 2) {
+          // Lane l gets the minima of both 16-row halves for query l of the wave's 64.
+          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(min16(acc[0])),
+                                                           __float_as_uint(min16(acc[1])), false, false);
+          const float m0 = __uint_as_float(sw[0]), m1 = __uint_as_float(sw[1]);
+          // Groups at +inf (no admitted row) never pass; ties with the bound do. Lanes past the last
+          // query never queue.
+          const bool p0 = qvalid && m0 <= thr && m0 < __builtin_huge_valf();
+          const bool p1 = qvalid && m1 <= thr && m1 < __builtin_huge_valf();
+          if (__builtin_amdgcn_ballot_w64(p0 || p1)) {
+            if (__builtin_amdgcn_ballot_w64(qcount > kCap - 2)) flush_queue();
+            if (p0) {
+              s_qd[qcount * kThreads + tid] = m0;
+              s_qg[qcount * kThreads + tid] = group0;
+              ++qcount;
+            }
+            if (p1) {
+              s_qd[qcount * kThreads + tid] = m1;
+              s_qg[qcount * kThreads + tid] = group0 + 1;
+              ++qcount;
+            }
+          }
+        } else {
+          const float m = min16(acc[0]);
+          const bool p = qvalid && m <= thr && m < __builtin_huge_valf();
+          if (__builtin_amdgcn_ballot_w64(p)) {
+            if (__builtin_amdgcn_ballot_w64(qcount > kCap - 1)) flush_queue();
+            if (p) {
+              s_qd[qcount * kThreads + tid] = m;
+              s_qg[qcount * kThreads + tid] = group0 + static_cast<uint32_t>(h);
+              ++qcount;
+            }
+          }
+        }
+      }
+      // Bounds are exchanged after tiles 0, 1, 3, 7, 15, 31 and 63 (the first rows move a bound the
+      // most), then every 64: an exchange waits for a device-scope round trip.
+      if (t < 64 ? (t & (t + 1)) == 0 : t % 64 == 63) {
+        flush_queue();
+        if (a.share) {
+          share_threshold();
+          thr = fminf(pthr, Ld[KL - 1]);
+        }
+      }
+    }
+    if (t + 1 < ntiles) store_tile(buf ^ 1);
+    __syncthreads();
+  }
+
+  if (wave_active) flush_queue();
+  if (rw == 2) {
+    // The wave of the second halves hands its lists to the one of the first through the queue
+    // arrays, free once every wave has flushed.
+    __syncthreads();
+    const uint32_t at = (qgroup * 64 + static_cast<uint32_t>(lane)) * KL;  // qgroup < 4
+    if (rslot == 1) {
+#pragma unroll
+      for (int x = 0; x < KL; ++x) {
+        s_qd[at + x] = Ld[x];
+        s_qg[at + x] = Lg[x];
+      }
+    }
+    __syncthreads();
+    if (rslot == 1) return;
+    for (int x = 0; x < KL; ++x) {
+      const float d = s_qd[at + x];
+      if (!__builtin_amdgcn_ballot_w64(d <= Ld[KL - 1] && d < __builtin_huge_valf())) break;
+      group_insert_any<KL>(Ld, Lg, d, s_qg[at + x]);
+    }
+  }
+  if (qvalid) {
+    // Back to distances: value / (s_q s_x), one power of two at a time.
+    const float iq = 1.0f / __uint_as_float(qw[kHalfScaleWord]), ix = 1.0f / sx;
+    const float qn = a.l2 ? a.qnorm[q] : 1.0f;
+    const size_t o = (static_cast<size_t>(q) * (a.nsplit * kLists) + list) * KL;
+#pragma unroll
+    for (int x = 0; x < KL; ++x) {
+      const float v = (a.l2 ? 2.0f : 1.0f) * (Ld[x] * iq * ix) + qn;
+      a.part_d[o + x] = Lg[x] == QVH_EMPTY_ROW ? __builtin_huge_valf() : v;
+      a.part_r[o + x] = Lg[x];
+    }
+  }
+}
+
+// ---- merge: the best groups, scored exactly ---------------------------------------------------
+
+constexpr int kListsPerLane = static_cast<int>(kHalfMaxLists) / 64;
+constexpr int kHeld = 4;    // keys held per list before it reloads
+constexpr int kKeys = 128;  // scored rows held per query: the k best (k <= 64) and the next 64
+
+/// Keys p .. p + kHeld - 1 of one list (positions at or past KL read the list's start, never used).
+template <int KL>
+__device__ __forceinline__ void load_held(const float* ld, const uint32_t* lg, uint32_t p, float (&d)[kHeld],
+                                          uint32_t (&g)[kHeld]) {
+  static_assert(kHeld == 4, "one 16-byte load per list");
+  if constexpr (KL % 4 == 0) {
+    const uint32_t at = p + 4 <= KL ? p : 0u;
+    const f32x4 dv = *reinterpret_cast<const f32x4*>(ld + at);
+    const f32x4 gv = *reinterpret_cast<const f32x4*>(lg + at);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      d[i] = dv[i];
+      g[i] = __float_as_uint(gv[i]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t at = p + i < KL ? p + i : 0u;
+      d[i] = ld[at];
+      g[i] = lg[at];
+    }
+  }
+}
+
+/// One wave per query. First the `sel` best groups over the query's lists (ascending by minimum,
+/// then group), popped from list heads held in registers. Then their rows in the reference's order,
+/// four groups at a time (eight lanes per row), keeping the k best (distance, row). After each step
+/// the next group's minimum decides: every row not yet scored has a scan distance of at least that,
+/// so an exact one of at least that minus delta, and once this is above the k-th best distance the
+/// answer is final. At the end of the selection the answer stands if the lists held no more groups
+/// or if delta is 0 (the scan's distances are exact: the sel >= k selected minima are rows that
+/// precede every row of any other group in (distance, row) order); otherwise the last selected
+/// minimum decides the same way, and a query that fails goes to the exact kernel.
+template <int KL>
+__global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
+  if (m.gate != nullptr && ((*m.gate != 0u) != (m.gate_want != 0u))) return;
+  __shared__ uint64_t s_sel[4][kHalfMaxSel];
+  __shared__ uint64_t s_key[4][kKeys];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t q = blockIdx.x * 4 + wave;
+  if (q >= m.nq) return;  // whole wave; this kernel has no block barriers
+  uint64_t* const sel = s_sel[wave];
+  uint64_t* const keys = s_key[wave];
+  const float* pd = m.part_d + static_cast<size_t>(q) * m.nlists * KL;
+  const uint32_t* pg = m.part_r + static_cast<size_t>(q) * m.nlists * KL;
+
+  uint64_t kk[kListsPerLane][kHeld];
+  uint32_t ptr[kListsPerLane];
+#pragma unroll
+  for (int u = 0; u < kListsPerLane; ++u) {
+    ptr[u] = 0;
+    if (64u * u < m.nlists) {  // wave-uniform
+      const uint32_t li = lane + 64 * u;
+      const bool ok = li < m.nlists;
+      const uint32_t lc = ok ? li : 0u;
+      float d[kHeld];
+      uint32_t g[kHeld];
+      load_held<KL>(pd + static_cast<size_t>(lc) * KL, pg + static_cast<size_t>(lc) * KL, 0, d, g);
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i) kk[u][i] = ok && i < KL ? make_key(d[i], g[i]) : ~0ull;
+    } else {
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i) kk[u][i] = ~0ull;
+    }
+  }
+  uint32_t count = 0;
+  bool spent = false;  // one of this lane's lists gave all of its entries before the selection ended
+  for (uint32_t x = 0; x < m.sel; ++x) {
+    uint64_t mine = kk[0][0];
+    int arg = 0;
+#pragma unroll
+    for (int u = 1; u < kListsPerLane; ++u) {
+      if (kk[u][0] < mine) {
+        mine = kk[u][0];
+        arg = u;
+      }
+    }
+    const uint64_t best = wave_min_u64(mine);
+    if (static_cast<uint32_t>(best) == QVH_EMPTY_ROW) break;  // only empty slots remain
+    if (lane == 0) sel[x] = best;
+    ++count;
+    if (mine == best) {
+#pragma unroll
+      for (int u = 0; u < kListsPerLane; ++u) {
+        if (u == arg) {
+#pragma unroll
+          for (int i = 0; i + 1 < kHeld; ++i) kk[u][i] = kk[u][i + 1];
+          kk[u][kHeld - 1] = ~0ull;
+          const uint32_t p = ++ptr[u];
+          if (p == KL) spent = spent || x + 1 < m.sel;
+          if (p % kHeld == 0 && p < KL) {
+            float d[kHeld];
+            uint32_t g[kHeld];
+            load_held<KL>(pd + static_cast<size_t>(lane + 64 * u) * KL, pg + static_cast<size_t>(lane + 64 * u) * KL, p,
+                          d, g);
+#pragma unroll
+            for (int i = 0; i < kHeld; ++i) kk[u][i] = p + i < KL ? make_key(d[i], g[i]) : ~0ull;
+          }
+        }
+      }
+    }
+  }
+  const double delta = static_cast<double>(m.delta[q]);
+  // A list that ran out (wide merge) may have held more of the answer; a non-finite bound certifies
+  // nothing.
+  if ((m.wide && __ballot(spent) != 0) || !(delta < static_cast<double>(__builtin_huge_valf()))) {
+    if (lane == 0) m.fallback[atomicAdd(m.nfallback, 1u)] = q;
+    return;
+  }
+  __builtin_amdgcn_wave_barrier();
+
+  const float* qp = m.Q + static_cast<size_t>(q) * m.dp;
+  const uint32_t oct = static_cast<uint32_t>(lane) >> 3;
+  const uint32_t k = m.k;
+  uint32_t held = 0;        // keys[0, held); the first min(held, k) sorted after each step
+  uint64_t bound = ~0ull;   // the k-th best key so far
+  uint64_t x2[2] = {~0ull, ~0ull};
+  bool done = false;
+  for (uint32_t c0 = 0; c0 < count && !done; c0 += 4) {
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+      const float* b[4];
+      uint32_t row[4];
+      bool ok[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint32_t e = static_cast<uint32_t>(pass) * 32 + static_cast<uint32_t>(c) * 8 + oct;  // row of the step
+        const uint32_t gi = c0 + e / 16;
+        ok[c] = gi < count;
+        const uint64_t pos =
+            static_cast<uint64_t>(static_cast<uint32_t>(sel[ok[c] ? gi : 0])) * kHalfGroupRows + e % 16;
+        ok[c] = ok[c] && pos < m.n;
+        row[c] = ok[c] ? (m.idx ? m.idx[pos] : static_cast<uint32_t>(pos)) : 0u;
+        if (m.bitmap) ok[c] = ok[c] && ((m.bitmap[row[c] >> 6] >> (row[c] & 63)) & 1u);
+        b[c] = ok[c] ? m.X + static_cast<size_t>(row[c]) * m.dp : qp;
+      }
+      float e4[4];
+      if (m.l2) {
+        exact_group8_n<true, 4>(qp, b, m.dim, e4);
+      } else {
+        exact_group8_n<false, 4>(qp, b, m.dim, e4);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float d = m.l2 ? e4[c] : 1.0f - e4[c];
+        d = d == d ? d : __builtin_huge_valf();
+        const uint64_t key = make_key(d, row[c]);
+        const bool take = ok[c] && (lane & 7) == 0 && key < bound;
+        const uint64_t mk = __ballot(take);
+        if (take) keys[held + lane_rank(mk)] = key;  // at most 64 past the k <= 64 kept
+        held += static_cast<uint32_t>(__popcll(mk));
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t e = static_cast<uint32_t>(i * 64 + lane);
+      x2[i] = e < held ? keys[e] : ~0ull;
+    }
+    wave_sort<2>(x2);
+    held = held < k ? held : k;
+    __builtin_amdgcn_wave_barrier();
+    if (static_cast<uint32_t>(lane) < held) keys[lane] = x2[0];
+    __builtin_amdgcn_wave_barrier();
+    if (held == k) {
+      bound = __shfl(x2[0], static_cast<int>(k) - 1, 64);
+      if (c0 + 4 < count) {
+        const double g_next = static_cast<double>(ordered_to_float(static_cast<uint32_t>(sel[c0 + 4] >> 32)));
+        done = g_next - delta > static_cast<double>(ordered_to_float(static_cast<uint32_t>(bound >> 32)));
+      }
+    }
+  }
+  if (!done && count >= m.sel && delta != 0.0) {
+    const double g_last = static_cast<double>(ordered_to_float(static_cast<uint32_t>(sel[count - 1] >> 32)));
+    const bool certified =
+        held == k && static_cast<double>(ordered_to_float(static_cast<uint32_t>(bound >> 32))) < g_last - delta;
+    if (!certified) {
+      if (lane == 0) m.fallback[atomicAdd(m.nfallback, 1u)] = q;
+      return;
+    }
+  }
+  if (static_cast<uint32_t>(lane) < k) {
+    const bool full = static_cast<uint32_t>(lane) < held;
+    m.out_rows[static_cast<size_t>(q) * k + lane] = full ? static_cast<uint32_t>(x2[0]) : QVH_EMPTY_ROW;
+    m.out_dist[static_cast<size_t>(q) * k + lane] =
+        full ? ordered_to_float(static_cast<uint32_t>(x2[0] >> 32)) : __builtin_huge_valf();
+  }
+}
+
+template <int NK>
+void launch_nk(int kl, int products, bool pair, dim3 grid, const HalfScanArgs& a, hipStream_t s) {
+  if (products == 1) {
+    if (kl != 10) throw Failure(QVH_EUNSUPPORTED, "half scan: one product takes lists of 10");
+    if (pair) {
+      hipLaunchKernelGGL((flat_half_kernel<NK, 10, 1, 1>), grid, dim3(kThreads), 0, s, a);
+    } else {
+      hipLaunchKernelGGL((flat_half_kernel<NK, 10, 1, 2>), grid, dim3(kThreads), 0, s, a);
+    }
+  } else if (kl == 16) {
+    if (pair) {
+      hipLaunchKernelGGL((flat_half_kernel<NK, 16, 3, 1>), grid, dim3(kThreads), 0, s, a);
+    } else {
+      hipLaunchKernelGGL((flat_half_kernel<NK, 16, 3, 2>), grid, dim3(kThreads), 0, s, a);
+    }
+  } else if (kl == 32 && pair) {
+    hipLaunchKernelGGL((flat_half_kernel<NK, 32, 3, 1>), grid, dim3(kThreads), 0, s, a);
+  } else {
+    throw Failure(QVH_EUNSUPPORTED, "half scan: unsupported list length");
+  }
+}
+
+}  // namespace
+
+namespace qvh {
+
+void launch_half_scan(int kl, int products, bool pair, dim3 grid, const HalfScanArgs& a, hipStream_t s) {
+  switch ((a.dp + 15) / 16) {
+    case 1: launch_nk<1>(kl, products, pair, grid, a, s); break;
+    case 2: launch_nk<2>(kl, products, pair, grid, a, s); break;
+    case 3: launch_nk<3>(kl, products, pair, grid, a, s); break;
+    case 4: launch_nk<4>(kl, products, pair, grid, a, s); break;
+    case 5: launch_nk<5>(kl, products, pair, grid, a, s); break;
+    case 6: launch_nk<6>(kl, products, pair, grid, a, s); break;
+    case 7: launch_nk<7>(kl, products, pair, grid, a, s); break;
+    case 8: launch_nk<8>(kl, products, pair, grid, a, s); break;
+    default: throw Failure(QVH_EUNSUPPORTED, "half scan: unsupported row width");
+  }
+}
+
+void launch_half_merge(int kl, const HalfMergeArgs& m, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(ceil_div(m.nq, 4)));
+  if (kl == 10) {
+    hipLaunchKernelGGL(flat_half_merge_kernel<10>, grid, dim3(256), 0, s, m);
+  } else if (kl == 16) {
+    hipLaunchKernelGGL(flat_half_merge_kernel<16>, grid, dim3(256), 0, s, m);
+  } else {
+    hipLaunchKernelGGL(flat_half_merge_kernel<32>, grid, dim3(256), 0, s, m);
+  }
+}
+
+}  // namespace qvh

@@ -1,0 +1,92 @@
+// The flat scan on the 16-bit matrix unit (flat_half.hip): launch interface for flat.hip.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace qvh {
+
+constexpr uint32_t kHalfMaxDp = 128;      // register-resident query width
+constexpr uint32_t kHalfGroupRows = 16;   // rows per listed group
+constexpr uint32_t kHalfTileRows = 64;
+constexpr uint32_t kHalfMaxLists = 512;   // lists per query the merge takes
+constexpr uint32_t kHalfMaxSel = 64;      // groups the merge selects per query at most
+// The scan's words per query in `words`: word 0 the union bound, kHalfSlotBase and up the bound slots,
+// kHalfScaleWord the query's scale (float bits, written by the prep kernel).
+constexpr uint32_t kHalfWordStride = 64;
+constexpr uint32_t kHalfSlotBase = 32;
+constexpr uint32_t kHalfSlots = 32;
+constexpr uint32_t kHalfScaleWord = 1;
+
+/// 2^(11 - e) for a norm whose square is n2, 2^(e - 1) < norm <= 2^e (1 for zero and non-finite ones):
+/// brings the norm to (2^10, 2^11].
+__device__ __forceinline__ float half_scale(float n2) {
+  if (!(n2 > 0.0f) || !(n2 < __builtin_huge_valf())) return 1.0f;
+  int e = 0;
+  const float m = frexpf(sqrtf(n2), &e);  // m in [0.5, 1)
+  if (m == 0.5f) --e;
+  e = 11 - e;
+  return ldexpf(1.0f, e < -100 ? -100 : e > 100 ? 100 : e);
+}
+
+struct HalfScanArgs {
+  const float* X;          // [rows][dp] rows as stored (or the contiguous copy of listed rows)
+  const float* xnorm;      // [rows] ||x||^2 (L2)
+  uint64_t n;              // rows scanned
+  uint32_t dp;             // row width, a multiple of 8 in [16, 128]
+  const float* Q;          // [nq][dp] prepared queries
+  const float* qnorm;      // [nq] ||q||^2
+  uint32_t nq;
+  const uint64_t* bitmap;  // admitted rows, or null
+  int l2;
+  uint32_t nsplit;
+  uint32_t qblocks;
+  uint64_t rows_per_split;  // a multiple of kHalfTileRows
+  // Waves sharing each query group: 1 (every wave takes whole tiles), or 2 (the waves w and w + 4 hold
+  // the same queries and take the two 32-row halves of every tile).
+  uint32_t row_waves;
+  float* part_d;     // [nq][lists][KL] group minima as distances, ascending
+  uint32_t* part_r;  // their groups (rows 16 g .. 16 g + 15)
+  uint32_t* words;   // kHalfWordStride words per query
+  int share;            // 0: every list keeps its own KL best
+  uint32_t share_rank;  // nonzero: the shared bound is the larger of the lane pair's entries of this rank
+  int bound_slots;
+  const uint32_t* meta;  // store meta: [0] largest squared norm (float bits)
+  const uint32_t* gate;  // the launch runs when (*gate != 0) == (gate_want != 0); null: always
+  uint32_t gate_want;
+};
+
+struct HalfMergeArgs {
+  const float* X;  // the store
+  uint32_t dim, dp;
+  uint64_t n;  // rows scanned (positions in the list when idx is set)
+  const float* Q;
+  uint32_t nq, k;
+  int l2;
+  uint32_t nlists, sel;  // lists per query, groups selected (kl, or more for the wide merge)
+  int wide;              // a list all of whose entries were taken sends the query to the exact kernel
+  const float* part_d;
+  const uint32_t* part_r;
+  const uint32_t* idx;     // list positions -> rows, or null
+  const uint64_t* bitmap;  // admitted rows, or null
+  uint32_t* out_rows;
+  float* out_dist;
+  const float* delta;
+  uint32_t* fallback;
+  uint32_t* nfallback;
+  const uint32_t* gate;
+  uint32_t gate_want;
+};
+
+/// Queries per work-group and lists per (query, split) of a scan with lists of kl groups.
+/// pair: a lane pair holds each query (two lists); otherwise one lane does.
+inline uint32_t half_queries_per_block(bool pair, uint32_t row_waves) { return (pair ? 256u : 512u) / row_waves; }
+inline uint32_t half_lists_per_split(bool pair) { return pair ? 2u : 1u; }
+
+/// One scan launch. kl: 10, 16 or 32 (32 only with `pair`). products: 1 (every operand exact in
+/// 16 bits) or 3.
+void launch_half_scan(int kl, int products, bool pair, dim3 grid, const HalfScanArgs& a, hipStream_t s);
+void launch_half_merge(int kl, const HalfMergeArgs& m, hipStream_t s);
+
+}  // namespace qvh
