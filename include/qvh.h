@@ -70,6 +70,21 @@ qvh_status qvh_get_device(int* device);
 qvh_status qvh_device_info(char* name, size_t name_len, char* arch, size_t arch_len,
                            int* compute_units);
 
+/* Whether `count` device floats are all finite (*finite = 1 or 0): the input check of the host entry
+ * points' callers (src/flat_index.cc:50) for device-resident queries. Runs on `stream` (NULL = the
+ * legacy null stream here) and waits for it. */
+qvh_status qvh_device_finite(const float* d_x, uint64_t count, void* stream, int* finite);
+
+/* Result rows to labels on the device, enqueued on `stream` (not NULL): out[i] = table[rows[i]], or -1
+ * for QVH_EMPTY_ROW; `table` holds n labels by row. */
+qvh_status qvh_map_rows_device(const uint32_t* d_rows, uint64_t count, const uint64_t* d_table,
+                               uint64_t n, int64_t* d_labels, void* stream);
+/* The same for IVF-PQ refs ((list << 32) | offset in list): out[i] = table[offsets[list] + offset], or
+ * -1 for QVH_EMPTY_REF; `offsets` [nlist + 1] and `table` (n labels in list order) on the device. */
+qvh_status qvh_map_refs_device(const uint64_t* d_refs, uint64_t count, const uint64_t* d_offsets,
+                               uint64_t nlist, const uint64_t* d_table, uint64_t n, int64_t* d_labels,
+                               void* stream);
+
 /* Unit-normalizes n rows of `dim` floats in place, bit-identical to the reference's
  * simd::normalize with the AVX2 kernels (src/simd/dispatch.cc:119-135,
  * src/simd/kernels_avx2.cc:58-83). Host buffers. */

@@ -65,20 +65,11 @@ def _is_device_tensor(x) -> bool:
     return type(x).__module__.startswith("torch") and bool(getattr(x, "is_cuda", False))
 
 
-def _hip_runtimes():
-    """Paths of the HIP runtime libraries mapped into this process."""
-    try:
-        with open("/proc/self/maps") as f:
-            return {line.split()[-1] for line in f if "libamdhip64" in line}
-    except OSError:  # pragma: no cover - non-Linux
-        return set()
-
-
 def _device_queries(queries, dim: int, k: int):
     """Checks a device query batch the way _as_matrix and the host path check host ones."""
     import torch
 
-    runtimes = _hip_runtimes()
+    runtimes = set(_quiver._hip_runtimes())
     if len(runtimes) > 1:
         raise ValueError("torch and quiver_amd run on different HIP runtimes in this process "
                          f"({', '.join(sorted(runtimes))}), so device tensors cannot be shared: "
@@ -97,36 +88,47 @@ def _device_queries(queries, dim: int, k: int):
     if q.device.index != index_device:
         raise ValueError(f"queries are on {q.device}, the index on cuda:{index_device}")
     q = q.to(torch.float32).contiguous()
-    if q.numel() and not bool(torch.isfinite(q).all()):
+    if q.numel() and not _quiver._device_finite(q.data_ptr(), q.numel(),
+                                                torch.cuda.current_stream(q.device).cuda_stream):
         raise ValueError("vectors must be finite")
     return q
 
 
-def _device_results(nq: int, k: int, device):
+def _no_results(nq: int, k: int, device):
+    """The results of a search that finds nothing."""
     import torch
 
     return (torch.full((nq, k), -1, dtype=torch.int64, device=device),
             torch.full((nq, k), float("inf"), dtype=torch.float32, device=device))
 
 
+def _device_results(nq: int, k: int, device):
+    """Label and distance buffers, every entry of which the search writes."""
+    import torch
+
+    return (torch.empty((nq, k), dtype=torch.int64, device=device),
+            torch.empty((nq, k), dtype=torch.float32, device=device))
+
+
 def _on_torch_stream(device, tensors, launch) -> None:
     """Calls launch(stream) so that its device work runs after the work already queued on torch's
-    current stream and before the work queued there afterwards. The library reads a null stream
-    as "the handle's own stream", so torch's null stream is replaced by a side stream that joins
-    it on both ends."""
+    current stream and before the work queued there afterwards; launch returns the tensors it used
+    beyond `tensors`. The library reads a null stream as "the handle's own stream", so torch's null
+    stream is replaced by a side stream that joins it on both ends."""
     import torch
 
     cur = torch.cuda.current_stream(device)
-    if cur.cuda_stream != 0:
-        launch(cur.cuda_stream)
-        return
-    side = torch.cuda.Stream(device=device)
-    side.wait_stream(cur)
-    for t in tensors:
-        if t is not None:
-            t.record_stream(side)
-    launch(side.cuda_stream)
-    cur.wait_stream(side)
+    stream = cur
+    if cur.cuda_stream == 0:
+        stream = torch.cuda.Stream(device=device)
+        stream.wait_stream(cur)
+        for t in tensors:
+            if t is not None:
+                t.record_stream(stream)
+    for t in launch(stream.cuda_stream):
+        t.record_stream(stream)
+    if stream is not cur:
+        cur.wait_stream(stream)
 
 
 def _device_bitmap(bits: np.ndarray, device):
@@ -236,21 +238,26 @@ class IvfPqIndex:
         q = _device_queries(queries, self.dim, k)
         if refine_factor < 0:
             raise ValueError("refine_factor must be non-negative")
-        labels, dist = _device_results(q.shape[0], k, q.device)
         n = len(self)
         if q.shape[0] == 0 or n == 0 or not self.is_trained:
-            return labels, dist
+            return _no_results(q.shape[0], k, q.device)
+        labels, dist = _device_results(q.shape[0], k, q.device)
         bitmap = None
         if filter is not None:
             bitmap = _device_bitmap(self._index._position_bitmap(_as_labels(filter)), q.device)
         refs = torch.empty((q.shape[0], k), dtype=torch.int64, device=q.device)
-        _on_torch_stream(q.device, (q, bitmap, refs, dist), lambda stream: self._index._search_device(
-            q.data_ptr(), q.shape[0], k, max(nprobe, 1), refine_factor, 0 if bitmap is None else bitmap.data_ptr(),
-            refs.data_ptr(), dist.data_ptr(), stream))
-        offsets, table = self._label_tables(q.device, n)
-        found = refs != -1
-        pos = offsets[(refs >> 32).clamp(0, offsets.numel() - 1)] + (refs & 0xFFFFFFFF)
-        return torch.where(found, table[pos.clamp(0, n - 1)], labels), dist
+
+        def launch(stream):
+            self._index._search_device(q.data_ptr(), q.shape[0], k, max(nprobe, 1), refine_factor,
+                                       0 if bitmap is None else bitmap.data_ptr(), refs.data_ptr(), dist.data_ptr(),
+                                       stream)
+            offsets, table = self._label_tables(q.device, n)  # a new index's upload runs beside the search
+            _quiver._map_refs(refs.data_ptr(), refs.numel(), offsets.data_ptr(), offsets.numel() - 1,
+                              table.data_ptr(), n, labels.data_ptr(), stream)
+            return offsets, table
+
+        _on_torch_stream(q.device, (q, bitmap, refs, dist, labels), launch)
+        return labels, dist
 
     def _label_tables(self, device, n: int):
         """CSR offsets and labels on `device` (refs -> labels), rebuilt when the index grows."""
@@ -342,24 +349,28 @@ class FlatIndex:
         import torch
 
         q = _device_queries(queries, self.dim, k)
-        labels, dist = _device_results(q.shape[0], k, q.device)
         n = len(self)
         if q.shape[0] == 0 or n == 0:
-            return labels, dist
+            return _no_results(q.shape[0], k, q.device)
+        labels, dist = _device_results(q.shape[0], k, q.device)
         rows = torch.empty((q.shape[0], k), dtype=torch.int32, device=q.device)
         listed = None
         if filter is not None:
             # The admitted rows, ascending, as a device list: the scan then reads only those rows.
             listed = _device_rows(self._index._row_bitmap(_as_labels(filter)), n, q.device)
-        if listed is None:
-            _on_torch_stream(q.device, (q, rows, dist), lambda stream: self._index._search_device(
-                q.data_ptr(), q.shape[0], k, 0, rows.data_ptr(), dist.data_ptr(), stream))
-        else:
-            _on_torch_stream(q.device, (q, listed, rows, dist), lambda stream: self._index._search_device_rows(
-                q.data_ptr(), q.shape[0], k, listed.data_ptr(), listed.numel(), rows.data_ptr(), dist.data_ptr(),
-                stream))
-        table = self._label_table(q.device, n)
-        return torch.where(rows != -1, table[rows.clamp(0, n - 1).long()], labels), dist
+
+        def launch(stream):
+            if listed is None:
+                self._index._search_device(q.data_ptr(), q.shape[0], k, 0, rows.data_ptr(), dist.data_ptr(), stream)
+            else:
+                self._index._search_device_rows(q.data_ptr(), q.shape[0], k, listed.data_ptr(), listed.numel(),
+                                                rows.data_ptr(), dist.data_ptr(), stream)
+            table = self._label_table(q.device, n)  # a new index's upload runs beside the search
+            _quiver._map_rows(rows.data_ptr(), rows.numel(), table.data_ptr(), n, labels.data_ptr(), stream)
+            return (table,)
+
+        _on_torch_stream(q.device, (q, listed, rows, dist, labels), launch)
+        return labels, dist
 
     def _label_table(self, device, n: int):
         """Labels by row on `device`, rebuilt when the index grows."""

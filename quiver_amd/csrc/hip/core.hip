@@ -1,5 +1,6 @@
 // Process-wide state of the qvh library: error reporting, device selection, the allocation
 // fault hook, and row normalization.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <string>
@@ -63,6 +64,58 @@ __global__ void normalize_rows_kernel(float* __restrict__ rows, uint64_t n, uint
   const float inv = 1.0f / sqrtf(norm_sq);
   for (uint32_t i = l; i < dim; i += 8) v[i] = v[i] * inv;
 }
+
+/// Raises *flag (host memory the device can write) when some value is not finite.
+__global__ void __launch_bounds__(256) finite_kernel(const float* __restrict__ x, uint64_t n, uint32_t* flag) {
+  bool ok = true;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
+       i += static_cast<uint64_t>(gridDim.x) * 256) {
+    ok = ok && isfinite(x[i]);
+  }
+  if (__builtin_amdgcn_ballot_w64(!ok) != 0 && (threadIdx.x & 63) == 0) {
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+__global__ void __launch_bounds__(256) map_rows_kernel(const uint32_t* __restrict__ rows, uint64_t count,
+                                                       const uint64_t* __restrict__ table, uint64_t n,
+                                                       int64_t* __restrict__ out) {
+  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= count) return;
+  const uint32_t r = rows[i];
+  out[i] = r < n ? static_cast<int64_t>(table[r]) : -1;
+}
+
+__global__ void __launch_bounds__(256) map_refs_kernel(const uint64_t* __restrict__ refs, uint64_t count,
+                                                       const uint64_t* __restrict__ offsets, uint64_t nlist,
+                                                       const uint64_t* __restrict__ table, uint64_t n,
+                                                       int64_t* __restrict__ out) {
+  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= count) return;
+  const uint64_t ref = refs[i], list = ref >> 32;
+  const uint64_t pos = list < nlist ? offsets[list] + (ref & 0xFFFFFFFFull) : n;
+  out[i] = ref != QVH_EMPTY_REF && pos < n ? static_cast<int64_t>(table[pos]) : -1;
+}
+
+/// One word of pinned host memory per thread that checks device inputs, released when it ends.
+struct PinnedWord {
+  uint32_t* ptr = nullptr;
+  PinnedWord() = default;
+  PinnedWord(const PinnedWord&) = delete;
+  PinnedWord& operator=(const PinnedWord&) = delete;
+  ~PinnedWord() {
+    if (ptr) (void)hipHostFree(ptr);
+  }
+  uint32_t* get() {
+    if (!ptr) {
+      void* p = nullptr;
+      QVH_HIP(hipHostMalloc(&p, sizeof(uint32_t), hipHostMallocPortable));
+      ptr = static_cast<uint32_t*>(p);
+    }
+    return ptr;
+  }
+};
+thread_local PinnedWord t_finite;
 
 }  // namespace
 
@@ -154,6 +207,48 @@ qvh_status qvh_device_info(char* name, size_t name_len, char* arch, size_t arch_
       arch[arch_len - 1] = '\0';
     }
     if (compute_units) *compute_units = prop.multiProcessorCount;
+  });
+}
+
+qvh_status qvh_device_finite(const float* d_x, uint64_t count, void* stream, int* finite) {
+  return qvh::guarded([&] {
+    QVH_REQUIRE(finite != nullptr, "qvh_device_finite: null output");
+    *finite = 1;
+    if (count == 0) return;
+    QVH_REQUIRE(d_x != nullptr, "qvh_device_finite: null buffer");
+    qvh::current_device();
+    uint32_t* flag = qvh::t_finite.get();
+    __atomic_store_n(flag, 0u, __ATOMIC_RELEASE);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const uint64_t blocks = std::min<uint64_t>(qvh::ceil_div(count, 1024), 1024);
+    hipLaunchKernelGGL(qvh::finite_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, d_x, count, flag);
+    QVH_HIP(hipGetLastError());
+    QVH_HIP(hipStreamSynchronize(s));
+    *finite = __atomic_load_n(flag, __ATOMIC_ACQUIRE) == 0u ? 1 : 0;
+  });
+}
+
+qvh_status qvh_map_rows_device(const uint32_t* d_rows, uint64_t count, const uint64_t* d_table, uint64_t n,
+                               int64_t* d_labels, void* stream) {
+  return qvh::guarded([&] {
+    if (count == 0) return;
+    QVH_REQUIRE(d_rows && d_table && d_labels && stream, "qvh_map_rows_device: null argument");
+    qvh::current_device();
+    hipLaunchKernelGGL(qvh::map_rows_kernel, dim3(static_cast<unsigned>(qvh::ceil_div(count, 256))), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), d_rows, count, d_table, n, d_labels);
+    QVH_HIP(hipGetLastError());
+  });
+}
+
+qvh_status qvh_map_refs_device(const uint64_t* d_refs, uint64_t count, const uint64_t* d_offsets, uint64_t nlist,
+                               const uint64_t* d_table, uint64_t n, int64_t* d_labels, void* stream) {
+  return qvh::guarded([&] {
+    if (count == 0) return;
+    QVH_REQUIRE(d_refs && d_offsets && d_table && d_labels && stream, "qvh_map_refs_device: null argument");
+    qvh::current_device();
+    hipLaunchKernelGGL(qvh::map_refs_kernel, dim3(static_cast<unsigned>(qvh::ceil_div(count, 256))), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), d_refs, count, d_offsets, nlist, d_table, n, d_labels);
+    QVH_HIP(hipGetLastError());
   });
 }
 

@@ -5,8 +5,11 @@
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
+#include <link.h>
+
 #include <algorithm>
 #include <cstring>
+#include <string>
 #include <utility>
 #include <vector>
 #include <memory>
@@ -125,6 +128,43 @@ PYBIND11_MODULE(_quiver, m) {
     int d = 0;
     if (qvh_get_device(&d) != QVH_OK) throw quiver::Error(std::string("no device: ") + qvh_last_error());
     return d;
+  });
+
+  // Paths of the HIP runtime libraries loaded in this process.
+  m.def("_hip_runtimes", [] {
+    std::vector<std::string> found;
+    dl_iterate_phdr(
+        [](dl_phdr_info* info, std::size_t, void* out) {
+          if (info->dlpi_name != nullptr && std::strstr(info->dlpi_name, "libamdhip64") != nullptr) {
+            static_cast<std::vector<std::string>*>(out)->emplace_back(info->dlpi_name);
+          }
+          return 0;
+        },
+        &found);
+    return found;
+  });
+
+  const auto check = [](qvh_status st) {
+    if (st != QVH_OK) throw quiver::Error(qvh_last_error());
+  };
+  m.def("_device_finite", [check](std::uintptr_t x, std::uint64_t count, std::uintptr_t stream) {
+    int finite = 0;
+    py::gil_scoped_release release;
+    check(qvh_device_finite(reinterpret_cast<const float*>(x), count, reinterpret_cast<void*>(stream), &finite));
+    return finite != 0;
+  });
+  m.def("_map_rows", [check](std::uintptr_t rows, std::uint64_t count, std::uintptr_t table, std::uint64_t n,
+                             std::uintptr_t out, std::uintptr_t stream) {
+    check(qvh_map_rows_device(reinterpret_cast<const std::uint32_t*>(rows), count,
+                              reinterpret_cast<const std::uint64_t*>(table), n, reinterpret_cast<std::int64_t*>(out),
+                              reinterpret_cast<void*>(stream)));
+  });
+  m.def("_map_refs", [check](std::uintptr_t refs, std::uint64_t count, std::uintptr_t offsets, std::uint64_t nlist,
+                             std::uintptr_t table, std::uint64_t n, std::uintptr_t out, std::uintptr_t stream) {
+    check(qvh_map_refs_device(reinterpret_cast<const std::uint64_t*>(refs), count,
+                              reinterpret_cast<const std::uint64_t*>(offsets), nlist,
+                              reinterpret_cast<const std::uint64_t*>(table), n, reinterpret_cast<std::int64_t*>(out),
+                              reinterpret_cast<void*>(stream)));
   });
 
   m.def(
