@@ -1700,8 +1700,9 @@ __global__ void __launch_bounds__(256) row_norms_kernel(const float* __restrict_
 ///   2          the value's way back to a distance;
 /// and the reference's own sum, which adds every term through at most n/32 + 15 roundings
 /// (src/simd/kernels_avx2.cc:35-83: four 8-lane chains, a tree, a tail of up to 7), two of them in
-/// the difference: n/32 + 18. Together below 1.16 n + 50; delta uses 1.25 n + 64. It is 0 under the
-/// condition above if also no stored or query value exceeds 2048 in magnitude: hi then holds every
+/// the difference: n/32 + 18. Together below 1.16 n + 50; delta uses 1.25 n + 64. The form for wide rows
+/// (half = 2) takes its three products step by step, so all 3 n/16 of its steps count in full
+/// (3.375 n): 3.5 n + 64. delta is 0 under the condition above if also no stored or query value exceeds 2048 in magnitude: hi then holds every
 /// value, lo is 0, and the sums are exact.
 __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restrict__ src, float* __restrict__ qp,
                                                            uint64_t nq, uint32_t dim, uint32_t dp,
@@ -1746,7 +1747,7 @@ __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restri
   const double P = sqrt(static_cast<double>(n2));
   const double R = sqrt(static_cast<double>(__uint_as_float(meta[0])));
   const double u = 1.0 / 16777216.0;
-  const double coef = (half ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;
+  const double coef = (half == 2 ? 3.5 * dp + 64.0 : half == 1 ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;
   double d;
   if (integral && meta[1] == 0 && (P + R) * (P + R) * (1.0 + 1e-12) <= 16777216.0 &&
       (!half || (largest <= 2048.0f && __uint_as_float(meta[2]) <= 2048.0f))) {
@@ -2685,6 +2686,7 @@ struct qvh_flat {
   // per-call workspace (grown on demand, serialized by mu)
   DeviceBuffer w_stage, w_q, w_qn, w_pd, w_pr, w_rows, w_dist, w_bits, w_thr, w_idx, w_fb, w_mflag, w_delta;
   DeviceBuffer w_skin, w_skout, w_soff, w_stmp;  // k above kExactMaxK: sort keys and scratch
+  DeviceBuffer w_qf;                              // split queries of the 16-bit scan over wide rows
   DeviceBuffer w_cx, w_cn;                        // listed rows gathered for the MFMA scan, their norms
   // optional per-stage timing of the last search: events before prep, scan, merge and after
   bool timing = false;
@@ -2729,8 +2731,10 @@ struct FlatPlan {
   enum Path { kFew, kSplit, kExactOnly, kMfma, kSorted } path = kMfma;
   bool wide = false;
   bool ring = false;  // kMfma: the ring scan (one 32-query group, unfiltered) instead of the MFMA scan
-  // kMfma: the scan on the 16-bit matrix unit (rows up to kHalfMaxDp, up to kHalfMaxSel groups a query).
+  // kMfma: the scan on the 16-bit matrix unit (rows up to kHalfMaxDp, or its wide form up to
+  // kHalfWideMaxDp; up to kHalfMaxSel groups a query).
   bool half = false;
+  bool half_wide = false;
   bool pair = false;       // its list layout: two lanes per query
   uint32_t row_waves = 1;  // and waves per query group
   int kl = 16;
@@ -2745,6 +2749,7 @@ struct FlatPlan {
   size_t stage = 0, q = 0, qn = 0, delta = 0, pd = 0, pr = 0, thr = 0, fb = 0, mflag = 0;
   // Listed rows for the MFMA scan: their contiguous copy and (L2) its squared norms.
   size_t cx = 0, cn = 0;
+  size_t qf = 0;  // wide form of the 16-bit scan: the split queries
   // k above kExactMaxK: sort_chunk queries per pass; two key buffers, segment offsets, sort scratch.
   uint64_t sort_chunk = 0;
   size_t skeys = 0, soff = 0, stmp = 0;
@@ -2753,7 +2758,7 @@ struct FlatPlan {
   size_t total() const {
     return aligned(stage) + aligned(q) + aligned(qn) + aligned(delta) + aligned(pd) + aligned(pr) + aligned(thr) +
            aligned(fb) + aligned(mflag) + 2 * aligned(skeys) + aligned(soff) + aligned(stmp) + aligned(cx) +
-           aligned(cn);
+           aligned(cn) + aligned(qf);
   }
 };
 
@@ -2774,6 +2779,7 @@ struct FlatBuffers {
   void* stmp = nullptr;
   float* cx = nullptr;
   float* cn = nullptr;
+  void* qf = nullptr;
 };
 
 /// Row splits for `qblocks` query blocks over `tiles` row tiles: one work-group per CU at a time, so
@@ -2804,9 +2810,10 @@ uint64_t choose_splits(uint64_t qblocks, uint64_t tiles, uint64_t max_splits, in
   return pick;
 }
 
-/// d_idx (listed admitted rows) is in use when n_idx > 0 or `indexed`.
+/// d_idx (listed admitted rows) is in use when n_idx > 0 or `indexed`. half_wide = false keeps rows wider
+/// than kHalfMaxDp on the fp32 scan, which needs no split queries.
 FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool indexed, bool filtered, uint64_t n_idx,
-                          int cus) {
+                          int cus, bool half_wide = true) {
   QVH_REQUIRE(nq <= 0xFFFFFFFFull, "flat search: too many queries in one call");
   FlatPlan p;
   if (k > kExactMaxK) {
@@ -2873,11 +2880,13 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
   p.qn = nq * sizeof(float);
   p.delta = nq * sizeof(float);
   p.kl = p.wide ? 32 : shared_list_length(k);
-  p.half = !ring && f->dp <= kHalfMaxDp && (!p.wide || wide_selection(k) <= kHalfMaxSel);
+  p.half = !ring && f->dp <= (half_wide ? kHalfWideMaxDp : kHalfMaxDp) && (!p.wide || wide_selection(k) <= kHalfMaxSel);
+  p.half_wide = p.half && f->dp > kHalfMaxDp;
   // The ring scan takes the margin's lists for integer stores too (exact distances certify with any
   // list length): a second, gated launch of its scan and merge would cost more than it saves.
-  p.kl_exact =
-      !p.wide && !ring && (p.half ? f->half_integral_rows : f->integral_rows) ? exact_list_length(k) : 0;
+  p.kl_exact = !p.wide && !ring && !p.half_wide && (p.half ? f->half_integral_rows : f->integral_rows)
+                   ? exact_list_length(k)
+                   : 0;
   p.qblocks = static_cast<uint32_t>(ceil_div(nq, kQueriesPerBlock));
   p.scan_rows = indexed ? n_idx : f->n;
   if (ring) {
@@ -2902,7 +2911,13 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
   p.pr = parts * sizeof(uint32_t);
   p.thr = nq * (p.ring ? kRingBoundStride : kScanBoundStride) * sizeof(uint32_t);
   p.fb = (nq + 2) * sizeof(uint32_t);  // count, listed queries, then the launch gate word
-  if (p.half) {
+  if (p.half_wide) {
+    // 256 queries and 256-row tiles per work-group, two lists per query and split: the splits above.
+    p.pair = true;
+    const uint64_t tiles = std::max<uint64_t>(1, ceil_div(p.scan_rows, kHalfWideTileRows));
+    p.rows_per_split = ceil_div(tiles, p.nsplit) * kHalfWideTileRows;
+    p.qf = half_query_frag_bytes(nq, f->dp);
+  } else if (p.half) {
     // 512 queries per work-group (64 per wave) share a tile's conversion and LDS reads; fewer, two
     // waves take the halves of each tile for the same queries, up to 128 in 32-query groups (more
     // waves at work). Lists of 32 leave registers for 32 queries per wave. The partial lists stay
@@ -2946,6 +2961,7 @@ FlatBuffers handle_buffers(qvh_flat* f, const FlatPlan& p) {
   b.stmp = take(f->w_stmp, p.stmp);
   b.cx = static_cast<float*>(take(f->w_cx, p.cx));
   b.cn = static_cast<float*>(take(f->w_cn, p.cn));
+  b.qf = take(f->w_qf, p.qf);
   return b;
 }
 
@@ -2954,7 +2970,7 @@ FlatBuffers handle_buffers(qvh_flat* f, const FlatPlan& p) {
 /// beforehand) is set when some query's bound is not 0. With thr, also the MFMA scan's words:
 /// thr_stride prune bounds per query in thr and the fallback count in b.fb.
 void flat_prep_queries(qvh_flat* f, const FlatBuffers& b, const float* d_raw, uint64_t nq, hipStream_t s,
-                       bool half = false, uint32_t* any_delta = nullptr, uint32_t* thr = nullptr,
+                       int half = 0, uint32_t* any_delta = nullptr, uint32_t* thr = nullptr,
                        uint32_t thr_stride = 0) {
   const float* qs = d_raw;
   if (f->metric == QVH_METRIC_COSINE) {  // normalized in a copy
@@ -2965,8 +2981,8 @@ void flat_prep_queries(qvh_flat* f, const FlatBuffers& b, const float* d_raw, ui
     qs = b.stage;
   }
   hipLaunchKernelGGL(prep_queries_kernel, dim3(static_cast<unsigned>(ceil_div(nq, 4))), dim3(256), 0, s, qs, b.q, nq,
-                     f->dim, f->dp, b.qn, f->meta.as<uint32_t>(), f->metric == QVH_METRIC_L2 ? 1 : 0, half ? 1 : 0,
-                     b.delta, any_delta, thr != nullptr ? b.fb : nullptr, thr, thr_stride);
+                     f->dim, f->dp, b.qn, f->meta.as<uint32_t>(), f->metric == QVH_METRIC_L2 ? 1 : 0, half, b.delta,
+                     any_delta, thr != nullptr ? b.fb : nullptr, thr, thr_stride);
   QVH_HIP(hipGetLastError());
 }
 
@@ -2985,7 +3001,7 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   // prep (its shared bounds, strided for the ring scan, and the fallback count).
   if (gate) hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, s, gate, 1, 0u);
   if (p.path == FlatPlan::kMfma) {
-    flat_prep_queries(f, b, d_queries, nq, s, p.half, gate, b.thr, p.ring ? kRingBoundStride : kScanBoundStride);
+    flat_prep_queries(f, b, d_queries, nq, s, p.half_wide ? 2 : p.half ? 1 : 0, gate, b.thr, p.ring ? kRingBoundStride : kScanBoundStride);
   } else {
     flat_prep_queries(f, b, d_queries, nq, s);
   }
@@ -3145,12 +3161,21 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
     ha.share_rank = a.share_rank;
     ha.bound_slots = p.wide ? 0 : 1;
     ha.meta = f->meta.as<uint32_t>();
+    if (p.half_wide) {
+      launch_half_query_frags(b.q, a.nq, f->dp, b.thr, b.qf, s);
+      QVH_HIP(hipGetLastError());
+      ha.qfrag = b.qf;
+    }
   }
   auto scan = [&](int kl) {
     if (p.half) {
       ha.gate = a.gate;
       ha.gate_want = a.gate_want;
-      launch_half_scan(kl, gate && kl == p.kl_exact ? 1 : 3, p.pair, sgrid, ha, s);
+      if (p.half_wide) {
+        launch_half_wide_scan(kl, sgrid, ha, s);
+      } else {
+        launch_half_scan(kl, gate && kl == p.kl_exact ? 1 : 3, p.pair, sgrid, ha, s);
+      }
     } else if (p.ring) {
       launch_ring(f->dp, kl, sgrid, a, s);
     } else {
@@ -3664,6 +3689,7 @@ FlatBuffers scratch_buffers(unsigned char* base, const FlatPlan& p) {
   b.stmp = take(p.stmp);
   b.cx = static_cast<float*>(take(p.cx));
   b.cn = static_cast<float*>(take(p.cn));
+  b.qf = take(p.qf);
   return b;
 }
 
@@ -3683,7 +3709,11 @@ qvh_status qvh_flat_search_device_noalloc(qvh_flat* f, const float* d_queries, u
     ScratchSlot& slot = scratch_on(f->device);
     std::lock_guard<std::mutex> use(slot.use);  // after the handle's lock, never before it
     unsigned char* base = static_cast<unsigned char*>(slot.ptr);
-    const FlatPlan p = plan_flat_search(f, nq, k, false, d_row_bitmap != nullptr, 0, device_cus(f->device));
+    FlatPlan p = plan_flat_search(f, nq, k, false, d_row_bitmap != nullptr, 0, device_cus(f->device));
+    // Split queries are taken only where they fit beside the rest.
+    if (p.total() > kScratchBytes) {
+      p = plan_flat_search(f, nq, k, false, d_row_bitmap != nullptr, 0, device_cus(f->device), false);
+    }
     if (p.total() > kScratchBytes) {
       throw Failure(QVH_EINVAL, "qvh_flat_search_device_noalloc: this search needs " + std::to_string(p.total()) +
                                     " bytes of workspace, above the fixed scratch of " +

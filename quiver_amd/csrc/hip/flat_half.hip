@@ -1,4 +1,4 @@
-// Flat exact search for rows of up to 128 dims on the 16-bit matrix unit.
+// Flat exact search on the 16-bit matrix unit.
 //
 // The fp32 matrix instructions run at 157 TFLOP/s, the fp16 ones at 2.5 PFLOP/s with fp32
 // accumulation. A float times a power of two splits into two halves, x = hi + lo with |lo| <= 2^-11
@@ -482,6 +482,293 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
   }
 }
 
+// ---- rows wider than 128 dims -----------------------------------------------------------------
+//
+// A 256-row x 256-query tile per work-group, accumulated over 32-dim chunks: wave w takes 128 rows
+// (half w / 4) and 64 queries (w % 4) in 128 accumulators, so a 16-dim step reads 12 fragments from
+// LDS for 24 matrix instructions (at 64 x 64 per wave the LDS, not the matrix unit, would be the
+// limit). Rows are split into halves on their way into LDS; the queries come split, in fragment
+// order, from a workspace written once per search, since their conversion would cost every
+// work-group as much as the rows'. Selection happens once per tile and touches few values, so the
+// lists live in the output arrays and only a lane with a passing group loads its own.
+//
+// Fragment (row block, step, half) in LDS: 64 slots of 16 bytes; lane (i, h) of the matrix step reads
+// slot 32 h + (i ^ (4 h + 16 step)), a permutation that spreads the row loader's 8-byte stores over
+// the banks.
+
+constexpr int kWideTile = static_cast<int>(kHalfWideTileRows);
+
+__global__ void __launch_bounds__(256) half_query_frags_kernel(const float* __restrict__ Q, uint32_t nq, uint32_t dp,
+                                                               uint32_t steps, const uint32_t* __restrict__ words,
+                                                               f16x8* __restrict__ out) {
+  const uint64_t item = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);  // (query block, step)
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t qb = item / steps;
+  const uint32_t step = static_cast<uint32_t>(item % steps);
+  if (qb >= ceil_div(nq, 32)) return;
+  const uint64_t q = qb * 32 + (lane & 31);
+  const uint32_t c = step * 16 + 8 * (lane >> 5);
+  const bool in = q < nq && c < dp;
+  const float sq = in ? __uint_as_float(words[q * kHalfWordStride + kHalfScaleWord]) : 0.0f;
+  const f32x4* src = reinterpret_cast<const f32x4*>(Q + (in ? q * dp + c : 0));
+  const f32x4 v0 = src[0], v1 = src[1];
+  f16x8 hi, lo;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float v = in ? -sq * (i < 4 ? v0[i & 3] : v1[i & 3]) : 0.0f;
+    hi[i] = static_cast<_Float16>(v);
+    lo[i] = static_cast<_Float16>(v - static_cast<float>(hi[i]));
+  }
+  out[item * 128 + lane] = hi;
+  out[item * 128 + 64 + lane] = lo;
+}
+
+template <int KL>
+__global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a) {
+  constexpr int kFrag = 1024;                            // bytes
+  constexpr int kXBytes = kWideTile / 32 * 2 * 2 * kFrag;  // 8 row blocks x 2 steps x (hi, lo)
+  constexpr int kQBytes = static_cast<int>(kHalfWideQueries) / 32 * 2 * 2 * kFrag;
+  __shared__ __attribute__((aligned(16))) unsigned char s_x[2][kXBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char s_q[2][kQBytes];
+  __shared__ __attribute__((aligned(16))) f16x8 s_aug[2][kWideTile];  // the norm's three halves per row
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, h = lane >> 5;
+  uint32_t qb, split;
+  const uint32_t wg = blockIdx.x;
+  if (a.nsplit % 8 == 0) {  // XCD wg % 8 takes its own splits
+    const uint32_t x = wg % 8, li = wg / 8;
+    split = (li / a.qblocks) * 8 + x;
+    qb = li % a.qblocks;
+  } else {
+    split = wg / a.qblocks;
+    qb = wg % a.qblocks;
+  }
+  const int rhalf = wave >> 2;  // rows 128 rhalf .. + 127 of every tile
+  const uint32_t q0 = qb * kHalfWideQueries + static_cast<uint32_t>(wave & 3) * 64;
+  const bool wave_active = q0 < a.nq;
+  const uint32_t q = q0 + static_cast<uint32_t>(lane);  // the query this lane lists
+  const bool qvalid = q < a.nq;
+  const float sx = half_scale(__uint_as_float(a.meta[0]));
+  f16x8 baug[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const uint32_t qc = q0 + 32 * g + j;
+    const float sq = qc < a.nq ? __uint_as_float(a.words[static_cast<size_t>(qc) * kHalfWordStride + kHalfScaleWord]) : 0.0f;
+    const _Float16 w = static_cast<_Float16>(qc < a.nq && h == 0 && a.l2 ? 256.0f * sq / sx : 0.0f);
+    baug[g] = f16x8{w, w, w, 0, 0, 0, 0, 0};
+  }
+
+  const uint32_t list = split * 2 + static_cast<uint32_t>(rhalf);
+  const uint32_t src = list % kHalfSlots;
+  uint32_t* const qw = a.words + static_cast<size_t>(qvalid ? q : 0u) * kHalfWordStride;
+  float* const my_d = a.part_d + (static_cast<size_t>(qvalid ? q : 0u) * (2 * a.nsplit) + list) * KL;
+  uint32_t* const my_g = a.part_r + (static_cast<size_t>(qvalid ? q : 0u) * (2 * a.nsplit) + list) * KL;
+  if (qvalid) {
+#pragma unroll
+    for (int x = 0; x < KL; ++x) {
+      my_d[x] = __builtin_huge_valf();
+      my_g[x] = QVH_EMPTY_ROW;
+    }
+  }
+  float kth = __builtin_huge_valf(), first = __builtin_huge_valf(), published = __builtin_huge_valf();
+  float pthr = __builtin_huge_valf();
+
+  const uint64_t r0 = static_cast<uint64_t>(split) * a.rows_per_split;
+  const uint64_t r1 = r0 < a.n ? (a.n < r0 + a.rows_per_split ? a.n : r0 + a.rows_per_split) : r0;
+  const uint32_t ntiles = static_cast<uint32_t>(ceil_div(r1 - r0, kWideTile));
+  const uint32_t nchunks = (a.dp + 31) / 32;
+  const uint32_t nsteps = ntiles * nchunks;
+  const uint64_t last_row = r1 > r0 ? r1 - 1 : r0;
+  const uint32_t qblocks32 = static_cast<uint32_t>(ceil_div(a.nq, 32));
+
+  // Loader: 16 bytes (4 dims) of 4 rows per thread, a row's 8 pieces on adjacent lanes, and 64 bytes of
+  // the query fragments. Unconditional loads at clamped addresses.
+  f32x4 xs[4];
+  f32x4 qs[4];
+  float norm = 0.0f;
+  const uint32_t col = static_cast<uint32_t>(tid & 7), row0 = static_cast<uint32_t>(tid >> 3);
+  auto load_step = [&](uint32_t t, uint32_t c) {
+    const uint64_t base = r0 + static_cast<uint64_t>(t) * kWideTile;
+    const uint32_t d = c * 32 + col * 4;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      uint64_t gr = base + row0 + 64 * p;
+      gr = gr < last_row ? gr : last_row;
+      xs[p] = *reinterpret_cast<const f32x4*>(a.X + gr * a.dp + (d < a.dp ? d : 0u));
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t unit = static_cast<uint32_t>(tid + p * kThreads);  // 256 units per 32 queries
+      uint32_t b = qb * (kHalfWideQueries / 32) + unit / 256;
+      b = b < qblocks32 ? b : qblocks32 - 1;
+      qs[p] = reinterpret_cast<const f32x4*>(a.qfrag)[(static_cast<size_t>(b) * (2 * nchunks) + 2 * c) * 128 + unit % 256];
+    }
+    if (c == 0 && a.l2) {
+      uint64_t gn = base + static_cast<uint32_t>(tid & (kWideTile - 1));
+      gn = gn < last_row ? gn : last_row;
+      norm = a.xnorm[gn];
+    }
+  };
+  auto store_step = [&](uint32_t t, uint32_t c, int buf) {
+    const uint32_t step = col >> 2, hh = (col >> 1) & 1u;
+    const float s = c * 32 + col * 4 < a.dp ? sx : 0.0f;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t row = row0 + 64 * p, i = (row >> 2 & 3u) << 3 | (row >> 4 & 1u) << 2 | (row & 3u);
+      typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+      f16x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = s * xs[p][e];
+        hi[e] = static_cast<_Float16>(v);
+        lo[e] = static_cast<_Float16>(v - static_cast<float>(hi[e]));
+      }
+      const uint32_t at = ((row >> 5) * 2 + step) * 2 * kFrag + (32 * hh + (i ^ (4 * hh + 16 * step))) * 16 + (col & 1u) * 8;
+      *reinterpret_cast<f16x4*>(&s_x[buf][at]) = hi;
+      *reinterpret_cast<f16x4*>(&s_x[buf][at + kFrag]) = lo;
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) *reinterpret_cast<f32x4*>(&s_q[buf][(tid + p * kThreads) * 16]) = qs[p];
+    if (c == 0 && tid < kWideTile) {
+      float v = norm * sx * sx * 0x1p-9f;
+      f16x8 n = {};
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        n[e] = static_cast<_Float16>(v);
+        v -= static_cast<float>(n[e]);
+      }
+      const uint32_t row = static_cast<uint32_t>(tid);
+      s_aug[t & 1][(row & ~31u) | (row >> 2 & 3u) << 3 | (row >> 4 & 1u) << 2 | (row & 3u)] = n;
+    }
+  };
+
+  if (nsteps > 0) {
+    load_step(0, 0);
+    store_step(0, 0, 0);
+  }
+  __syncthreads();
+
+  f32x16 acc[4][2];
+  uint32_t t = 0, c = 0;
+  for (uint32_t i = 0; i < nsteps; ++i) {
+    const int buf = static_cast<int>(i & 1);
+    const uint32_t nc = c + 1 == nchunks ? 0u : c + 1, nt = c + 1 == nchunks ? t + 1 : t;
+    if (i + 1 < nsteps) load_step(nt, nc);
+    if (wave_active) {
+      if (c == 0) {
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          acc[rb][0] = f32x16{};
+          acc[rb][1] = f32x16{};
+        }
+      }
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        const unsigned char* qbase = &s_q[buf][((2 * (wave & 3)) * 2 + kk) * 2 * kFrag + lane * 16];
+        const f16x8 bh0 = *reinterpret_cast<const f16x8*>(qbase), bl0 = *reinterpret_cast<const f16x8*>(qbase + kFrag);
+        const f16x8 bh1 = *reinterpret_cast<const f16x8*>(qbase + 4 * kFrag);
+        const f16x8 bl1 = *reinterpret_cast<const f16x8*>(qbase + 5 * kFrag);
+        const unsigned char* xbase = &s_x[buf][(4 * rhalf * 2 + kk) * 2 * kFrag + (32 * h + (j ^ (4 * h + 16 * kk))) * 16];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          const f16x8 ah = *reinterpret_cast<const f16x8*>(xbase + rb * 4 * kFrag);
+          const f16x8 al = *reinterpret_cast<const f16x8*>(xbase + rb * 4 * kFrag + kFrag);
+          acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh0, acc[rb][0], 0, 0, 0);
+          acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh1, acc[rb][1], 0, 0, 0);
+          acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl0, acc[rb][0], 0, 0, 0);
+          acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl1, acc[rb][1], 0, 0, 0);
+          acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh0, acc[rb][0], 0, 0, 0);
+          acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh1, acc[rb][1], 0, 0, 0);
+        }
+      }
+      if (c + 1 == nchunks) {
+        const uint64_t wave_row0 = r0 + static_cast<uint64_t>(t) * kWideTile + 128 * static_cast<uint64_t>(rhalf);
+        float m[8];  // the minima of this lane's query over the wave's eight 16-row groups
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          if (a.l2) {
+            const f16x8 xn = s_aug[t & 1][128 * rhalf + 32 * rb + j];
+            acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xn, baug[0], acc[rb][0], 0, 0, 0);
+            acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xn, baug[1], acc[rb][1], 0, 0, 0);
+          }
+          const uint64_t block0 = wave_row0 + 32 * static_cast<uint64_t>(rb);
+          uint32_t bits = block0 >= r1 ? 0u : r1 - block0 < 32 ? (1u << (r1 - block0)) - 1u : 0xFFFFFFFFu;
+          if (a.bitmap && bits) bits &= static_cast<uint32_t>(a.bitmap[block0 >> 6] >> (block0 & 32));
+          bits = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(bits)));
+          if (bits != 0xFFFFFFFFu) {
+            const uint32_t lb = bits >> (16 * h);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              acc[rb][0][r] = (lb >> r) & 1u ? acc[rb][0][r] : __builtin_huge_valf();
+              acc[rb][1][r] = (lb >> r) & 1u ? acc[rb][1][r] : __builtin_huge_valf();
+            }
+          }
+          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(min16(acc[rb][0])),
+                                                           __float_as_uint(min16(acc[rb][1])), false, false);
+          m[2 * rb] = __uint_as_float(sw[0]);
+          m[2 * rb + 1] = __uint_as_float(sw[1]);
+        }
+        const float thr = fminf(pthr, kth);
+        bool any = false;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) any = any || (m[e] <= thr && m[e] < __builtin_huge_valf());
+        if (qvalid && any) {
+          float Ld[KL];
+          uint32_t Lg[KL];
+#pragma unroll
+          for (int x = 0; x < KL; ++x) {
+            Ld[x] = my_d[x];
+            Lg[x] = my_g[x];
+          }
+          const uint32_t group0 = static_cast<uint32_t>(wave_row0 / kHalfGroupRows);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            if (m[e] <= thr && m[e] < Ld[KL - 1]) group_insert<KL>(Ld, Lg, m[e], group0 + e);
+          }
+#pragma unroll
+          for (int x = 0; x < KL; ++x) {
+            my_d[x] = Ld[x];
+            my_g[x] = Lg[x];
+          }
+          kth = Ld[KL - 1];
+          first = Ld[0];
+        }
+        // Bounds through the query's words, as the narrow scan does; a tile is long enough to do so
+        // after each. Where the merge takes more than KL groups (share_rank set) only this list's own
+        // bound prunes.
+        if (a.share && a.share_rank == 0 && qvalid) {
+          const uint32_t g = __hip_atomic_fetch_min(qw, float_to_ordered(kth), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          float b = ordered_to_float(g);
+          if (a.bound_slots) {
+            if (first < published) {
+              published = first;
+              __hip_atomic_fetch_min(qw + kHalfSlotBase + src, float_to_ordered(first), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+            }
+            b = fminf(b, ordered_to_float(slots_kth_smallest<KL>(qw + kHalfSlotBase)));
+          }
+          pthr = fminf(pthr, b);
+        }
+      }
+    }
+    if (i + 1 < nsteps) store_step(nt, nc, buf ^ 1);
+    t = nt;
+    c = nc;
+    __syncthreads();
+  }
+
+  if (qvalid) {
+    const float iq = 1.0f / __uint_as_float(qw[kHalfScaleWord]), ix = 1.0f / sx;
+    const float qn = a.l2 ? a.qnorm[q] : 1.0f;
+#pragma unroll
+    for (int x = 0; x < KL; ++x) {
+      if (my_g[x] != QVH_EMPTY_ROW) my_d[x] = (a.l2 ? 2.0f : 1.0f) * (my_d[x] * iq * ix) + qn;
+    }
+  }
+}
+
 // ---- merge: the best groups, scored exactly ---------------------------------------------------
 
 constexpr int kListsPerLane = static_cast<int>(kHalfMaxLists) / 64;
@@ -714,6 +1001,21 @@ void launch_half_scan(int kl, int products, bool pair, dim3 grid, const HalfScan
     case 7: launch_nk<7>(kl, products, pair, grid, a, s); break;
     case 8: launch_nk<8>(kl, products, pair, grid, a, s); break;
     default: throw Failure(QVH_EUNSUPPORTED, "half scan: unsupported row width");
+  }
+}
+
+void launch_half_query_frags(const float* Q, uint32_t nq, uint32_t dp, const uint32_t* words, void* out,
+                             hipStream_t s) {
+  const uint64_t steps = half_wide_steps(dp), items = ceil_div(nq, 32) * steps;
+  hipLaunchKernelGGL(half_query_frags_kernel, dim3(static_cast<unsigned>(ceil_div(items, 4))), dim3(256), 0, s, Q, nq,
+                     dp, static_cast<uint32_t>(steps), words, static_cast<f16x8*>(out));
+}
+
+void launch_half_wide_scan(int kl, dim3 grid, const HalfScanArgs& a, hipStream_t s) {
+  if (kl == 16) {
+    hipLaunchKernelGGL(flat_half_wide_kernel<16>, grid, dim3(kThreads), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(flat_half_wide_kernel<32>, grid, dim3(kThreads), 0, s, a);
   }
 }
 

@@ -5,11 +5,16 @@
 
 #include <cstdint>
 
+#include "common.hpp"
+
 namespace qvh {
 
 constexpr uint32_t kHalfMaxDp = 128;      // register-resident query width
 constexpr uint32_t kHalfGroupRows = 16;   // rows per listed group
 constexpr uint32_t kHalfTileRows = 64;
+constexpr uint32_t kHalfWideTileRows = 256;    // rows wider than kHalfMaxDp: 256 rows x 256 queries
+constexpr uint32_t kHalfWideQueries = 256;     // per work-group
+constexpr uint32_t kHalfWideMaxDp = 4096;
 constexpr uint32_t kHalfMaxLists = 512;   // lists per query the merge takes
 constexpr uint32_t kHalfMaxSel = 64;      // groups the merge selects per query at most
 // The scan's words per query in `words`: word 0 the union bound, kHalfSlotBase and up the bound slots,
@@ -55,6 +60,7 @@ struct HalfScanArgs {
   const uint32_t* meta;  // store meta: [0] largest squared norm (float bits)
   const uint32_t* gate;  // the launch runs when (*gate != 0) == (gate_want != 0); null: always
   uint32_t gate_want;
+  const void* qfrag;  // wide rows: the split queries (launch_half_query_frags)
 };
 
 struct HalfMergeArgs {
@@ -87,6 +93,15 @@ inline uint32_t half_lists_per_split(bool pair) { return pair ? 2u : 1u; }
 /// One scan launch. kl: 10, 16 or 32 (32 only with `pair`). products: 1 (every operand exact in
 /// 16 bits) or 3.
 void launch_half_scan(int kl, int products, bool pair, dim3 grid, const HalfScanArgs& a, hipStream_t s);
+
+/// Rows wider than kHalfMaxDp (dp a multiple of 16): bytes of the split queries, the kernel that writes
+/// them, and the scan (lists of 16 or 32 groups, two per query and split).
+inline uint64_t half_wide_steps(uint32_t dp) { return (dp + 31) / 32 * 2; }  // 16-dim steps, whole 32-dim chunks
+inline size_t half_query_frag_bytes(uint64_t nq, uint32_t dp) { return ceil_div(nq, 32) * half_wide_steps(dp) * 2048; }
+void launch_half_query_frags(const float* Q, uint32_t nq, uint32_t dp, const uint32_t* words, void* out,
+                             hipStream_t s);
+void launch_half_wide_scan(int kl, dim3 grid, const HalfScanArgs& a, hipStream_t s);
+
 void launch_half_merge(int kl, const HalfMergeArgs& m, hipStream_t s);
 
 }  // namespace qvh

@@ -1,7 +1,8 @@
 """The flat scan on the 16-bit matrix unit, at the sizes where its split of the work changes: row
 widths around its 16-dim steps (8-dim padding included), batches around its 128-, 256- and 512-query
-blocks, row counts around its 16-row groups and 64-row tiles, list lengths (k 10/11, 21/22, 43), and
-magnitudes far from 1. Distances must equal the oracle's bit for bit and labels must agree within
+blocks, row counts around its 16-row groups and 64-row tiles, list lengths (k 10/11, 21/22, 43),
+magnitudes far from 1, and for rows wider than 128 dims around the 32-dim chunks, 256-row tiles and
+64- and 256-query blocks. Distances must equal the oracle's bit for bit and labels must agree within
 equal-distance groups, so no tolerance is involved."""
 
 import numpy as np
@@ -88,3 +89,23 @@ def test_equal_rows(oracle):
     q = np.round(20.0 * _normal(rng, 200, 16))
     _check(oracle, np.repeat(base, 40, axis=0), q, 10, "l2")
     _check(oracle, np.tile(base, (40, 1)), q, 10, "l2")
+
+
+@pytest.mark.parametrize("dim", [129, 144, 145, 160, 161, 300, 1_000])
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_wide_row_widths(oracle, dim, metric):
+    rng = np.random.default_rng(dim)
+    base, q = _normal(rng, 3_001, dim), _normal(rng, 77, dim)
+    _check(oracle, base, q, 10, metric)
+    _check(oracle, base, q, 40, metric)
+
+
+@pytest.mark.parametrize("nq", [33, 63, 64, 65, 255, 256, 257, 600])
+@pytest.mark.parametrize("n", [1, 16, 255, 256, 257, 2_000])
+def test_wide_blocks_and_filters(oracle, nq, n):
+    rng = np.random.default_rng(nq * n)
+    base, q = _normal(rng, n, 130), np.ldexp(_normal(rng, nq, 130), rng.integers(-6, 7, (nq, 1))).astype(np.float32)
+    _check(oracle, base, q, 11, "l2")
+    _check(oracle, base, q, 25, "cosine")
+    _check(oracle, base, q, 10, "l2", np.arange(0, n, 3, dtype=np.uint64))
+    _check(oracle, np.round(2.0 * base), np.round(2.0 * q / np.abs(q).max()), 10, "l2")
