@@ -40,6 +40,9 @@ constexpr int kTile = static_cast<int>(kHalfTileRows);
 // Queued groups per lane before a wave-wide flush (a 32-row block queues up to two). The queue arrays
 // also carry the hand-off of two row waves: four query groups' lists, 4 * 64 * KL entries.
 constexpr int queue_cap(int kl) { return kl > 16 ? 16 : 8; }
+/// The three-product form with 64 queries per wave has no registers left for its lists: they live in
+/// LDS, and a flush brings a lane's list into the accumulators' registers and back.
+constexpr bool lists_in_lds(int np, int qg) { return np == 3 && qg == 2; }
 
 /// Inserts (d, g) into the sorted list (the caller has checked d <= Ld[KL - 1]); a lane's groups come in
 /// increasing order, so an equal minimum already listed stays ahead. One parallel step: every
@@ -73,47 +76,19 @@ __device__ __forceinline__ void group_insert_any(float (&Ld)[KL], uint32_t (&Lg)
   Lg[0] = lt[0] ? g : Lg[0];
 }
 
-/// Sorts N values ascending in registers (a bitonic network).
-template <int N>
-__device__ __forceinline__ void sort_u32(uint32_t (&v)[N]) {
-#pragma unroll
-  for (int size = 2; size <= N; size <<= 1) {
-#pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const int l = i ^ stride;
-        if (l > i) {
-          const uint32_t lo = min(v[i], v[l]), hi = max(v[i], v[l]);
-          const bool up = (i & size) == 0;
-          v[i] = up ? lo : hi;
-          v[l] = up ? hi : lo;
-        }
-      }
-    }
-  }
-}
-
-/// The K-th smallest of a query's 32 bound slots.
+/// The largest of the query's first K bound slots. Each holds the smallest minimum any of its sources
+/// has found, so K different groups lie at or below it.
 template <int K>
-__device__ __forceinline__ uint32_t slots_kth_smallest(const uint32_t* slots) {
-  uint32_t v[32];
+__device__ __forceinline__ uint32_t slots_bound(const uint32_t* slots) {
+  static_assert(K % 2 == 0 && K <= static_cast<int>(kHalfSlots), "whole 8-byte words");
+  uint32_t m = 0;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
+  for (int i = 0; i < K / 2; ++i) {
     const uint64_t w = __hip_atomic_load(reinterpret_cast<const uint64_t*>(slots) + i, __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
-    v[2 * i] = static_cast<uint32_t>(w);
-    v[2 * i + 1] = static_cast<uint32_t>(w >> 32);
+    m = max(m, max(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32)));
   }
-  if constexpr (K == 32) {
-    uint32_t m = v[0];
-#pragma unroll
-    for (int i = 1; i < 32; ++i) m = max(m, v[i]);
-    return m;
-  } else {
-    sort_u32<32>(v);
-    return v[K - 1];
-  }
+  return m;
 }
 
 /// Minimum of 16 accumulators.
@@ -144,10 +119,13 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
   __shared__ __attribute__((aligned(16))) _Float16 s_lo[NP == 3 ? 2 : 1][NP == 3 ? kTile * STRIDE : 8];
   __shared__ uint64_t s_bits[2];
   // Queued (minimum, group) per lane, entry-major.
-  constexpr int kCap = queue_cap(KL);
-  static_assert(4 * 64 * KL <= kCap * kThreads, "the row waves' hand-off fits the queue arrays");
+  constexpr bool kLdsLists = lists_in_lds(NP, QG);
+  constexpr int kCap = kLdsLists ? 4 : queue_cap(KL);
   __shared__ float s_qd[kCap * kThreads];
   __shared__ uint32_t s_qg[kCap * kThreads];
+  __shared__ float s_ld[kLdsLists ? KL * kThreads : 1];  // entry-major
+  __shared__ uint32_t s_lg[kLdsLists ? KL * kThreads : 1];
+  static_assert(kLdsLists || 4 * 64 * KL <= kCap * kThreads, "the row waves' hand-off fits the queue arrays");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -204,19 +182,27 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
     baug[g] = f16x8{w, w, w, 0, 0, 0, 0, 0};
   }
 
-  float Ld[KL];
-  uint32_t Lg[KL];
+  // The lane's list, ascending; in LDS form only its first and last minima stay in registers.
+  constexpr int kRegs = kLdsLists ? 1 : KL;
+  float Ld[kRegs];
+  uint32_t Lg[kRegs];
 #pragma unroll
   for (int x = 0; x < KL; ++x) {
-    Ld[x] = __builtin_huge_valf();
-    Lg[x] = QVH_EMPTY_ROW;
+    if constexpr (kLdsLists) {
+      s_ld[x * kThreads + tid] = __builtin_huge_valf();
+      s_lg[x * kThreads + tid] = QVH_EMPTY_ROW;
+    } else {
+      Ld[x] = __builtin_huge_valf();
+      Lg[x] = QVH_EMPTY_ROW;
+    }
   }
+  float first = __builtin_huge_valf(), kth = __builtin_huge_valf();
 
   // Prune threshold: the smaller of this list's KL-th minimum and the shared per-query value. Any
   // list's KL-th bounds the KL-th of the union of all lists, so groups above it can never be among
   // the query's KL best (equal minima pass: ties are decided by group). Bound slots: every list
-  // publishes its best minimum to one of the query's 32 slots; different slots hold minima of
-  // different groups, so the KL-th smallest slot bounds the query's KL-th best minimum from above.
+  // publishes its best minimum to one of the query's first KL slots; different slots hold minima of
+  // different groups, so the largest of them bounds the query's KL-th best minimum from above.
   uint32_t* const qw = a.words + static_cast<size_t>(qvalid ? q : 0u) * kHalfWordStride;
   float pthr = __builtin_huge_valf();
   if (qvalid && a.share) {
@@ -224,10 +210,10 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
   }
   constexpr uint32_t kLists = QG == 2 ? 1u : 2u;  // per split and query
   const uint32_t list = split * kLists + (QG == 2 ? 0u : static_cast<uint32_t>(h));
-  const uint32_t src = (list * rw + rslot) % kHalfSlots;
+  const uint32_t src = (list * rw + rslot) % KL;
   float published = __builtin_huge_valf();
   auto share_threshold = [&]() {
-    float t = Ld[KL - 1];
+    float t = kth;
     if constexpr (QG == 1) {
       // The lane pair's lists hold disjoint groups: their union has KL at or below
       // max(own[KL/2-1], other[KL/2-1]) as well as below either list's KL-th.
@@ -247,12 +233,12 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
       const uint32_t g = __hip_atomic_fetch_min(qw, float_to_ordered(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       t = fminf(t, ordered_to_float(g));
       if (a.bound_slots) {
-        if (Ld[0] < published) {
-          published = Ld[0];
+        if (first < published) {
+          published = first;
           __hip_atomic_fetch_min(qw + kHalfSlotBase + src, float_to_ordered(published), __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
         }
-        t = fminf(t, ordered_to_float(slots_kth_smallest<KL>(qw + kHalfSlotBase)));
+        t = fminf(t, ordered_to_float(slots_bound<KL>(qw + kHalfSlotBase)));
       }
     }
     pthr = fminf(pthr, t);
@@ -264,14 +250,36 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
     int m = qcount;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
-    for (int e = 0; e < m; ++e) {
-      if (e < qcount) {
-        const float v = s_qd[e * kThreads + tid];
-        if (v < Ld[KL - 1]) group_insert<KL>(Ld, Lg, v, s_qg[e * kThreads + tid]);
+    if (m == 0) return;
+    auto insert_queued = [&](float(&D)[KL], uint32_t(&G)[KL]) {
+      for (int e = 0; e < m; ++e) {
+        if (e < qcount) {
+          const float v = s_qd[e * kThreads + tid];
+          if (v < D[KL - 1]) group_insert<KL>(D, G, v, s_qg[e * kThreads + tid]);
+        }
       }
+      first = D[0];
+      kth = D[KL - 1];
+    };
+    if constexpr (kLdsLists) {
+      float D[KL];
+      uint32_t G[KL];
+#pragma unroll
+      for (int x = 0; x < KL; ++x) {
+        D[x] = s_ld[x * kThreads + tid];
+        G[x] = s_lg[x * kThreads + tid];
+      }
+      insert_queued(D, G);
+#pragma unroll
+      for (int x = 0; x < KL; ++x) {
+        s_ld[x * kThreads + tid] = D[x];
+        s_lg[x * kThreads + tid] = G[x];
+      }
+    } else {
+      insert_queued(Ld, Lg);
     }
     qcount = 0;
-    thr = fminf(pthr, Ld[KL - 1]);
+    thr = fminf(pthr, kth);
   };
 
   const uint64_t r0 = static_cast<uint64_t>(split) * a.rows_per_split;
@@ -345,12 +353,23 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
   if (ntiles > 0) {
     load_tile(0);
     store_tile(0);
+    if (ntiles > 1) load_tile(1);
   }
   __syncthreads();
 
+  // The next tile is converted into the other buffer in the middle of this one: its loads went out a
+  // whole tile earlier, nothing waits for them next to the barrier, and the two waves of a SIMD
+  // (w and w + 4) convert at different times, one's conversion beside the other's matrix steps.
+  const int convert_at = wave < 4 ? 0 : 1;
   for (uint32_t t = 0; t < ntiles; ++t) {
     const int buf = static_cast<int>(t & 1);
-    if (t + 1 < ntiles) load_tile(t + 1);
+    auto convert_next = [&]() {
+      if (t + 1 < ntiles) {
+        store_tile(buf ^ 1);
+        if (t + 2 < ntiles) load_tile(t + 2);
+      }
+    };
+    if (convert_at == 0 || !wave_active) convert_next();
     if (wave_active) {
       const uint64_t tile_row0 = r0 + static_cast<uint64_t>(t) * kTile;
       const uint64_t left = r1 - tile_row0;
@@ -360,33 +379,68 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(admit)));
       for (int blk = blk0; blk < blk1; ++blk) {
         const _Float16* ah = &s_hi[buf][(32 * blk + j) * STRIDE + 8 * h];
+        // Every lane reads its row's norm parts; the upper half's weights are zero.
+        const _Float16* an = &s_hi[buf][(32 * blk + j) * STRIDE + 16 * NK];
+        auto frag = [](const _Float16* p) { return *reinterpret_cast<const f16x8*>(p); };
         f32x16 acc[QG];
 #pragma unroll
         for (int g = 0; g < QG; ++g) acc[g] = f32x16{};
-        if constexpr (NP == 3) {
+        // The LDS reads run ahead of the matrix steps that use them (a read takes longer than a
+        // step's two or four matrix instructions); the scheduling barriers keep the compiler from
+        // pulling each read down to its use. The norm step is last: without L2 its weights are zero.
+        if constexpr (NP == 1) {
+          f16x8 x[NK + 1];
+#pragma unroll
+          for (int kk = 0; kk < NK; ++kk) x[kk] = frag(ah + 16 * kk);
+          x[NK] = frag(an);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int kk = 0; kk <= NK; ++kk) {
+#pragma unroll
+            for (int g = 0; g < QG; ++g) {
+              acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[kk], kk < NK ? bh[g][kk] : baug[g], acc[g], 0, 0, 0);
+            }
+          }
+        } else {
           // The small products first: their roundings are 2^-11 of the sum's.
           const _Float16* al = &s_lo[buf][(32 * blk + j) * STRIDE + 8 * h];
+          constexpr int AHEAD = 2;
+          f16x8 xh[AHEAD + 1], xl[AHEAD + 1];
+#pragma unroll
+          for (int kk = 0; kk < AHEAD && kk < NK; ++kk) {
+            xh[kk] = frag(ah + 16 * kk);
+            xl[kk] = frag(al + 16 * kk);
+          }
 #pragma unroll
           for (int kk = 0; kk < NK; ++kk) {
-            const f16x8 xh = *reinterpret_cast<const f16x8*>(ah + 16 * kk);
-            const f16x8 xl = *reinterpret_cast<const f16x8*>(al + 16 * kk);
+            if (kk + AHEAD < NK) {
+              xh[(kk + AHEAD) % (AHEAD + 1)] = frag(ah + 16 * (kk + AHEAD));
+              xl[(kk + AHEAD) % (AHEAD + 1)] = frag(al + 16 * (kk + AHEAD));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const f16x8 vh = xh[kk % (AHEAD + 1)], vl = xl[kk % (AHEAD + 1)];
 #pragma unroll
-            for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, bh[g][kk], acc[g], 0, 0, 0);
+            for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, bh[g][kk], acc[g], 0, 0, 0);
 #pragma unroll
-            for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, bl[g][kk], acc[g], 0, 0, 0);
+            for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, bl[g][kk], acc[g], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
           }
-        }
+          constexpr int AHEAD2 = 4;
+          f16x8 x[AHEAD2 + 1];
+          auto step = [&](int kk) { return frag(kk < NK ? ah + 16 * kk : an); };
 #pragma unroll
-        for (int kk = 0; kk < NK; ++kk) {
-          const f16x8 xh = *reinterpret_cast<const f16x8*>(ah + 16 * kk);
+          for (int kk = 0; kk < AHEAD2 && kk <= NK; ++kk) x[kk] = step(kk);
 #pragma unroll
-          for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, bh[g][kk], acc[g], 0, 0, 0);
-        }
-        if (a.l2) {
-          // Every lane reads its row's norm parts; the upper half's weights are zero.
-          const f16x8 xn = *reinterpret_cast<const f16x8*>(&s_hi[buf][(32 * blk + j) * STRIDE + 16 * NK]);
+          for (int kk = 0; kk <= NK; ++kk) {
+            if (kk + AHEAD2 <= NK) x[(kk + AHEAD2) % (AHEAD2 + 1)] = step(kk + AHEAD2);
+            __builtin_amdgcn_sched_barrier(0);
+            const f16x8 v = x[kk % (AHEAD2 + 1)];
 #pragma unroll
-          for (int g = 0; g < QG; ++g) acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xn, baug[g], acc[g], 0, 0, 0);
+            for (int g = 0; g < QG; ++g) {
+              acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, kk < NK ? bh[g][kk] : baug[g], acc[g], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
         const uint32_t bits = static_cast<uint32_t>(admit >> (32 * blk));
         if (bits != 0xFFFFFFFFu) {  // wave-uniform: a filter, or the split's last rows
@@ -432,40 +486,59 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
             }
           }
         }
+        if (convert_at == 1 && blk == blk0) convert_next();
       }
-      // Bounds are exchanged after tiles 0, 1, 3, 7, 15, 31 and 63 (the first rows move a bound the
-      // most), then every 64: an exchange waits for a device-scope round trip.
-      if (t < 64 ? (t & (t + 1)) == 0 : t % 64 == 63) {
+      // Bounds are exchanged after tiles 0, 1, 3, 7, ... (the first rows move a bound the most), then
+      // every 32, or every 8 where an exchange is one atomic and no slots. An exchange waits for a
+      // device-scope round trip (1M x 128, 10,000 queries, with slots: every 64 tiles 3.41-3.51 ms a
+      // search, 32 3.43, 16 3.59, 8 3.86; 300,007 x 96, 1,003 queries, k = 30, without: 0.88-0.99, 0.95,
+      // 0.81, 0.72).
+      const uint32_t period = a.bound_slots ? 32u : 8u;
+      if (t < period ? (t & (t + 1)) == 0 : t % period == period - 1) {
         flush_queue();
         if (a.share) {
           share_threshold();
-          thr = fminf(pthr, Ld[KL - 1]);
+          thr = fminf(pthr, kth);
         }
       }
     }
-    if (t + 1 < ntiles) store_tile(buf ^ 1);
     __syncthreads();
   }
 
   if (wave_active) flush_queue();
+  float D[KL];
+  uint32_t G[KL];
+#pragma unroll
+  for (int x = 0; x < KL; ++x) {
+    if constexpr (kLdsLists) {
+      D[x] = s_ld[x * kThreads + tid];
+      G[x] = s_lg[x * kThreads + tid];
+    } else {
+      D[x] = Ld[x];
+      G[x] = Lg[x];
+    }
+  }
   if (rw == 2) {
-    // The wave of the second halves hands its lists to the one of the first through the queue
-    // arrays, free once every wave has flushed.
+    // The wave of the second halves (w + 4) hands its lists to the one of the first: through the
+    // queue arrays, free once every wave has flushed, or where they are, in LDS.
+    float* const hd = kLdsLists ? s_ld : s_qd;
+    uint32_t* const hg = kLdsLists ? s_lg : s_qg;
+    const uint32_t stride = kLdsLists ? kThreads : kThreads / 2;  // entry-major, 256 lanes hand over
+    const uint32_t at = qgroup * 64 + static_cast<uint32_t>(lane) + (kLdsLists ? 256u : 0u);  // qgroup < 4
     __syncthreads();
-    const uint32_t at = (qgroup * 64 + static_cast<uint32_t>(lane)) * KL;  // qgroup < 4
-    if (rslot == 1) {
+    if (!kLdsLists && rslot == 1) {
 #pragma unroll
       for (int x = 0; x < KL; ++x) {
-        s_qd[at + x] = Ld[x];
-        s_qg[at + x] = Lg[x];
+        hd[x * stride + at] = D[x];
+        hg[x * stride + at] = G[x];
       }
     }
     __syncthreads();
     if (rslot == 1) return;
     for (int x = 0; x < KL; ++x) {
-      const float d = s_qd[at + x];
-      if (!__builtin_amdgcn_ballot_w64(d <= Ld[KL - 1] && d < __builtin_huge_valf())) break;
-      group_insert_any<KL>(Ld, Lg, d, s_qg[at + x]);
+      const float d = hd[x * stride + at];
+      if (!__builtin_amdgcn_ballot_w64(d <= D[KL - 1] && d < __builtin_huge_valf())) break;
+      group_insert_any<KL>(D, G, d, hg[x * stride + at]);
     }
   }
   if (qvalid) {
@@ -475,9 +548,9 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
     const size_t o = (static_cast<size_t>(q) * (a.nsplit * kLists) + list) * KL;
 #pragma unroll
     for (int x = 0; x < KL; ++x) {
-      const float v = (a.l2 ? 2.0f : 1.0f) * (Ld[x] * iq * ix) + qn;
-      a.part_d[o + x] = Lg[x] == QVH_EMPTY_ROW ? __builtin_huge_valf() : v;
-      a.part_r[o + x] = Lg[x];
+      const float v = (a.l2 ? 2.0f : 1.0f) * (D[x] * iq * ix) + qn;
+      a.part_d[o + x] = G[x] == QVH_EMPTY_ROW ? __builtin_huge_valf() : v;
+      a.part_r[o + x] = G[x];
     }
   }
 }
@@ -561,7 +634,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
   }
 
   const uint32_t list = split * 2 + static_cast<uint32_t>(rhalf);
-  const uint32_t src = list % kHalfSlots;
+  const uint32_t src = list % KL;
   uint32_t* const qw = a.words + static_cast<size_t>(qvalid ? q : 0u) * kHalfWordStride;
   float* const my_d = a.part_d + (static_cast<size_t>(qvalid ? q : 0u) * (2 * a.nsplit) + list) * KL;
   uint32_t* const my_g = a.part_r + (static_cast<size_t>(qvalid ? q : 0u) * (2 * a.nsplit) + list) * KL;
@@ -644,9 +717,18 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
     }
   };
 
+  auto after = [&](uint32_t& tt, uint32_t& cc) {  // the step after (tt, cc)
+    if (++cc == nchunks) {
+      cc = 0;
+      ++tt;
+    }
+  };
   if (nsteps > 0) {
     load_step(0, 0);
     store_step(0, 0, 0);
+    uint32_t t1 = 0, c1 = 0;
+    after(t1, c1);
+    if (nsteps > 1) load_step(t1, c1);
   }
   __syncthreads();
 
@@ -654,8 +736,19 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
   uint32_t t = 0, c = 0;
   for (uint32_t i = 0; i < nsteps; ++i) {
     const int buf = static_cast<int>(i & 1);
-    const uint32_t nc = c + 1 == nchunks ? 0u : c + 1, nt = c + 1 == nchunks ? t + 1 : t;
-    if (i + 1 < nsteps) load_step(nt, nc);
+    uint32_t nt = t, nc = c;
+    after(nt, nc);
+    // As in the narrow scan: the next step goes into the other buffer from loads issued a step
+    // earlier, the two waves of a SIMD at different times.
+    auto convert_next = [&]() {
+      if (i + 1 < nsteps) {
+        store_step(nt, nc, buf ^ 1);
+        uint32_t t2 = nt, c2 = nc;
+        after(t2, c2);
+        if (i + 2 < nsteps) load_step(t2, c2);
+      }
+    };
+    if (wave < 4 || !wave_active) convert_next();
     if (wave_active) {
       if (c == 0) {
 #pragma unroll
@@ -682,6 +775,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
           acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh0, acc[rb][0], 0, 0, 0);
           acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh1, acc[rb][1], 0, 0, 0);
         }
+        if (kk == 0 && wave >= 4) convert_next();
       }
       if (c + 1 == nchunks) {
         const uint64_t wave_row0 = r0 + static_cast<uint64_t>(t) * kWideTile + 128 * static_cast<uint64_t>(rhalf);
@@ -747,13 +841,12 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
               __hip_atomic_fetch_min(qw + kHalfSlotBase + src, float_to_ordered(first), __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_AGENT);
             }
-            b = fminf(b, ordered_to_float(slots_kth_smallest<KL>(qw + kHalfSlotBase)));
+            b = fminf(b, ordered_to_float(slots_bound<KL>(qw + kHalfSlotBase)));
           }
           pthr = fminf(pthr, b);
         }
       }
     }
-    if (i + 1 < nsteps) store_step(nt, nc, buf ^ 1);
     t = nt;
     c = nc;
     __syncthreads();
