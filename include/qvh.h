@@ -274,6 +274,17 @@ void qvh_points_destroy(qvh_points* points);
 qvh_status qvh_points_nearest(qvh_points* points, const float* centroids, uint32_t k,
                               int max_inner_product, uint32_t* out_assign);
 
+/* Lloyd iterations of the same points (src/product_quantizer.cc:79-100) with centroids that stay on
+ * the device. The dim columns are `nsub` equal sub-spaces (dim % nsub == 0), each with k centroids of
+ * its own. set installs them ([nsub][k][dim / nsub]); step assigns every point to its nearest centroid
+ * per sub-space (as qvh_points_nearest) and replaces each centroid that got points by their mean:
+ * summed in double in point order, divided by the count, rounded once. counts[nsub][k] receives the
+ * points per centroid; a centroid without points keeps its value. get copies the centroids out. */
+qvh_status qvh_points_set_centroids(qvh_points* points, const float* centroids, uint32_t k,
+                                    uint32_t nsub);
+qvh_status qvh_points_step(qvh_points* points, uint32_t* counts);
+qvh_status qvh_points_get_centroids(qvh_points* points, float* centroids);
+
 /* ------------------------------------------------------------------------------------------ *
  * ProductQuantizer (include/quiver/quantizer.h:59-114, src/product_quantizer.cc:119-217) and
  * nearest_centroid (src/product_quantizer.cc:14-27), over batches: the reference's per-vector

@@ -10,6 +10,7 @@
 #include "qvh.h"
 #include "quiver/common.h"
 #include "quiver/filter.h"
+#include "quiver/quantizer.h"
 #include "quiver/thread_pool.h"
 
 namespace quiver::internal {
@@ -46,5 +47,11 @@ std::vector<std::uint64_t> filter_bitmap(const Filter& filter, std::size_t n, La
   });
   return bits;
 }
+
+/// One k-means per sub-space over the columns of n x dim points (sub-space j: the columns
+/// [j * dim / nsub, (j + 1) * dim / nsub), seeded params.seed + j), each as quiver::kmeans runs it on
+/// those columns alone: nsub x k x (dim / nsub) centroids. n <= k * max_points_per_centroid.
+std::vector<float> kmeans_subspaces(const float* vectors, std::size_t n, std::size_t dim, std::size_t nsub,
+                                    const KMeansParams& params);
 
 }  // namespace quiver::internal

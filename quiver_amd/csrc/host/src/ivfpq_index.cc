@@ -120,7 +120,7 @@ struct IvfPqIndex::Impl {
       std::shared_lock lock(mu);
       QUIVER_CHECK(!trained, "index is already trained");
     }
-    const std::size_t d = params.dim, m = params.m, dsub = d / m;
+    const std::size_t d = params.dim, m = params.m;
     std::vector<float> data(in, in + n * d);
     if (params.metric == Metric::kCosine) normalize_rows(data.data(), n, d);
     KMeansParams kp;
@@ -147,19 +147,11 @@ struct IvfPqIndex::Impl {
                          residuals.begin() + static_cast<std::ptrdiff_t>(j * d));
       }
     }
-    std::vector<float> cb(m * kSubCentroids * dsub);
-    std::vector<float> sub(pq_n * dsub);
-    for (std::size_t j = 0; j < m; ++j) {
-      for (std::size_t i = 0; i < pq_n; ++i) {
-        std::memcpy(sub.data() + i * dsub, residuals.data() + i * d + j * dsub, dsub * sizeof(float));
-      }
-      KMeansParams sp;
-      sp.k = kSubCentroids;
-      sp.iterations = params.train_iterations;
-      sp.seed = params.seed + 1 + j;
-      const std::vector<float> c = kmeans(sub.data(), pq_n, dsub, sp, pool);
-      std::copy(c.begin(), c.end(), cb.begin() + static_cast<std::ptrdiff_t>(j * kSubCentroids * dsub));
-    }
+    KMeansParams sp;
+    sp.k = kSubCentroids;
+    sp.iterations = params.train_iterations;
+    sp.seed = params.seed + 1;  // sub-space j: seed + 1 + j
+    std::vector<float> cb = internal::kmeans_subspaces(residuals.data(), pq_n, d, m, sp);
     std::unique_lock lock(mu);
     QUIVER_CHECK(!trained, "index is already trained");
     commit(std::move(cent), std::move(cb));
