@@ -201,6 +201,84 @@ __device__ inline void exact_group8_n(const float* __restrict__ a, const float* 
   }
 }
 
+/// exact_group8_n for 16-byte aligned a and b[c]: lane l of the group loads elements 4 l .. 4 l + 3 of each
+/// 32-element block (whole 128-byte lines per group and load, a quarter of the loads) and so holds
+/// accumulators 4 (l & 1) .. + 3 of 8-lane accumulator u = l >> 1. Lane 0 returns the sums.
+template <bool L2, int NC>
+__device__ inline void exact_group8_lines(const float* __restrict__ a, const float* const (&b)[NC], uint32_t dim,
+                                          float (&out)[NC]) {
+  const uint32_t l = threadIdx.x & 7u;
+  auto term = [](float x, float y, float s) {
+    if constexpr (L2) {
+      const float d = x - y;
+      return fmaf(d, d, s);
+    } else {
+      return fmaf(x, y, s);
+    }
+  };
+  auto swap = [](float v, int stride) { return __uint_as_float(lane_xor_u32(__float_as_uint(v), stride)); };
+  float s[NC][4];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s[c][t] = 0.0f;
+  const uint32_t n8 = dim / 8 * 8;  // where the 32- and 8-element loops of exact_l2sqr stop
+  uint32_t i = 0;
+#pragma unroll 2
+  for (; i + 32 <= dim; i += 32) {
+    const float4 x = *reinterpret_cast<const float4*>(a + i + 4 * l);
+    float4 y[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) y[c] = *reinterpret_cast<const float4*>(b[c] + i + 4 * l);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      s[c][0] = term(x.x, y[c].x, s[c][0]);
+      s[c][1] = term(x.y, y[c].y, s[c][1]);
+      s[c][2] = term(x.z, y[c].z, s[c][2]);
+      s[c][3] = term(x.w, y[c].w, s[c][3]);
+    }
+  }
+  if (l < 2) {  // blocks of 8 go to accumulator 0
+    for (; i < n8; i += 8) {
+      const float4 x = *reinterpret_cast<const float4*>(a + i + 4 * l);
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const float4 y = *reinterpret_cast<const float4*>(b[c] + i + 4 * l);
+        s[c][0] = term(x.x, y.x, s[c][0]);
+        s[c][1] = term(x.y, y.y, s[c][1]);
+        s[c][2] = term(x.z, y.z, s[c][2]);
+        s[c][3] = term(x.w, y.w, s[c][3]);
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    float lo[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float v = s[c][t];
+      v = v + swap(v, 2);      // s0 + s1, s2 + s3
+      v = v + swap(v, 4);      // v[4 (l & 1) + t]
+      lo[t] = v + swap(v, 1);  // v[t] + v[t + 4]
+    }
+    float sum = (lo[0] + lo[1]) + (lo[2] + lo[3]);
+    if (l == 0) {
+      uint32_t k = n8;
+      const uint32_t v4 = k + (dim - k) / 4 * 4;
+      for (; k < v4; ++k) {
+        if constexpr (L2) {
+          const float d = a[k] - b[c][k];
+          sum = sum + d * d;
+        } else {
+          sum = sum + a[k] * b[c][k];
+        }
+      }
+      for (; k < dim; ++k) sum = term(a[k], b[c][k], sum);
+    }
+    out[c] = sum;
+  }
+}
+
 /// simd::normalize (src/simd/dispatch.cc:119-135) of one row in place.
 __device__ inline void exact_normalize(float* v, uint32_t dim) {
   const float norm_sq = exact_dot(v, v, dim);

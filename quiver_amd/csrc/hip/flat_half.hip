@@ -864,9 +864,8 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
 
 // ---- merge: the best groups, scored exactly ---------------------------------------------------
 
-constexpr int kListsPerLane = static_cast<int>(kHalfMaxLists) / 64;
-constexpr int kHeld = 4;    // keys held per list before it reloads
-constexpr int kKeys = 128;  // scored rows held per query: the k best (k <= 64) and the next 64
+constexpr int kHeld = 4;     // keys held per list before it reloads
+constexpr int kWavesPerQuery = 4;  // of the small-batch form
 
 /// Keys p .. p + kHeld - 1 of one list (positions at or past KL read the list's start, never used).
 template <int KL>
@@ -892,32 +891,18 @@ __device__ __forceinline__ void load_held(const float* ld, const uint32_t* lg, u
   }
 }
 
-/// One wave per query. First the `sel` best groups over the query's lists (ascending by minimum,
-/// then group), popped from list heads held in registers. Then their rows in the reference's order,
-/// four groups at a time (eight lanes per row), keeping the k best (distance, row). After each step
-/// the next group's minimum decides: every row not yet scored has a scan distance of at least that,
-/// so an exact one of at least that minus delta, and once this is above the k-th best distance the
-/// answer is final. At the end of the selection the answer stands if the lists held no more groups
-/// or if delta is 0 (the scan's distances are exact: the sel >= k selected minima are rows that
-/// precede every row of any other group in (distance, row) order); otherwise the last selected
-/// minimum decides the same way, and a query that fails goes to the exact kernel.
-template <int KL>
-__global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
-  if (m.gate != nullptr && ((*m.gate != 0u) != (m.gate_want != 0u))) return;
-  __shared__ uint64_t s_sel[4][kHalfMaxSel];
-  __shared__ uint64_t s_key[4][kKeys];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t q = blockIdx.x * 4 + wave;
-  if (q >= m.nq) return;  // whole wave; this kernel has no block barriers
-  uint64_t* const sel = s_sel[wave];
-  uint64_t* const keys = s_key[wave];
+/// The m.sel best groups over a query's lists, ascending by (minimum, group), into sel: popped by one
+/// wave from list heads held in registers (LPL lists per lane). Returns their count; *spent: some list
+/// gave all of its entries before the selection ended.
+template <int KL, int LPL>
+__device__ __forceinline__ uint32_t select_groups(const HalfMergeArgs& m, uint32_t q, uint64_t* sel, bool* spent) {
+  const int lane = threadIdx.x & 63;
   const float* pd = m.part_d + static_cast<size_t>(q) * m.nlists * KL;
   const uint32_t* pg = m.part_r + static_cast<size_t>(q) * m.nlists * KL;
-
-  uint64_t kk[kListsPerLane][kHeld];
-  uint32_t ptr[kListsPerLane];
+  uint64_t kk[LPL][kHeld];
+  uint32_t ptr[LPL];
 #pragma unroll
-  for (int u = 0; u < kListsPerLane; ++u) {
+  for (int u = 0; u < LPL; ++u) {
     ptr[u] = 0;
     if (64u * u < m.nlists) {  // wave-uniform
       const uint32_t li = lane + 64 * u;
@@ -934,12 +919,12 @@ __global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
     }
   }
   uint32_t count = 0;
-  bool spent = false;  // one of this lane's lists gave all of its entries before the selection ended
+  bool out = false;
   for (uint32_t x = 0; x < m.sel; ++x) {
     uint64_t mine = kk[0][0];
     int arg = 0;
 #pragma unroll
-    for (int u = 1; u < kListsPerLane; ++u) {
+    for (int u = 1; u < LPL; ++u) {
       if (kk[u][0] < mine) {
         mine = kk[u][0];
         arg = u;
@@ -951,13 +936,13 @@ __global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
     ++count;
     if (mine == best) {
 #pragma unroll
-      for (int u = 0; u < kListsPerLane; ++u) {
+      for (int u = 0; u < LPL; ++u) {
         if (u == arg) {
 #pragma unroll
           for (int i = 0; i + 1 < kHeld; ++i) kk[u][i] = kk[u][i + 1];
           kk[u][kHeld - 1] = ~0ull;
           const uint32_t p = ++ptr[u];
-          if (p == KL) spent = spent || x + 1 < m.sel;
+          if (p == KL) out = out || x + 1 < m.sel;
           if (p % kHeld == 0 && p < KL) {
             float d[kHeld];
             uint32_t g[kHeld];
@@ -970,91 +955,170 @@ __global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
       }
     }
   }
-  const double delta = static_cast<double>(m.delta[q]);
-  // A list that ran out (wide merge) may have held more of the answer; a non-finite bound certifies
-  // nothing.
-  if ((m.wide && __ballot(spent) != 0) || !(delta < static_cast<double>(__builtin_huge_valf()))) {
-    if (lane == 0) m.fallback[atomicAdd(m.nfallback, 1u)] = q;
-    return;
-  }
-  __builtin_amdgcn_wave_barrier();
+  *spent = __ballot(out) != 0;
+  return count;
+}
 
-  const float* qp = m.Q + static_cast<size_t>(q) * m.dp;
+/// One wave scores the 64 rows of groups sel[c0 .. c0 + 3] (below count) in the reference's order, eight
+/// lanes per row, and returns their (distance, row) keys sorted, one per lane (absent rows last).
+__device__ __forceinline__ uint64_t score_groups(const HalfMergeArgs& m, const float* qp, const uint64_t* sel,
+                                                 uint32_t c0, uint32_t count, uint64_t* keys) {
+  const int lane = threadIdx.x & 63;
   const uint32_t oct = static_cast<uint32_t>(lane) >> 3;
-  const uint32_t k = m.k;
-  uint32_t held = 0;        // keys[0, held); the first min(held, k) sorted after each step
-  uint64_t bound = ~0ull;   // the k-th best key so far
-  uint64_t x2[2] = {~0ull, ~0ull};
-  bool done = false;
-  for (uint32_t c0 = 0; c0 < count && !done; c0 += 4) {
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-      const float* b[4];
-      uint32_t row[4];
-      bool ok[4];
+  for (int pass = 0; pass < 2; ++pass) {
+    const float* b[4];
+    uint32_t row[4];
+    bool ok[4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint32_t e = static_cast<uint32_t>(pass) * 32 + static_cast<uint32_t>(c) * 8 + oct;  // row of the step
-        const uint32_t gi = c0 + e / 16;
-        ok[c] = gi < count;
-        const uint64_t pos =
-            static_cast<uint64_t>(static_cast<uint32_t>(sel[ok[c] ? gi : 0])) * kHalfGroupRows + e % 16;
-        ok[c] = ok[c] && pos < m.n;
-        row[c] = ok[c] ? (m.idx ? m.idx[pos] : static_cast<uint32_t>(pos)) : 0u;
-        if (m.bitmap) ok[c] = ok[c] && ((m.bitmap[row[c] >> 6] >> (row[c] & 63)) & 1u);
-        b[c] = ok[c] ? m.X + static_cast<size_t>(row[c]) * m.dp : qp;
-      }
-      float e4[4];
-      if (m.l2) {
-        exact_group8_n<true, 4>(qp, b, m.dim, e4);
-      } else {
-        exact_group8_n<false, 4>(qp, b, m.dim, e4);
-      }
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t e = static_cast<uint32_t>(pass) * 32 + static_cast<uint32_t>(c) * 8 + oct;  // row of the 64
+      const uint32_t gi = c0 + e / 16;
+      ok[c] = gi < count;
+      const uint64_t pos = static_cast<uint64_t>(static_cast<uint32_t>(sel[ok[c] ? gi : 0])) * kHalfGroupRows + e % 16;
+      ok[c] = ok[c] && pos < m.n;
+      row[c] = ok[c] ? (m.idx ? m.idx[pos] : static_cast<uint32_t>(pos)) : 0u;
+      if (m.bitmap) ok[c] = ok[c] && ((m.bitmap[row[c] >> 6] >> (row[c] & 63)) & 1u);
+      b[c] = ok[c] ? m.X + static_cast<size_t>(row[c]) * m.dp : qp;
+    }
+    float e4[4];
+    if (m.l2) {
+      exact_group8_lines<true, 4>(qp, b, m.dim, e4);
+    } else {
+      exact_group8_lines<false, 4>(qp, b, m.dim, e4);
+    }
+    if ((lane & 7) == 0) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         float d = m.l2 ? e4[c] : 1.0f - e4[c];
         d = d == d ? d : __builtin_huge_valf();
-        const uint64_t key = make_key(d, row[c]);
-        const bool take = ok[c] && (lane & 7) == 0 && key < bound;
-        const uint64_t mk = __ballot(take);
-        if (take) keys[held + lane_rank(mk)] = key;  // at most 64 past the k <= 64 kept
-        held += static_cast<uint32_t>(__popcll(mk));
-      }
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t e = static_cast<uint32_t>(i * 64 + lane);
-      x2[i] = e < held ? keys[e] : ~0ull;
-    }
-    wave_sort<2>(x2);
-    held = held < k ? held : k;
-    __builtin_amdgcn_wave_barrier();
-    if (static_cast<uint32_t>(lane) < held) keys[lane] = x2[0];
-    __builtin_amdgcn_wave_barrier();
-    if (held == k) {
-      bound = __shfl(x2[0], static_cast<int>(k) - 1, 64);
-      if (c0 + 4 < count) {
-        const double g_next = static_cast<double>(ordered_to_float(static_cast<uint32_t>(sel[c0 + 4] >> 32)));
-        done = g_next - delta > static_cast<double>(ordered_to_float(static_cast<uint32_t>(bound >> 32)));
+        keys[pass * 32 + c * 8 + static_cast<int>(oct)] = ok[c] ? make_key(d, row[c]) : ~0ull;
       }
     }
   }
+  __builtin_amdgcn_wave_barrier();
+  uint64_t key[1] = {keys[lane]};
+  wave_sort<1>(key);
+  __builtin_amdgcn_wave_barrier();
+  return key[0];
+}
+
+/// The 64 smallest of two sorted lists of 64 keys, one per lane: `best` and, reversed, `other`.
+__device__ __forceinline__ uint64_t merge64(uint64_t best, uint64_t other_reversed) {
+  uint64_t v[1] = {best < other_reversed ? best : other_reversed};
+  wave_merge<1>(v);
+  return v[0];
+}
+
+/// First the `sel` best groups over the query's lists. Then their rows in the reference's order, keeping
+/// the best (distance, row), 64 rows per wave and step. After each step the next group's minimum
+/// decides: every row not yet scored has a scan distance of at least that, so an exact one of at least
+/// that minus delta, and once this is above the k-th best distance the answer is final. At the end
+/// of the selection the answer stands if the lists held no more groups or if delta is 0 (the scan's
+/// distances are exact: the sel >= k selected minima are rows that precede every row of any other
+/// group in (distance, row) order); otherwise the last selected minimum decides the same way, and a
+/// query that fails goes to the exact kernel.
+///
+/// W = 1: one wave per query, four queries per work-group. In a large batch the reads of the scored
+/// rows bound it (10,000 queries of 12 groups x 16 rows x 512 bytes), and it stops after the fewest.
+/// W = 4: four waves per query score 16 groups per step, for batches too small to fill the chip, where
+/// the chain of dependent reads counts. LPL = 1 where a query has at most 64 lists: the eight lists
+/// per lane of the other form cost registers that hold a third of the waves.
+template <int KL, int LPL, int W>
+__global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
+  if (m.gate != nullptr && ((*m.gate != 0u) != (m.gate_want != 0u))) return;
+  __shared__ uint64_t s_sel[4][kHalfMaxSel];
+  __shared__ uint64_t s_key[4][64];
+  __shared__ uint32_t s_state[2];  // W = 4: count (or ~0 when the query falls back), done
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t q = W == 4 ? blockIdx.x : blockIdx.x * 4 + wave;
+  if (q >= m.nq) return;  // W = 1: whole waves, no block barriers; W = 4: never
+  uint64_t* const sel = s_sel[W == 4 ? 0 : wave];
+  const double delta = static_cast<double>(m.delta[q]);
+  const bool lead = W == 1 || wave == 0;
+  uint32_t count = 0;
+  bool failed = false;
+  if (lead) {
+    bool spent = false;
+    count = select_groups<KL, LPL>(m, q, sel, &spent);
+    // A list that ran out (wide merge) may have held more of the answer; a non-finite bound certifies
+    // nothing.
+    failed = (m.wide && spent) || !(delta < static_cast<double>(__builtin_huge_valf()));
+  }
+  if constexpr (W == 4) {
+    if (threadIdx.x == 0) s_state[0] = failed ? ~0u : count;
+    __syncthreads();
+    count = s_state[0];
+    failed = count == ~0u;
+  } else {
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (failed) {
+    if (lead && lane == 0) m.fallback[atomicAdd(m.nfallback, 1u)] = q;
+    return;
+  }
+
+  const float* qp = m.Q + static_cast<size_t>(q) * m.dp;
+  const uint32_t k = m.k;  // at most 64
+  uint64_t best = ~0ull;   // the 64 best keys so far, ascending over the lanes (the leading wave's)
+  uint64_t kth = ~0ull;
+  bool done = false;
+  for (uint32_t c0 = 0; c0 < count && !done; c0 += 4 * W) {
+    const uint64_t mine = score_groups(m, qp, sel, c0 + (W == 4 ? 4u * static_cast<uint32_t>(wave) : 0u), count, s_key[wave]);
+    s_key[wave][lane] = mine;
+    if constexpr (W == 4) {
+      __syncthreads();
+      if (wave == 0) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) best = merge64(best, s_key[w][63 - lane]);
+      }
+    } else {
+      __builtin_amdgcn_wave_barrier();
+      best = merge64(best, s_key[wave][63 - lane]);
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (lead) {
+      kth = __shfl(best, static_cast<int>(k) - 1, 64);
+      if (kth != ~0ull && c0 + 4 * W < count) {
+        const double g_next = static_cast<double>(ordered_to_float(static_cast<uint32_t>(sel[c0 + 4 * W] >> 32)));
+        done = g_next - delta > static_cast<double>(ordered_to_float(static_cast<uint32_t>(kth >> 32)));
+      }
+    }
+    if constexpr (W == 4) {
+      if (threadIdx.x == 0) s_state[1] = done ? 1u : 0u;
+      __syncthreads();
+      done = s_state[1] != 0u;
+    }
+  }
+  if (!lead) return;
   if (!done && count >= m.sel && delta != 0.0) {
     const double g_last = static_cast<double>(ordered_to_float(static_cast<uint32_t>(sel[count - 1] >> 32)));
     const bool certified =
-        held == k && static_cast<double>(ordered_to_float(static_cast<uint32_t>(bound >> 32))) < g_last - delta;
+        kth != ~0ull && static_cast<double>(ordered_to_float(static_cast<uint32_t>(kth >> 32))) < g_last - delta;
     if (!certified) {
       if (lane == 0) m.fallback[atomicAdd(m.nfallback, 1u)] = q;
       return;
     }
   }
   if (static_cast<uint32_t>(lane) < k) {
-    const bool full = static_cast<uint32_t>(lane) < held;
-    m.out_rows[static_cast<size_t>(q) * k + lane] = full ? static_cast<uint32_t>(x2[0]) : QVH_EMPTY_ROW;
+    const bool full = best != ~0ull;
+    m.out_rows[static_cast<size_t>(q) * k + lane] = full ? static_cast<uint32_t>(best) : QVH_EMPTY_ROW;
     m.out_dist[static_cast<size_t>(q) * k + lane] =
-        full ? ordered_to_float(static_cast<uint32_t>(x2[0] >> 32)) : __builtin_huge_valf();
+        full ? ordered_to_float(static_cast<uint32_t>(best >> 32)) : __builtin_huge_valf();
   }
+}
+
+/// Batches up to which four waves take each query (100 queries over 128 dims: 33 -> 15 us; 1,003 over 96
+/// dims, k = 30: 85 us with one wave, 101 with four; 2,000 over 768 dims: 194 and 226).
+constexpr uint32_t kMergeWideQueries = 512;
+
+template <int KL>
+void launch_merge_kl(const HalfMergeArgs& m, hipStream_t s) {
+  const bool four = m.nq <= kMergeWideQueries;
+  const dim3 grid(static_cast<unsigned>(four ? m.nq : ceil_div(m.nq, 4)));
+  auto kernel = m.nlists <= 64 ? (four ? flat_half_merge_kernel<KL, 1, 4> : flat_half_merge_kernel<KL, 1, 1>)
+                               : (four ? flat_half_merge_kernel<KL, 8, 4> : flat_half_merge_kernel<KL, 8, 1>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, m);
 }
 
 template <int NK>
@@ -1113,13 +1177,13 @@ void launch_half_wide_scan(int kl, dim3 grid, const HalfScanArgs& a, hipStream_t
 }
 
 void launch_half_merge(int kl, const HalfMergeArgs& m, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(ceil_div(m.nq, 4)));
+  static_assert(kHalfMaxLists <= 8 * 64, "eight lists per lane");
   if (kl == 10) {
-    hipLaunchKernelGGL(flat_half_merge_kernel<10>, grid, dim3(256), 0, s, m);
+    launch_merge_kl<10>(m, s);
   } else if (kl == 16) {
-    hipLaunchKernelGGL(flat_half_merge_kernel<16>, grid, dim3(256), 0, s, m);
+    launch_merge_kl<16>(m, s);
   } else {
-    hipLaunchKernelGGL(flat_half_merge_kernel<32>, grid, dim3(256), 0, s, m);
+    launch_merge_kl<32>(m, s);
   }
 }
 
