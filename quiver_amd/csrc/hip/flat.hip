@@ -3,7 +3,8 @@
 // Pipeline for one call:
 //   1. prep:  queries -> device, unit-normalized for cosine (exact simd::normalize order),
 //             zero-padded to DP floats, ||q||^2.
-//   2. scan:  fp32 MFMA GEMM (v_mfma_f32_32x32x2_f32) of a 32-query column block held in VGPRs
+//   2. scan:  k up to 43 on the 16-bit matrix unit (flat_half.hip); else, and without workspace for
+//             wide rows, an fp32 MFMA GEMM (v_mfma_f32_32x32x2_f32) of a 32-query column block held in VGPRs
 //             against 64-row base tiles staged through LDS (double buffered, padded stride),
 //             with the distance epilogue ||q||^2 + ||x||^2 - 2<q,x> (or 1 - <q,x>) and a per-lane
 //             register top-KL list fused in, so the nq x n distance matrix never reaches HBM.
@@ -67,11 +68,6 @@ struct ScanArgs {
   int share;                // 0: every lane list keeps its own KL best (k > KL: no shared bound)
   uint32_t dp;              // row width (the chunked scan; the register scan has it as DP)
   int rowsplit;             // register scan, unfiltered, at most 128 queries: two waves per query group
-  int bound_slots;          // register scan: publish and read the per-query bound slots
-  // Register scan with 32-entry lists for k above 21 (the wide merge takes R = k + max(16, k / 2)
-  // keys): when nonzero, c = ceil(R / 2) <= 32, and the shared bound is the larger of the lane
-  // pair's c-th entries (2c >= R rows of the pair lie at or below it, so it bounds the R-th best).
-  uint32_t share_rank;
   // Launch gate: when set, the launch does nothing unless (*gate != 0) == (gate_want != 0), read
   // once at the start. Two list lengths are launched back to back and the device picks one.
   const uint32_t* gate;
@@ -83,27 +79,9 @@ __device__ __forceinline__ bool gate_closed(const uint32_t* gate, uint32_t want)
 }
 
 constexpr int kShareEvery = 8;  // chunked scan: tiles between exchanges of the shared per-query bound
-// The MFMA scan's words per query in ScanArgs::qthr: word 0 the union bound, words kScanSlotBase
-// and up the bound slots (one per list source, at most 32), on the query's second 128-byte line.
+// The MFMA scans' words per query in ScanArgs::qthr (word 0 is the shared bound).
 constexpr uint32_t kScanBoundStride = 64;
-constexpr uint32_t kScanSlotBase = 32;
-constexpr int kScanSlots = 32;
-// Splits per query up to which the row-split form of the register scan (four lists per split and
-// query) uses the bound slots: with more, the atomics of its many lists on the query's slot line
-// queue up (1M x 128, 128 queries on 256 splits: 0.39 ms without the slots, 0.49 ms with them). The
-// register scan's full-block form (two lists per split and query) uses them at any split count
-// (10,000 queries on 32 splits: 21.50 ms without, 21.23 ms with; 512 queries on 256 splits 1.33 ->
-// 1.23 ms, 1,024 on 256 2.46 -> 2.30 ms, 2,048 on 128 4.71 -> 4.26 ms).
-constexpr uint64_t kScanSlotMaxSplits = 64;
-
-/// Tiles after which the register scan exchanges bounds: 0, 1, 3, 7, 15, 31 and 63 (the lists' first
-/// rows move a bound the most, and a split of a few tiles would otherwise never take the shared
-/// one), then every 64. An exchange stalls the wave for a device-scope round trip, and late in a
-/// split the bounds move little (1M x 128, 10,000 queries: every 8 tiles 21.07 ms, every 16 20.58,
-/// every 32 20.30, this schedule 20.22, every 128 after 127 20.21).
-__device__ __forceinline__ bool scan_share_after(uint32_t t) {
-  return t < 64 ? (t & (t + 1)) == 0 : t % 64 == 63;
-}
+static_assert(kScanBoundStride == kHalfWordStride, "one layout for the fp32 and the 16-bit scans");
 constexpr int kQueueCap = 20;   // queued candidates per lane before a wave-wide flush
 
 /// Inserts (d, r) into the ascending list (Ld, Lr) in (distance, row) order, dropping the last.
@@ -139,50 +117,6 @@ __device__ __forceinline__ void list_insert_ordered(float (&Ld)[KL], uint32_t (&
   }
   Ld[0] = lt[0] ? d : Ld[0];
   Lr[0] = lt[0] ? r : Lr[0];
-}
-
-/// Sorts 16 values ascending in registers (a bitonic network of 80 compare-exchanges).
-__device__ __forceinline__ void sort16_u32(uint32_t (&v)[16]) {
-#pragma unroll
-  for (int size = 2; size <= 16; size <<= 1) {
-#pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int l = i ^ stride;
-        if (l > i) {
-          const uint32_t lo = min(v[i], v[l]), hi = max(v[i], v[l]);
-          const bool up = (i & size) == 0;
-          v[i] = up ? lo : hi;
-          v[l] = up ? hi : lo;
-        }
-      }
-    }
-  }
-}
-
-/// The K-th smallest of the 32 values held 16 by this lane and 16 by its partner (lane ^ 32),
-/// the same in both lanes. K = 32 is the maximum; below it both halves are sorted and the K-th
-/// smallest of the union is min over i of max(S[i - 1], P[K - 1 - i]) (i values from this lane's
-/// sorted S, the rest from the partner's P).
-template <int K>
-__device__ __forceinline__ uint32_t pair_kth_smallest(uint32_t (&v)[16]) {
-  static_assert(K >= 1 && (K <= 16 || K == 32), "K-th of 32");
-  if constexpr (K == 32) {
-    uint32_t m = v[0];
-#pragma unroll
-    for (int i = 1; i < 16; ++i) m = max(m, v[i]);
-    return max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), 32, 64)));
-  } else {
-    sort16_u32(v);
-    uint32_t p[K];
-#pragma unroll
-    for (int i = 0; i < K; ++i) p[i] = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v[i]), 32, 64));
-    uint32_t r = min(v[K - 1], p[K - 1]);
-#pragma unroll
-    for (int i = 1; i < K; ++i) r = min(r, max(v[i - 1], p[K - 1 - i]));
-    return r;
-  }
 }
 
 /// Appends a lane's passing candidates of one 32x32 distance block to its queue (entry e at
@@ -344,10 +278,12 @@ __device__ __forceinline__ void scan_block_coords(const ScanArgs& a, uint32_t& q
 // RS (row split, small batches): the block serves 128 queries, and the two waves of a 32-query group
 // take the two 32-row halves of every tile, so a batch of 32 queries keeps two SIMDs of a CU busy
 // rather than one; at the end the odd wave's lists go through LDS into the even wave's.
-template <int DP, int KL, bool L2, int MODE, bool RS = false>
+// The lists have no common bound: each holds the 32 best of its own rows, of which the wide merge takes
+// more than 64 (k from 44 up; smaller k runs on the 16-bit matrix unit, flat_half.hip).
+template <int DP, bool L2, int MODE, bool RS = false>
 __global__ void __launch_bounds__(kThreads) flat_scan_kernel(ScanArgs a) {
+  constexpr int KL = 32;
   static_assert(!RS || 4 * 64 * KL <= kQueueCap * kThreads, "row-split hand-off must fit the queue arrays");
-  if (gate_closed(a.gate, a.gate_want)) return;  // the same for every thread of the grid
   constexpr bool FILTER = MODE == 1;
   constexpr int H = DP / 2;                   // dims per lane half (K split in two halves)
   // LDS row stride in floats: conflict-free b128 reads. Columns DP and DP + 1 of a row hold the
@@ -415,64 +351,6 @@ __global__ void __launch_bounds__(kThreads) flat_scan_kernel(ScanArgs a) {
     Ld[x] = __builtin_huge_valf();
     Lr[x] = QVH_EMPTY_ROW;
   }
-
-  // Prune threshold: the smaller of this lane's KL-th best and the shared per-query value. Any
-  // list's KL-th best bounds the KL-th best of the union of all lists, so candidates above it can
-  // never be among the query's KL best (equal distances pass: ties are decided by row).
-  uint32_t* const qw = a.qthr + static_cast<size_t>(qvalid ? q : 0u) * kScanBoundStride;
-  float pthr = qvalid ? ordered_to_float(qw[0]) : __builtin_huge_valf();
-  // Bound slots: every list of the query (one per split, row half rb and lane half h) publishes
-  // its best distance, atomic min, to slot src of kScanSlots. A slot holds one row's distance at
-  // any time, and different slots come from different lists, which hold different rows, so the
-  // KL-th smallest slot value is at or above the query's KL-th best distance (KL distinct rows lie
-  // at or below it); unwritten slots hold +inf. Slots read stale are larger, still bounds. With
-  // many splits running at once this bound falls long before any one list holds KL good rows.
-  static_assert(KL <= kScanSlots && kScanSlotBase + kScanSlots <= kScanBoundStride, "a query's slots fit its words");
-  const uint32_t src =
-      (split * (RS ? 4u : 2u) + static_cast<uint32_t>(rb) * 2u + static_cast<uint32_t>(h)) % kScanSlots;
-  float published = __builtin_huge_valf();
-  auto share_threshold = [&]() {
-    // The two lanes of a query hold disjoint rows: their union has KL candidates at or below
-    // max(own[KL/2-1], other[KL/2-1]) as well as below either list's KL-th.
-    const float own_k = Ld[KL - 1], own_h = Ld[KL / 2 - 1];
-    const float oth_k = __shfl_xor(own_k, 32, 64), oth_h = __shfl_xor(own_h, 32, 64);
-    float t = fminf(fminf(own_k, oth_k), fmaxf(own_h, oth_h));
-    if (a.share_rank != 0) {
-      // k above KL (the wide merge): the pair's union has 2c >= R rows at or below the larger of
-      // the two lanes' c-th entries.
-      float own_c = Ld[0];
-#pragma unroll
-      for (int x = 1; x < KL; ++x) own_c = static_cast<uint32_t>(x) + 1 == a.share_rank ? Ld[x] : own_c;
-      t = fmaxf(own_c, __shfl_xor(own_c, 32, 64));
-    }
-    if (qvalid) {
-      uint32_t g = 0;
-      if (h == 0) g = atomicMin(qw, float_to_ordered(t));
-      uint32_t m = 0xFF800000u;  // +inf
-      if (a.bound_slots) {
-        if (Ld[0] < published) {
-          published = Ld[0];
-          __hip_atomic_fetch_min(qw + kScanSlotBase + src, float_to_ordered(published), __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-        }
-        // Each lane half reads half of the slots (ordered bits compare as the distances do) and
-        // sorts them; the pair then takes the KL-th smallest of all kScanSlots.
-        constexpr int kHalf = kScanSlots / 2;
-        uint32_t sv[kHalf];
-        uint64_t* sw = reinterpret_cast<uint64_t*>(qw + kScanSlotBase + h * kHalf);
-#pragma unroll
-        for (int i = 0; i < kHalf / 2; ++i) {
-          const uint64_t w = __hip_atomic_load(sw + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          sv[2 * i] = static_cast<uint32_t>(w);
-          sv[2 * i + 1] = static_cast<uint32_t>(w >> 32);
-        }
-        m = pair_kth_smallest<KL>(sv);
-      }
-      g = __shfl(g, j, 64);
-      t = fminf(t, fminf(ordered_to_float(g), ordered_to_float(m)));
-    }
-    pthr = fminf(pthr, t);
-  };
 
   // Candidate queue of this lane: appended in row order, inserted into the list by a wave-wide
   // flush (all lanes at once) when any queue could overflow on the next block.
@@ -571,7 +449,7 @@ __global__ void __launch_bounds__(kThreads) flat_scan_kernel(ScanArgs a) {
       if (left < 64) admit &= (1ull << left) - 1;
       const bool masked = FILTER || left < 64;
       const uint32_t lane_bits = static_cast<uint32_t>(admit >> (32 * rb)) >> (4 * h);
-      const float thr = fminf(pthr, Ld[KL - 1]);
+      const float thr = Ld[KL - 1];
       bool any = false;
       if (!masked) {
         float m = acc[0];
@@ -644,7 +522,7 @@ __global__ void __launch_bounds__(kThreads) flat_scan_kernel(ScanArgs a) {
         const uint32_t lane_bits = static_cast<uint32_t>(admit >> (32 * blk)) >> (4 * h);
         // Pass test: !(d > thr). Ties pass (a tied row may still win on row number), and so
         // does NaN, which the flush turns into +inf as the reference does.
-        const float thr = fminf(pthr, Ld[KL - 1]);
+        const float thr = Ld[KL - 1];
         float d[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r) d[r] = acc[r];
@@ -676,10 +554,8 @@ __global__ void __launch_bounds__(kThreads) flat_scan_kernel(ScanArgs a) {
         }
       }
     }
-    if (wave_active && scan_share_after(t)) {
-      flush_queue();
-      if (a.share) share_threshold();
-    }
+    // Early flushes tighten the lists' own bounds.
+    if (wave_active && (t < 64 ? (t & (t + 1)) == 0 : t % 64 == 63)) flush_queue();
     if (t + 1 < ntiles) store_tile(buf ^ 1);
     __syncthreads();
   }
@@ -2556,27 +2432,27 @@ uint32_t wide_selection(uint32_t k) { return k + std::max<uint32_t>(16, k / 2); 
 /// entries: 21.79 ms).
 int exact_list_length(uint32_t k) { return k <= 10 ? 10 : 0; }
 
-template <int DP, int KL>
-void launch_scan_kl(bool l2, int mode, dim3 grid, const ScanArgs& a, hipStream_t s) {
+template <int DP>
+void launch_scan_dp(bool l2, int mode, dim3 grid, const ScanArgs& a, hipStream_t s) {
   if (a.rowsplit) {  // unfiltered batches of at most 128 queries
     if (l2) {
-      hipLaunchKernelGGL((flat_scan_kernel<DP, KL, true, 0, true>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((flat_scan_kernel<DP, true, 0, true>), grid, dim3(kThreads), 0, s, a);
     } else {
-      hipLaunchKernelGGL((flat_scan_kernel<DP, KL, false, 0, true>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((flat_scan_kernel<DP, false, 0, true>), grid, dim3(kThreads), 0, s, a);
     }
     return;
   }
   if (l2) {
     if (mode == 1) {
-      hipLaunchKernelGGL((flat_scan_kernel<DP, KL, true, 1>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((flat_scan_kernel<DP, true, 1>), grid, dim3(kThreads), 0, s, a);
     } else {
-      hipLaunchKernelGGL((flat_scan_kernel<DP, KL, true, 0>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((flat_scan_kernel<DP, true, 0>), grid, dim3(kThreads), 0, s, a);
     }
   } else {
     if (mode == 1) {
-      hipLaunchKernelGGL((flat_scan_kernel<DP, KL, false, 1>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((flat_scan_kernel<DP, false, 1>), grid, dim3(kThreads), 0, s, a);
     } else {
-      hipLaunchKernelGGL((flat_scan_kernel<DP, KL, false, 0>), grid, dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((flat_scan_kernel<DP, false, 0>), grid, dim3(kThreads), 0, s, a);
     }
   }
 }
@@ -2613,21 +2489,21 @@ void launch_scan(uint32_t dp, int kl, dim3 grid, const ScanArgs& a, hipStream_t 
     return;
   }
   switch (dp) {
-    case 16: launch_scan_kl<16, 32>(l2, filter, grid, a, s); break;
-    case 24: launch_scan_kl<24, 32>(l2, filter, grid, a, s); break;
-    case 32: launch_scan_kl<32, 32>(l2, filter, grid, a, s); break;
-    case 40: launch_scan_kl<40, 32>(l2, filter, grid, a, s); break;
-    case 48: launch_scan_kl<48, 32>(l2, filter, grid, a, s); break;
-    case 56: launch_scan_kl<56, 32>(l2, filter, grid, a, s); break;
-    case 64: launch_scan_kl<64, 32>(l2, filter, grid, a, s); break;
-    case 72: launch_scan_kl<72, 32>(l2, filter, grid, a, s); break;
-    case 80: launch_scan_kl<80, 32>(l2, filter, grid, a, s); break;
-    case 88: launch_scan_kl<88, 32>(l2, filter, grid, a, s); break;
-    case 96: launch_scan_kl<96, 32>(l2, filter, grid, a, s); break;
-    case 104: launch_scan_kl<104, 32>(l2, filter, grid, a, s); break;
-    case 112: launch_scan_kl<112, 32>(l2, filter, grid, a, s); break;
-    case 120: launch_scan_kl<120, 32>(l2, filter, grid, a, s); break;
-    case 128: launch_scan_kl<128, 32>(l2, filter, grid, a, s); break;
+    case 16: launch_scan_dp<16>(l2, filter, grid, a, s); break;
+    case 24: launch_scan_dp<24>(l2, filter, grid, a, s); break;
+    case 32: launch_scan_dp<32>(l2, filter, grid, a, s); break;
+    case 40: launch_scan_dp<40>(l2, filter, grid, a, s); break;
+    case 48: launch_scan_dp<48>(l2, filter, grid, a, s); break;
+    case 56: launch_scan_dp<56>(l2, filter, grid, a, s); break;
+    case 64: launch_scan_dp<64>(l2, filter, grid, a, s); break;
+    case 72: launch_scan_dp<72>(l2, filter, grid, a, s); break;
+    case 80: launch_scan_dp<80>(l2, filter, grid, a, s); break;
+    case 88: launch_scan_dp<88>(l2, filter, grid, a, s); break;
+    case 96: launch_scan_dp<96>(l2, filter, grid, a, s); break;
+    case 104: launch_scan_dp<104>(l2, filter, grid, a, s); break;
+    case 112: launch_scan_dp<112>(l2, filter, grid, a, s); break;
+    case 120: launch_scan_dp<120>(l2, filter, grid, a, s); break;
+    case 128: launch_scan_dp<128>(l2, filter, grid, a, s); break;
     default: throw Failure(QVH_EUNSUPPORTED, "flat scan: unsupported padded dimension");
   }
 }
@@ -3128,16 +3004,15 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
   a.part_d = b.pd;
   a.part_r = b.pr;
   a.qthr = b.thr;
-  // The wide merge's R keys: up to R = 64 the register scan shares a bound of rank ceil(R / 2) (1M x
-  // 128 integer mixture, 10k queries, k = 32: 28.9 ms with no shared bound).
+  // The wide merge's R keys: up to R = 64 the scan shares a bound of rank ceil(R / 2) (with the fp32
+  // scan, 1M x 128 integer mixture, 10k queries, k = 32: 28.9 ms without, 25.5 ms with it).
   const uint32_t wide_sel = wide_selection(k);
-  a.share_rank = p.wide && wide_sel <= 64 && f->dp <= static_cast<uint32_t>(kMaxDp) ? (wide_sel + 1) / 2 : 0;
-  a.share = !p.wide || a.share_rank != 0 ? 1 : 0;
+  const uint32_t share_rank = p.half && !p.half_wide && p.wide ? (wide_sel + 1) / 2 : 0;
+  a.share = !p.wide || share_rank != 0 ? 1 : 0;
   a.dp = f->dp;
   // One query block of at most 128 queries, unfiltered, register-resident queries: the row-split
   // form of the scan (two waves per 32-query group).
   a.rowsplit = nq <= static_cast<uint64_t>(kQueriesPerBlock / 2) && !d_idx && !d_bitmap && f->dp <= kMaxDp ? 1 : 0;
-  a.bound_slots = !p.wide && (!a.rowsplit || p.nsplit <= kScanSlotMaxSplits) ? 1 : 0;
   const dim3 sgrid(static_cast<unsigned>(p.qblocks * p.nsplit));
   HalfScanArgs ha{};
   if (p.half) {
@@ -3158,7 +3033,7 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
     ha.part_r = a.part_r;
     ha.words = a.qthr;
     ha.share = a.share;
-    ha.share_rank = a.share_rank;
+    ha.share_rank = share_rank;
     ha.bound_slots = p.wide ? 0 : 1;
     ha.meta = f->meta.as<uint32_t>();
     if (p.half_wide) {

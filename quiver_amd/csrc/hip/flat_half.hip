@@ -864,8 +864,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
 
 // ---- merge: the best groups, scored exactly ---------------------------------------------------
 
-constexpr int kHeld = 4;     // keys held per list before it reloads
-constexpr int kWavesPerQuery = 4;  // of the small-batch form
+constexpr int kHeld = 4;  // keys held per list before it reloads
 
 /// Keys p .. p + kHeld - 1 of one list (positions at or past KL read the list's start, never used).
 template <int KL>
