@@ -16,9 +16,10 @@ Prints ONE JSON line. `value` is the flat workload's queries per second (query p
 scan + merge/exact re-score), timed over K steps with the device synchronized on both sides;
 the "ivfpq" object carries the same fields for the IVF-PQ workload, "flat_small_batches" the
 flat search time of 1, 8, 32 and 128 of the same queries, and "flat_wide_rows" a 500,000 x 768
-flat search (the chunked MFMA scan for rows wider than 128). `roofline` is each
+flat search (the scan for rows wider than 128). `roofline` is each
 workload's dominant kernel measured with HIP events on the stream it runs on: the flat scan's
-algorithmic 2*n*d*nq FLOP per launch against the dense FP32 matrix peak (157.3 TFLOP/s), the
+algorithmic 2*n*d*nq FLOP per launch against the dense fp16 matrix peak (2.5 PFLOP/s; operands that
+one fp16 value does not hold take three products, counted once here), the
 IVF-PQ list scan's algorithmic code bytes (sum over queries and probed lists of len * m) against
 HBM peak (8 TB/s). `host_api` is the reference's own way of timing (bench/ann_bench.cc:351-357,
 378): search_batch through the C++ classes with host buffers in and out, best of 3, which adds the
@@ -45,7 +46,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "batched QPS @k=10: flat 1M×128 L2 and IVF-PQ nprobe=32; % of MFMA/HBM peak"
-FP32_MFMA_PEAK_TFLOPS = 157.3
+FP16_MFMA_PEAK_TFLOPS = 2500.0  # dense, fp32 accumulation: the unit the flat scans run on
 HBM_PEAK_GBS = 8000.0
 
 
@@ -213,10 +214,10 @@ def bench_flat(args, hip: Hip, qvh: Qvh):
         "ms_per_step": ms_per_step,
         "stage_ms": {"prep": float(st[:, 0].mean()), "scan": scan_ms, "merge": float(st[:, 2].mean())},
         "nsplit": int(st[0, 3]),
-        "roofline": {"bound": "mfma", "kernel": "flat_scan_kernel<128,10>", "achieved": achieved,
-                     "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": achieved / FP32_MFMA_PEAK_TFLOPS,
-                     "traffic": load_traffic("flat_scan_int_mix_1m_pmc")},
+        "roofline": {"bound": "mfma", "kernel": "flat_half_kernel<8,10,1,2>", "achieved": achieved,
+                     "peak": FP16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": achieved / FP16_MFMA_PEAK_TFLOPS,
+                     "traffic": load_traffic("flat_half_int_mix_1m_pmc")},
         "config": {"workload": "flat exact L2 k=10: 1,000,000 x 128 fp32 integer-valued mixture, "
                                "10,000 queries batched", "n": n, "dim": dim, "nq": nq, "k": k},
     }
@@ -233,7 +234,7 @@ def bench_flat(args, hip: Hip, qvh: Qvh):
     del host_index
     if not args.no_extra:
         # Small batches (the first query: the few-query kernel; 8 and 32: the ring scan; 128: the
-        # row-split MFMA scan): device time of one search from its stage events, and the caller's
+        # row-split form of the scan): device time of one search from its stage events, and the caller's
         # wall time of search + sync.
         small = {}
         for b in (1, 8, 32, 128):
@@ -424,7 +425,7 @@ def bench_flat_filtered(args, qvh: Qvh):
         tflops = 2.0 * admitted * dim * q.shape[0] / (scan_ms * 1e-3) / 1e12
         out[name] = {"qps_host_api": q.shape[0] / float(np.mean(times)), "admitted_rows": int(admitted),
                      "scan_ms": scan_ms, "scan_tflops_admitted": tflops,
-                     "frac_of_fp32_mfma_peak": tflops / FP32_MFMA_PEAK_TFLOPS}
+                     "frac_of_fp16_mfma_peak": tflops / FP16_MFMA_PEAK_TFLOPS}
     return {"config": {"workload": "flat exact cosine k=10: 1,183,514 x 100 unit-norm 256-component mixture, "
                                    "10,000 queries, host-buffer API, allowed-id filters", "n": n, "dim": dim,
                        "nq": int(q.shape[0]), "k": k},
@@ -432,7 +433,7 @@ def bench_flat_filtered(args, qvh: Qvh):
 
 
 def bench_flat_wide(args, hip: Hip, qvh: Qvh):
-    """Rows wider than the register-resident scan (the chunked MFMA scan): 500,000 x 768 N(0,1)
+    """Rows wider than the register-resident scan (wide rows): 500,000 x 768 N(0,1)
     fp32, L2, k=10, 10,000 queries, device-resident, median of 3 after one warm-up."""
     n, dim, nq, k = 500_000, 768, 10_000, 10
     rng = np.random.default_rng(768)
@@ -463,11 +464,11 @@ def bench_flat_wide(args, hip: Hip, qvh: Qvh):
         hip.lib.hipFree(ptr)
     st = np.median(np.array(stages), axis=0)
     tflops = 2.0 * n * dim * nq / (st[1] * 1e-3) / 1e12
-    return {"config": {"workload": "flat exact L2 k=10: 500,000 x 768 N(0,1) fp32, 10,000 queries batched (chunked "
-                                   "MFMA scan)", "n": n, "dim": dim, "nq": nq, "k": k},
+    return {"config": {"workload": "flat exact L2 k=10: 500,000 x 768 N(0,1) fp32, 10,000 queries batched (wide "
+                                   "rows)", "n": n, "dim": dim, "nq": nq, "k": k},
             "qps": nq / float(np.median(walls)),
             "stage_ms": {"prep": float(st[0]), "scan": float(st[1]), "merge": float(st[2])},
-            "scan_tflops": tflops, "frac_of_fp32_mfma_peak": tflops / FP32_MFMA_PEAK_TFLOPS}
+            "scan_tflops": tflops, "frac_of_fp16_mfma_peak": tflops / FP16_MFMA_PEAK_TFLOPS}
 
 
 def bench_ivfpq_cosine_refine(args, hip: Hip, qvh: Qvh):
