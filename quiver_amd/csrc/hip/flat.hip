@@ -1554,6 +1554,9 @@ __global__ void __launch_bounds__(256) row_norms_kernel(const float* __restrict_
 /// product's path, u = 2^-24, P = ||q||, R = the largest stored ||x||):
 ///   L2:            |g - e| <= (2n + 4) u (P + R)^2 (1 + O(nu))
 ///   inner product: |g - e| <= (2n + 2) u (1 + P R) (1 + O(nu))
+/// and, for L2, (n + 32) 2^-149 for roundings among subnormal values (2^-150 each), which the relative
+/// terms do not cover; beside the 1 of the inner product these vanish. R is taken as a bound where
+/// the largest squared norm is near float's underflow (stored_norm). The relative terms come
 /// from the standard bound gamma_n = nu / (1 - nu) on a sum of n rounded terms, applied to the
 /// GEMM form ||q||^2 + ||x||^2 - 2<q,x> and to the reference's sum of squared differences (or to
 /// the two dot products). delta uses the coefficient (4n + 16): a factor of two over the
@@ -1615,13 +1618,16 @@ __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restri
   if (lane != 0) return;
   const float n2 = static_cast<float>(s);
   qn[q] = n2;
+  // Not from the squares as floats, which may have underflowed; a square past float's range leaves the
+  // query without a bound.
+  const double P = n2 < __builtin_huge_valf() ? sqrt(s) : __builtin_huge_val();
+  const double R = stored_norm(meta, dp);
   if (half) {
     // L2: the norm step's weight 2^8 s_q / s_x stays within fp16.
-    const float sx = half_scale(__uint_as_float(meta[0])), sq = half_scale(n2);
-    thr[q * thr_stride + kHalfScaleWord] = __float_as_uint(l2 && sq > 128.0f * sx ? 128.0f * sx : sq);
+    const float sx = half_scale(R), sq = half_scale(P);
+    thr[q * thr_stride + kHalfScaleWord] =
+        __float_as_uint(l2 && sq > 128.0f * sx ? 128.0f * sx : sq);
   }
-  const double P = sqrt(static_cast<double>(n2));
-  const double R = sqrt(static_cast<double>(__uint_as_float(meta[0])));
   const double u = 1.0 / 16777216.0;
   const double coef = (half == 2 ? 3.5 * dp + 64.0 : half == 1 ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;
   double d;
@@ -1629,7 +1635,7 @@ __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restri
       (!half || (largest <= 2048.0f && __uint_as_float(meta[2]) <= 2048.0f))) {
     d = 0.0;
   } else if (l2) {
-    d = coef * (P + R) * (P + R);
+    d = coef * (P + R) * (P + R) + (dp + 32.0) * 0x1p-149;
   } else {
     d = coef * (1.0 + P * R);
   }

@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
   const bool wave_active = q0 < a.nq;
   const uint32_t q = q0 + (QG == 2 ? static_cast<uint32_t>(lane) : static_cast<uint32_t>(j));  // the query this lane lists
   const bool qvalid = q < a.nq;
-  const float sx = half_scale(__uint_as_float(a.meta[0]));
+  const float sx = half_scale(stored_norm(a.meta, a.dp));
 
   // Query operands: column j of group g, dims 16 kk + 8 h .. + 7 of step kk, negated and scaled.
   f16x8 bh[QG][NK], bl[NP == 3 ? QG : 1][NP == 3 ? NK : 1];
@@ -623,7 +623,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
   const bool wave_active = q0 < a.nq;
   const uint32_t q = q0 + static_cast<uint32_t>(lane);  // the query this lane lists
   const bool qvalid = q < a.nq;
-  const float sx = half_scale(__uint_as_float(a.meta[0]));
+  const float sx = half_scale(stored_norm(a.meta, a.dp));
   f16x8 baug[2];
 #pragma unroll
   for (int g = 0; g < 2; ++g) {

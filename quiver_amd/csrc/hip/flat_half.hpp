@@ -24,13 +24,23 @@ constexpr uint32_t kHalfSlotBase = 32;
 constexpr uint32_t kHalfSlots = 32;
 constexpr uint32_t kHalfScaleWord = 1;
 
-/// 2^(11 - e) for a norm whose square is n2, 2^(e - 1) < norm <= 2^e (1 for zero and non-finite ones):
-/// brings the norm to (2^10, 2^11].
-__device__ __forceinline__ float half_scale(float n2) {
-  if (!(n2 > 0.0f) || !(n2 < __builtin_huge_valf())) return 1.0f;
+/// The largest stored norm, from the store's meta words ([0] the largest squared norm, [2] the largest
+/// magnitude, both float bits). Where the square is subnormal in float or has lost its bits to zero
+/// (norms below 2^-50 here), the bound sqrt(dp) times the largest magnitude instead.
+__device__ __forceinline__ double stored_norm(const uint32_t* meta, uint32_t dp) {
+  const float n2 = __uint_as_float(meta[0]);
+  return n2 < 0x1p-100f ? sqrt(static_cast<double>(dp)) * static_cast<double>(__uint_as_float(meta[2]))
+                        : sqrt(static_cast<double>(n2));
+}
+
+/// 2^(11 - e) for a norm in (2^(e - 1), 2^e] (1 for zero and non-finite ones): brings the norm to
+/// (2^10, 2^11]. Within 2^100 either way: smaller norms stay below it, and what they lose in 16 bits
+/// is below 2^-89 times the other operand's norm, itself below 2^64.
+__device__ __forceinline__ float half_scale(double norm) {
+  if (!(norm > 0.0) || !(norm < __builtin_huge_val())) return 1.0f;
   int e = 0;
-  const float m = frexpf(sqrtf(n2), &e);  // m in [0.5, 1)
-  if (m == 0.5f) --e;
+  const double m = frexp(norm, &e);  // m in [0.5, 1)
+  if (m == 0.5) --e;
   e = 11 - e;
   return ldexpf(1.0f, e < -100 ? -100 : e > 100 ? 100 : e);
 }
@@ -57,7 +67,7 @@ struct HalfScanArgs {
   int share;            // 0: every list keeps its own KL best
   uint32_t share_rank;  // nonzero: the shared bound is the larger of the lane pair's entries of this rank
   int bound_slots;
-  const uint32_t* meta;  // store meta: [0] largest squared norm (float bits)
+  const uint32_t* meta;  // the store's meta words (stored_norm)
   const uint32_t* gate;  // the launch runs when (*gate != 0) == (gate_want != 0); null: always
   uint32_t gate_want;
   const void* qfrag;  // wide rows: the split queries (launch_half_query_frags)

@@ -71,6 +71,21 @@ def test_magnitudes(oracle, rows_exp, query_exp, metric):
     _check(oracle, base, q, 10, metric)
 
 
+@pytest.mark.parametrize("rows_exp,query_exp", [(-80, 60), (60, -80), (-80, -70), (-76, -76), (-74, -74), (-74, -148),
+                                                (-84, -70), (-148, -148), (-140, 40)])
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+@pytest.mark.parametrize("dim", [16, 32, 136])
+def test_magnitudes_whose_squares_underflow(oracle, rows_exp, query_exp, metric, dim):
+    """Norms whose squares are subnormal or zero in float, beside normal ones on the other side: the
+    16-bit scans (k = 10, 30), the fp32 scan (k = 50) and, for 8 queries, the ring scan."""
+    rng = np.random.default_rng(11)
+    base = np.ldexp(_normal(rng, 1_500, dim), rows_exp).astype(np.float32)
+    q = np.ldexp(_normal(rng, 40, dim), query_exp).astype(np.float32)
+    for k in (10, 30, 50):
+        _check(oracle, base, q, k, metric)
+    _check(oracle, base, q[:8], 10, metric)
+
+
 @pytest.mark.parametrize("top", [255, 2_048, 2_049, 4_000])
 def test_integer_magnitudes(oracle, top):
     """Integers up to and above 2,048, up to which an fp16 value holds every integer."""
