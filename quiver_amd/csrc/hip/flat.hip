@@ -1623,10 +1623,11 @@ __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restri
   const double P = n2 < __builtin_huge_valf() ? sqrt(s) : __builtin_huge_val();
   const double R = stored_norm(meta, dp);
   if (half) {
-    // L2: the norm step's weight 2^8 s_q / s_x stays within fp16.
+    // L2: the norm step's weight 2^8 s_q / s_x stays within fp16 (a zero query takes its upper end:
+    // at 1 the weight would be 0 for rows of norms below 2^-22, and nothing could be certified).
     const float sx = half_scale(R), sq = half_scale(P);
     thr[q * thr_stride + kHalfScaleWord] =
-        __float_as_uint(l2 && sq > 128.0f * sx ? 128.0f * sx : sq);
+        __float_as_uint(l2 && (P == 0.0 || sq > 128.0f * sx) ? 128.0f * sx : sq);
   }
   const double u = 1.0 / 16777216.0;
   const double coef = (half == 2 ? 3.5 * dp + 64.0 : half == 1 ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;

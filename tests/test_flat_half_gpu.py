@@ -11,6 +11,7 @@ import pytest
 import quiver_amd as quiver
 from oracle.oracle import rows_bitmap
 from parity import assert_same_topk
+from qvh_ctypes import Qvh
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +85,23 @@ def test_magnitudes_whose_squares_underflow(oracle, rows_exp, query_exp, metric,
     for k in (10, 30, 50):
         _check(oracle, base, q, k, metric)
     _check(oracle, base, q[:8], 10, metric)
+
+
+@pytest.mark.parametrize("dim,k", [(16, 10), (40, 30), (136, 10)])
+@pytest.mark.parametrize("rows_exp", [-50, -24, 0, 40])
+def test_zero_queries_are_certified(oracle, dim, k, rows_exp):
+    """A zero query's L2 distances are the rows' squared norms: no query may need the exact kernel."""
+    rng = np.random.default_rng(dim)
+    base = np.ldexp(_normal(rng, 1_500, dim), rows_exp).astype(np.float32)
+    base *= rng.uniform(1.0, 2.0, (1_500, 1)).astype(np.float32)  # squared norms further apart than the bound
+    q = np.zeros((40, dim), np.float32)
+    idx = quiver.FlatIndex(dim, "l2")
+    idx.add(base)
+    print(f"case: {dim} {k} {rows_exp}", flush=True)
+    labels, dist = idx.search(q, k)
+    assert Qvh().last_fallbacks(idx._index._device_handle) == 0
+    rows, exp = oracle.flat_search(base, q, k, "l2")
+    assert np.array_equal(labels, rows.astype(np.int64)) and np.array_equal(dist.view(np.uint32), exp.view(np.uint32))
 
 
 @pytest.mark.parametrize("top", [255, 2_048, 2_049, 4_000])
