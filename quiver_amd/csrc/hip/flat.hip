@@ -3041,7 +3041,6 @@ void flat_search_run(qvh_flat* f, const FlatPlan& p, const FlatBuffers& b, const
     ha.words = a.qthr;
     ha.share = a.share;
     ha.share_rank = share_rank;
-    ha.bound_slots = p.wide ? 0 : 1;
     ha.meta = f->meta.as<uint32_t>();
     if (p.half_wide) {
       launch_half_query_frags(b.q, a.nq, f->dp, b.thr, b.qf, s);

@@ -76,21 +76,6 @@ __device__ __forceinline__ void group_insert_any(float (&Ld)[KL], uint32_t (&Lg)
   Lg[0] = lt[0] ? g : Lg[0];
 }
 
-/// The largest of the query's first K bound slots. Each holds the smallest minimum any of its sources
-/// has found, so K different groups lie at or below it.
-template <int K>
-__device__ __forceinline__ uint32_t slots_bound(const uint32_t* slots) {
-  static_assert(K % 2 == 0 && K <= static_cast<int>(kHalfSlots), "whole 8-byte words");
-  uint32_t m = 0;
-#pragma unroll
-  for (int i = 0; i < K / 2; ++i) {
-    const uint64_t w = __hip_atomic_load(reinterpret_cast<const uint64_t*>(slots) + i, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-    m = max(m, max(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32)));
-  }
-  return m;
-}
-
 /// Minimum of 16 accumulators.
 __device__ __forceinline__ float min16(const f32x16& a) {
   float m = fminf(fminf(a[0], a[1]), a[2]);
@@ -182,7 +167,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
     baug[g] = f16x8{w, w, w, 0, 0, 0, 0, 0};
   }
 
-  // The lane's list, ascending; in LDS form only its first and last minima stay in registers.
+  // The lane's list, ascending; in LDS form only its last minimum stays in registers.
   constexpr int kRegs = kLdsLists ? 1 : KL;
   float Ld[kRegs];
   uint32_t Lg[kRegs];
@@ -196,13 +181,14 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
       Lg[x] = QVH_EMPTY_ROW;
     }
   }
-  float first = __builtin_huge_valf(), kth = __builtin_huge_valf();
+  float kth = __builtin_huge_valf();
 
   // Prune threshold: the smaller of this list's KL-th minimum and the shared per-query value. Any
   // list's KL-th bounds the KL-th of the union of all lists, so groups above it can never be among
-  // the query's KL best (equal minima pass: ties are decided by group). Bound slots: every list
-  // publishes its best minimum to one of the query's first KL slots; different slots hold minima of
-  // different groups, so the largest of them bounds the query's KL-th best minimum from above.
+  // the query's KL best (equal minima pass: ties are decided by group). A tighter shared bound from the
+  // lists' best minima, one word per list, cost more in atomics than it pruned (50,000 x 64, k = 10,
+  // scan and merge: 40 queries 115 us with it, 66 without; 256 queries 203 and 64; 1M x 128, 10,000
+  // queries 3.18 ms a search and 3.05).
   uint32_t* const qw = a.words + static_cast<size_t>(qvalid ? q : 0u) * kHalfWordStride;
   float pthr = __builtin_huge_valf();
   if (qvalid && a.share) {
@@ -210,8 +196,6 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
   }
   constexpr uint32_t kLists = QG == 2 ? 1u : 2u;  // per split and query
   const uint32_t list = split * kLists + (QG == 2 ? 0u : static_cast<uint32_t>(h));
-  const uint32_t src = (list * rw + rslot) % KL;
-  float published = __builtin_huge_valf();
   auto share_threshold = [&]() {
     float t = kth;
     if constexpr (QG == 1) {
@@ -232,14 +216,6 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
     if (qvalid) {
       const uint32_t g = __hip_atomic_fetch_min(qw, float_to_ordered(t), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       t = fminf(t, ordered_to_float(g));
-      if (a.bound_slots) {
-        if (first < published) {
-          published = first;
-          __hip_atomic_fetch_min(qw + kHalfSlotBase + src, float_to_ordered(published), __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
-        }
-        t = fminf(t, ordered_to_float(slots_bound<KL>(qw + kHalfSlotBase)));
-      }
     }
     pthr = fminf(pthr, t);
   };
@@ -258,7 +234,6 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
           if (v < D[KL - 1]) group_insert<KL>(D, G, v, s_qg[e * kThreads + tid]);
         }
       }
-      first = D[0];
       kth = D[KL - 1];
     };
     if constexpr (kLdsLists) {
@@ -488,13 +463,10 @@ __global__ void __launch_bounds__(kThreads) flat_half_kernel(HalfScanArgs a) {
         }
         if (convert_at == 1 && blk == blk0) convert_next();
       }
-      // Bounds are exchanged after tiles 0, 1, 3, 7, ... (the first rows move a bound the most), then
-      // every 32, or every 8 where an exchange is one atomic and no slots. An exchange waits for a
-      // device-scope round trip (1M x 128, 10,000 queries, with slots: every 64 tiles 3.41-3.51 ms a
-      // search, 32 3.43, 16 3.59, 8 3.86; 300,007 x 96, 1,003 queries, k = 30, without: 0.88-0.99, 0.95,
-      // 0.81, 0.72).
-      const uint32_t period = a.bound_slots ? 32u : 8u;
-      if (t < period ? (t & (t + 1)) == 0 : t % period == period - 1) {
+      // Bounds are exchanged after tiles 0, 1, 3, 7 (the first rows move a bound the most), then every 8:
+      // an exchange waits for a device-scope round trip (300,007 x 96, 1,003 queries, k = 30: every 64
+      // tiles 0.88-0.99 ms a search, 32 0.95, 16 0.81, 8 0.72).
+      if (t < 8 ? (t & (t + 1)) == 0 : t % 8 == 7) {
         flush_queue();
         if (a.share) {
           share_threshold();
@@ -634,7 +606,6 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
   }
 
   const uint32_t list = split * 2 + static_cast<uint32_t>(rhalf);
-  const uint32_t src = list % KL;
   uint32_t* const qw = a.words + static_cast<size_t>(qvalid ? q : 0u) * kHalfWordStride;
   float* const my_d = a.part_d + (static_cast<size_t>(qvalid ? q : 0u) * (2 * a.nsplit) + list) * KL;
   uint32_t* const my_g = a.part_r + (static_cast<size_t>(qvalid ? q : 0u) * (2 * a.nsplit) + list) * KL;
@@ -645,7 +616,7 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
       my_g[x] = QVH_EMPTY_ROW;
     }
   }
-  float kth = __builtin_huge_valf(), first = __builtin_huge_valf(), published = __builtin_huge_valf();
+  float kth = __builtin_huge_valf();
   float pthr = __builtin_huge_valf();
 
   const uint64_t r0 = static_cast<uint64_t>(split) * a.rows_per_split;
@@ -827,23 +798,12 @@ __global__ void __launch_bounds__(kThreads) flat_half_wide_kernel(HalfScanArgs a
             my_g[x] = Lg[x];
           }
           kth = Ld[KL - 1];
-          first = Ld[0];
         }
-        // Bounds through the query's words, as the narrow scan does; a tile is long enough to do so
-        // after each. Where the merge takes more than KL groups (share_rank set) only this list's own
-        // bound prunes.
-        if (a.share && a.share_rank == 0 && qvalid) {
+        // The shared bound, as in the narrow scan; a tile is long enough to exchange it after each. Where
+        // the merge takes more than KL groups (share is 0) only this list's own bound prunes.
+        if (a.share && qvalid) {
           const uint32_t g = __hip_atomic_fetch_min(qw, float_to_ordered(kth), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          float b = ordered_to_float(g);
-          if (a.bound_slots) {
-            if (first < published) {
-              published = first;
-              __hip_atomic_fetch_min(qw + kHalfSlotBase + src, float_to_ordered(first), __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-            }
-            b = fminf(b, ordered_to_float(slots_bound<KL>(qw + kHalfSlotBase)));
-          }
-          pthr = fminf(pthr, b);
+          pthr = fminf(pthr, fminf(kth, ordered_to_float(g)));
         }
       }
     }

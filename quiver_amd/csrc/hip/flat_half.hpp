@@ -17,11 +17,9 @@ constexpr uint32_t kHalfWideQueries = 256;     // per work-group
 constexpr uint32_t kHalfWideMaxDp = 4096;
 constexpr uint32_t kHalfMaxLists = 512;   // lists per query the merge takes
 constexpr uint32_t kHalfMaxSel = 64;      // groups the merge selects per query at most
-// The scan's words per query in `words`: word 0 the union bound, kHalfSlotBase and up the bound slots,
-// kHalfScaleWord the query's scale (float bits, written by the prep kernel).
+// The scan's words per query in `words`: word 0 the shared bound, kHalfScaleWord the query's scale (float
+// bits, written by the prep kernel). The stride keeps every query's words on lines of their own.
 constexpr uint32_t kHalfWordStride = 64;
-constexpr uint32_t kHalfSlotBase = 32;
-constexpr uint32_t kHalfSlots = 32;
 constexpr uint32_t kHalfScaleWord = 1;
 
 /// The largest stored norm, from the store's meta words ([0] the largest squared norm, [2] the largest
@@ -66,7 +64,6 @@ struct HalfScanArgs {
   uint32_t* words;   // kHalfWordStride words per query
   int share;            // 0: every list keeps its own KL best
   uint32_t share_rank;  // nonzero: the shared bound is the larger of the lane pair's entries of this rank
-  int bound_slots;
   const uint32_t* meta;  // the store's meta words (stored_norm)
   const uint32_t* gate;  // the launch runs when (*gate != 0) == (gate_want != 0); null: always
   uint32_t gate_want;
