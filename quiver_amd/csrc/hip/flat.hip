@@ -17,6 +17,7 @@
 // re-score makes every returned distance bit-identical to the reference's for that row, and KL > k
 // keeps a margin of near-tied candidates for the re-score to choose from.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 #include <type_traits>
@@ -2693,6 +2694,24 @@ uint64_t choose_splits(uint64_t qblocks, uint64_t tiles, uint64_t max_splits, in
   return pick;
 }
 
+/// Whether rows wider than kHalfMaxDp are searched faster by the fp32 scan, whose merge scores single
+/// rows where the 16-bit scan's scores the about 16 k rows of k groups: over few rows the groups cost
+/// more than the scan saves. Both sides in rows of a work-group's share of the fp32 scan, from the
+/// plan's rounds and rows per split: the 16-bit scan takes 0.55 of its time per row, the groups
+/// 6e-5 per row and query (more for wide rows, whose groups the caches hold less of). Fitted to 734
+/// searches (136 to 2,048 dims, 1,000 to 80,000 rows, 1,000 to 5,000 queries, k 11 to 43): total
+/// time within 0.4% of the better side's, 1.8% behind it with the 16-bit scan always (k = 43:
+/// 10,000 x 768, 2,000 queries 585 us on fp32 and 790 on 16 bits; 50,000 rows 2,050 and 1,475;
+/// 2,000 x 2,048, 5,000 queries 1,260 and 2,650). Smaller batches, whose merge takes four waves a
+/// query, and lists of 16 are faster on the 16-bit scan at every size.
+bool fp32_wide_scan_faster(uint64_t nq, uint32_t k, uint64_t n, uint32_t dp, uint64_t rounds, uint64_t fp32_rows,
+                           uint64_t half_rows) {
+  if (nq <= kHalfMergeFour || shared_list_length(k) == 16) return false;
+  const double scored = static_cast<double>(nq) * static_cast<double>(std::min<uint64_t>(n, 16ull * k));
+  return static_cast<double>(rounds * fp32_rows) <
+         0.55 * static_cast<double>(rounds * half_rows) + 6e-5 * scored * std::pow(dp / 1024.0, 0.75);
+}
+
 /// d_idx (listed admitted rows) is in use when n_idx > 0 or `indexed`. half_wide = false keeps rows wider
 /// than kHalfMaxDp on the fp32 scan, which needs no split queries.
 FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool indexed, bool filtered, uint64_t n_idx,
@@ -2796,10 +2815,16 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
   p.fb = (nq + 2) * sizeof(uint32_t);  // count, listed queries, then the launch gate word
   if (p.half_wide) {
     // 256 queries and 256-row tiles per work-group, two lists per query and split: the splits above.
-    p.pair = true;
     const uint64_t tiles = std::max<uint64_t>(1, ceil_div(p.scan_rows, kHalfWideTileRows));
-    p.rows_per_split = ceil_div(tiles, p.nsplit) * kHalfWideTileRows;
-    p.qf = half_query_frag_bytes(nq, f->dp);
+    const uint64_t rows = ceil_div(tiles, p.nsplit) * kHalfWideTileRows;
+    const uint64_t rounds = ceil_div(p.qblocks * p.nsplit, static_cast<uint64_t>(cus));
+    if (fp32_wide_scan_faster(nq, k, p.scan_rows, f->dp, rounds, p.rows_per_split, rows)) {
+      p.half = p.half_wide = false;
+    } else {
+      p.pair = true;
+      p.rows_per_split = rows;
+      p.qf = half_query_frag_bytes(nq, f->dp);
+    }
   } else if (p.half) {
     // 512 queries per work-group (64 per wave) share a tile's conversion and LDS reads; fewer, two
     // waves take the halves of each tile for the same queries, up to 128 in 32-query groups (more

@@ -1067,13 +1067,9 @@ __global__ void __launch_bounds__(256) flat_half_merge_kernel(HalfMergeArgs m) {
   }
 }
 
-/// Batches up to which four waves take each query (100 queries over 128 dims: 33 -> 15 us; 1,003 over 96
-/// dims, k = 30: 85 us with one wave, 101 with four; 2,000 over 768 dims: 194 and 226).
-constexpr uint32_t kMergeWideQueries = 512;
-
 template <int KL>
 void launch_merge_kl(const HalfMergeArgs& m, hipStream_t s) {
-  const bool four = m.nq <= kMergeWideQueries;
+  const bool four = m.nq <= kHalfMergeFour;
   const dim3 grid(static_cast<unsigned>(four ? m.nq : ceil_div(m.nq, 4)));
   auto kernel = m.nlists <= 64 ? (four ? flat_half_merge_kernel<KL, 1, 4> : flat_half_merge_kernel<KL, 1, 1>)
                                : (four ? flat_half_merge_kernel<KL, 8, 4> : flat_half_merge_kernel<KL, 8, 1>);

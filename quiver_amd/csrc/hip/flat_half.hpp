@@ -17,6 +17,10 @@ constexpr uint32_t kHalfWideQueries = 256;     // per work-group
 constexpr uint32_t kHalfWideMaxDp = 4096;
 constexpr uint32_t kHalfMaxLists = 512;   // lists per query the merge takes
 constexpr uint32_t kHalfMaxSel = 64;      // groups the merge selects per query at most
+// Batches up to which the merge takes each query with four waves (whole searches, four waves -> one:
+// 600 queries, 5,000 x 768, k = 43 380 -> 545 us, 20,000 x 136, k = 11 175 -> 191 us; 1,000 queries
+// over 20,000 x 136, k = 22 213 -> 192 us; 2,000 over 768 dims, k = 10, the merge alone 226 -> 194 us).
+constexpr uint32_t kHalfMergeFour = 768;
 // The scan's words per query in `words`: word 0 the shared bound, kHalfScaleWord the query's scale (float
 // bits, written by the prep kernel). The stride keeps every query's words on lines of their own.
 constexpr uint32_t kHalfWordStride = 64;

@@ -142,3 +142,16 @@ def test_wide_blocks_and_filters(oracle, nq, n):
     _check(oracle, base, q, 25, "cosine")
     _check(oracle, base, q, 10, "l2", np.arange(0, n, 3, dtype=np.uint64))
     _check(oracle, np.round(2.0 * base), np.round(2.0 * q / np.abs(q).max()), 10, "l2")
+
+
+@pytest.mark.parametrize("nq,n,dim,k", [(600, 2_000, 768, 43), (768, 2_000, 768, 43), (769, 2_000, 768, 43),
+                                        (1_025, 3_000, 1_040, 43), (1_025, 700, 1_040, 21), (1_025, 12_000, 520, 25),
+                                        (1_025, 2_000, 768, 11)])
+def test_wide_large_batches(oracle, nq, n, dim, k):
+    """Batches past the merge's four waves a query, on both sides of the rule that gives few wide rows to
+    the fp32 scan; with listed rows too."""
+    rng = np.random.default_rng(n + k)
+    base, q = _normal(rng, n, dim), _normal(rng, nq, dim)
+    _check(oracle, base, q, k, "l2")
+    if k <= 21:
+        _check(oracle, base, q, k, "ip", np.arange(0, n, 2, dtype=np.uint64))
