@@ -1508,42 +1508,60 @@ __device__ __forceinline__ bool small_integer(float v) { return v == rintf(v) &&
 /// screening uses it), eight lanes per row so that a wave reads whole lines. Folds the rows into the
 /// store's bound data: meta[0] = largest squared norm (as float bits; non-negative floats order
 /// like their bits), meta[1] != 0 once a row holds a value that is not a small integer, meta[2] =
-/// largest magnitude (float bits). One atomic per wave and word.
+/// largest magnitude (float bits). The grid's at most kNormBlocks work-groups walk the rows and fold
+/// once each, and only what raises a word: atomics on the one line take 10 ns each, so one per
+/// wave and word over all rows was most of the kernel (50,000 x 64: 217 us; 1M x 16: 4 ms of a 6.6 ms
+/// append).
+constexpr uint32_t kNormBlocks = 1024;
 __global__ void __launch_bounds__(256) row_norms_kernel(const float* __restrict__ rows, float* __restrict__ out,
                                                         uint64_t n, uint32_t dp, uint32_t* __restrict__ meta) {
-  const uint64_t r = (static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x) / 8;
+  __shared__ uint32_t s_top[4], s_mag[4], s_mixed[4];
   const uint32_t l = threadIdx.x & 7u;
   bool integral = true;
-  double s = 0.0;
   float largest = 0.0f;
-  if (r < n) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(rows + r * dp);
-    for (uint32_t c = l; c < dp / 4; c += 8) {
-      const f32x4 v = p[c];
+  uint32_t top = 0;
+  for (uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * 32; r0 < n; r0 += static_cast<uint64_t>(gridDim.x) * 32) {
+    const uint64_t r = r0 + threadIdx.x / 8;
+    double s = 0.0;
+    if (r < n) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(rows + r * dp);
+#pragma unroll 4
+      for (uint32_t c = l; c < dp / 4; c += 8) {
+        const f32x4 v = p[c];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        integral = integral && small_integer(v[i]);
-        largest = fmaxf(largest, fabsf(v[i]));
-        s = fma(static_cast<double>(v[i]), static_cast<double>(v[i]), s);
+        for (int i = 0; i < 4; ++i) {
+          integral = integral && small_integer(v[i]);
+          largest = fmaxf(largest, fabsf(v[i]));
+          s = fma(static_cast<double>(v[i]), static_cast<double>(v[i]), s);
+        }
       }
     }
-  }
 #pragma unroll
-  for (int off = 4; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
-  const float n2 = static_cast<float>(s);
-  if (r < n && l == 0) out[r] = n2;
-  uint32_t top = __float_as_uint(n2 == n2 ? n2 : __builtin_huge_valf());
+    for (int off = 4; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
+    const float n2 = static_cast<float>(s);
+    if (r < n && l == 0) out[r] = n2;
+    top = max(top, __float_as_uint(n2 == n2 ? n2 : __builtin_huge_valf()));
+  }
   uint32_t mag = __float_as_uint(largest);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     top = max(top, static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), off, 64)));
     mag = max(mag, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mag), off, 64)));
   }
-  const bool all_integral = __ballot(!integral) == 0;
+  const bool mixed = __ballot(!integral) != 0;
   if ((threadIdx.x & 63) == 0) {
-    atomicMax(&meta[0], top);
-    atomicMax(&meta[2], mag);
-    if (!all_integral) atomicOr(&meta[1], 1u);
+    s_top[threadIdx.x >> 6] = top;
+    s_mag[threadIdx.x >> 6] = mag;
+    s_mixed[threadIdx.x >> 6] = mixed ? 1u : 0u;
+  }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    const uint32_t* const from = threadIdx.x == 0 ? s_top : threadIdx.x == 1 ? s_mixed : s_mag;
+    const uint32_t v = max(max(from[0], from[1]), max(from[2], from[3]));
+    // A word read stale is too small: at worst an atomic that changes nothing.
+    if (v > __hip_atomic_load(&meta[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      atomicMax(&meta[threadIdx.x], v);
+    }
   }
 }
 
@@ -3351,7 +3369,8 @@ void flat_append(qvh_flat* f, const float* rows, uint64_t n, float* stored_out, 
   const uint64_t total = n * f->dp;
   hipLaunchKernelGGL(pack_rows_kernel, dim3(static_cast<unsigned>(ceil_div(total, 256))), dim3(256), 0,
                      f->stream, stage, dst, n, f->dim, f->dp);
-  hipLaunchKernelGGL(row_norms_kernel, dim3(static_cast<unsigned>(ceil_div(n, 32))), dim3(256), 0,
+  const uint64_t norm_blocks = std::min<uint64_t>(ceil_div(n, 32), kNormBlocks);
+  hipLaunchKernelGGL(row_norms_kernel, dim3(static_cast<unsigned>(norm_blocks)), dim3(256), 0,
                      f->stream, dst, f->norms.as<float>() + f->n, n, f->dp, f->meta.as<uint32_t>());
   QVH_HIP(hipGetLastError());
   QVH_HIP(hipMemcpyAsync(f->h_meta, f->meta.ptr, sizeof(f->h_meta), hipMemcpyDeviceToHost, f->stream));

@@ -115,6 +115,19 @@ def test_integer_magnitudes(oracle, top):
     _check(oracle, base, q, 10, "l2")
 
 
+@pytest.mark.parametrize("row", [0, 32_767, 32_768, 70_000])
+@pytest.mark.parametrize("value", [0.3, 3_000.0])
+def test_one_row_decides_the_bound(oracle, row, value):
+    """One row that is no small integer, or above 2,048, among many that are: the store's bound data must
+    see it wherever the work-groups that collect them come to it (32,768 rows a step)."""
+    rng = np.random.default_rng(row)
+    base = rng.integers(-9, 10, (70_001, 16)).astype(np.float32)
+    base[row, 3] = value
+    q = rng.integers(-9, 10, (40, 16)).astype(np.float32)
+    q[:8, 3] = value
+    _check(oracle, base, q, 10, "l2")
+
+
 def test_equal_rows(oracle):
     """Every row stored 40 times: equal distances in row order, inside a group and across groups."""
     rng = np.random.default_rng(3)
