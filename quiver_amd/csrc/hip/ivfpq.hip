@@ -4111,6 +4111,14 @@ qvh_status qvh_points_nearest(qvh_points* p, const float* centroids, uint32_t k,
   });
 }
 
+/// What assigning to k centroids in each of nsub sub-spaces writes. qvh_points_nearest shares these
+/// buffers, and a failure there may have released one: every step reserves them.
+static void reserve_step(qvh_points* p, uint32_t k, uint32_t nsub) {
+  p->ct.reserve(static_cast<size_t>(k) * p->dim * sizeof(float));
+  p->norms.reserve(static_cast<size_t>(nsub) * k * sizeof(float));
+  p->out.reserve(std::max<uint64_t>(p->n, 1) * nsub * sizeof(uint32_t));
+}
+
 qvh_status qvh_points_set_centroids(qvh_points* p, const float* centroids, uint32_t k, uint32_t nsub) {
   return guarded([&] {
     QVH_REQUIRE(p && centroids, "qvh_points_set_centroids: null argument");
@@ -4120,11 +4128,10 @@ qvh_status qvh_points_set_centroids(qvh_points* p, const float* centroids, uint3
     QVH_REQUIRE(p->n < 0xFFFFFFFFull, "qvh_points_set_centroids: too many points");
     QVH_HIP(hipSetDevice(p->device));
     const size_t bytes = static_cast<size_t>(k) * p->dim * sizeof(float);
+    p->lk = 0;  // none while the buffers change: a failure below leaves no centroids behind
     p->lcent.reserve(bytes);
     p->lcounts.reserve(static_cast<size_t>(nsub) * k * sizeof(uint32_t));
-    p->ct.reserve(bytes);
-    p->norms.reserve(static_cast<size_t>(nsub) * k * sizeof(float));
-    p->out.reserve(std::max<uint64_t>(p->n, 1) * nsub * sizeof(uint32_t));
+    reserve_step(p, k, nsub);
     QVH_HIP(hipMemcpy(p->lcent.ptr, centroids, bytes, hipMemcpyHostToDevice));
     p->lk = k;
     p->nsub = nsub;
@@ -4142,6 +4149,7 @@ qvh_status qvh_points_step(qvh_points* p, uint32_t* counts) {
       std::fill(counts, counts + static_cast<size_t>(nsub) * k, 0u);
       return;
     }
+    reserve_step(p, k, nsub);
     hipLaunchKernelGGL(centroid_prep_kernel, dim3(static_cast<unsigned>(ceil_div(k, 256)), nsub), dim3(256), 0, nullptr,
                        p->lcent.as<float>(), k, dsub, p->ct.as<float>(), p->norms.as<float>());
     NearestArgs na{};
