@@ -283,6 +283,12 @@ qvh_status qvh_points_nearest(qvh_points* points, const float* centroids, uint32
 qvh_status qvh_points_set_centroids(qvh_points* points, const float* centroids, uint32_t k,
                                     uint32_t nsub);
 qvh_status qvh_points_step(qvh_points* points, uint32_t* counts);
+/* The same where no centroid gets more than `limit` points (*stepped = 1). Otherwise, and always with
+ * limit 0, the points are assigned and the centroids stay as they are (*stepped = 0; counts are then
+ * undefined), for a caller that takes the means itself from assigned's [nsub][n]: every point's
+ * centroid in the last step. */
+qvh_status qvh_points_step_within(qvh_points* points, uint32_t limit, uint32_t* counts, int* stepped);
+qvh_status qvh_points_assigned(qvh_points* points, uint32_t* assign);
 qvh_status qvh_points_get_centroids(qvh_points* points, float* centroids);
 
 /* ------------------------------------------------------------------------------------------ *

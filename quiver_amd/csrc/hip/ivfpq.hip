@@ -3956,8 +3956,11 @@ struct qvh_points {
   uint32_t dim = 0;
   int device = 0;
   DeviceBuffer x, cent, ct, norms, out, fb;
-  DeviceBuffer lcent, lcounts;  // Lloyd iterations: centroids [nsub][k][dim / nsub], points per centroid
-  uint32_t lk = 0, nsub = 0;
+  // Lloyd iterations: centroids [2][nsub][k][dim / nsub] (half lcur the installed ones, the other the
+  // next ones) and points per centroid.
+  DeviceBuffer lcent, lcounts;
+  uint32_t lk = 0, nsub = 0, lcur = 0;
+  float* centroids(uint32_t half) { return lcent.as<float>() + static_cast<size_t>(half) * lk * dim; }
   AssignTable asg;
   std::mutex mu;
 };
@@ -3969,7 +3972,8 @@ namespace {
 /// The update step of Lloyd's k-means. One wave per centroid (blockIdx.y the sub-space, blockIdx.z a
 /// block of 64 R dims): it scans the assignments, 1,024 at a time with the next ones in flight, and
 /// lists its points in LDS in index order; then each lane adds its dims of the listed points in
-/// double, in that order, 16 points' loads in flight. The scan reads every assignment once per
+/// double, in that order, 16 points' loads in flight. A centroid without points keeps its value; one
+/// of more than `limit` points is counted and not averaged. The scan reads every assignment once per
 /// centroid, from L2: 512 centroids over 50,000 x 64 take 69 us, sixteen sub-spaces of 256 centroids over
 /// 50,000 x 4 119 us together; the host's sums and the copies both ways took about 3 ms and 0.2 ms a
 /// sub-space.
@@ -3977,7 +3981,8 @@ constexpr uint32_t kUpdateList = 2048;
 template <int R>
 __global__ void __launch_bounds__(256) points_update_kernel(const float* __restrict__ x, uint64_t n, uint32_t stride,
                                                             uint32_t dsub, const uint32_t* __restrict__ assign,
-                                                            uint32_t k, float* __restrict__ cent,
+                                                            uint32_t k, uint32_t limit,
+                                                            const float* __restrict__ cent, float* __restrict__ out,
                                                             uint32_t* __restrict__ counts) {
   __shared__ uint32_t s_list[4][kUpdateList];
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -3992,7 +3997,8 @@ __global__ void __launch_bounds__(256) points_update_kernel(const float* __restr
   uint32_t held = 0, count = 0;
   auto add_listed = [&]() {
     __builtin_amdgcn_wave_barrier();
-    for (uint32_t e0 = 0; e0 < held; e0 += 16) {
+    const uint32_t add = count + held <= limit ? held : 0u;
+    for (uint32_t e0 = 0; e0 < add; e0 += 16) {
       float v[16][R];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -4016,7 +4022,7 @@ __global__ void __launch_bounds__(256) points_update_kernel(const float* __restr
     __builtin_amdgcn_wave_barrier();
   };
   constexpr int U = 16;
-  uint32_t now[U], next[U];
+  uint32_t now[U], ahead[U];
   auto load = [&](uint64_t i0, uint32_t(&v)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -4026,7 +4032,7 @@ __global__ void __launch_bounds__(256) points_update_kernel(const float* __restr
   };
   load(0, now);
   for (uint64_t i0 = 0; i0 < n; i0 += 64 * U) {
-    if (i0 + 64 * U < n) load(i0 + 64 * U, next);
+    if (i0 + 64 * U < n) load(i0 + 64 * U, ahead);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint64_t i = i0 + static_cast<uint64_t>(u) * 64 + lane;
@@ -4037,17 +4043,16 @@ __global__ void __launch_bounds__(256) points_update_kernel(const float* __restr
     }
     if (held > kUpdateList - 64 * U) add_listed();
 #pragma unroll
-    for (int u = 0; u < U; ++u) now[u] = next[u];
+    for (int u = 0; u < U; ++u) now[u] = ahead[u];
   }
   add_listed();
   if (lane == 0 && blockIdx.z == 0) counts[static_cast<uint64_t>(sub) * k + c] = count;
-  if (count == 0) return;
+  if (count > limit) return;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const uint32_t j = j0 + 64 * r + lane;
-    if (j < dsub) {
-      cent[(static_cast<uint64_t>(sub) * k + c) * dsub + j] = static_cast<float>(sum[r] / static_cast<double>(count));
-    }
+    const uint64_t at = (static_cast<uint64_t>(sub) * k + c) * dsub + j;
+    if (j < dsub) out[at] = count == 0 ? cent[at] : static_cast<float>(sum[r] / static_cast<double>(count));
   }
 }
 
@@ -4125,33 +4130,38 @@ qvh_status qvh_points_set_centroids(qvh_points* p, const float* centroids, uint3
     QVH_REQUIRE(k >= 1 && nsub >= 1 && nsub <= 65535 && p->dim % nsub == 0,
                 "qvh_points_set_centroids: k must be positive and nsub must divide the dimension");
     std::lock_guard<std::mutex> lock(p->mu);
-    QVH_REQUIRE(p->n < 0xFFFFFFFFull, "qvh_points_set_centroids: too many points");
     QVH_HIP(hipSetDevice(p->device));
     const size_t bytes = static_cast<size_t>(k) * p->dim * sizeof(float);
     p->lk = 0;  // none while the buffers change: a failure below leaves no centroids behind
-    p->lcent.reserve(bytes);
+    p->lcent.reserve(2 * bytes);
     p->lcounts.reserve(static_cast<size_t>(nsub) * k * sizeof(uint32_t));
     reserve_step(p, k, nsub);
     QVH_HIP(hipMemcpy(p->lcent.ptr, centroids, bytes, hipMemcpyHostToDevice));
     p->lk = k;
     p->nsub = nsub;
+    p->lcur = 0;
   });
 }
 
-qvh_status qvh_points_step(qvh_points* p, uint32_t* counts) {
+qvh_status qvh_points_step_within(qvh_points* p, uint32_t limit, uint32_t* counts, int* stepped) {
   return guarded([&] {
-    QVH_REQUIRE(p && counts, "qvh_points_step: null argument");
+    QVH_REQUIRE(p && counts && stepped, "qvh_points_step: null argument");
     std::lock_guard<std::mutex> lock(p->mu);
     QVH_REQUIRE(p->lk != 0, "qvh_points_step: no centroids");
+    QVH_REQUIRE(limit == 0 || p->n < 0xFFFFFFFFull, "qvh_points_step: too many points");
     QVH_HIP(hipSetDevice(p->device));
     const uint32_t k = p->lk, nsub = p->nsub, dsub = p->dim / nsub;
+    const size_t cells = static_cast<size_t>(nsub) * k;
     if (p->n == 0) {
-      std::fill(counts, counts + static_cast<size_t>(nsub) * k, 0u);
+      std::fill(counts, counts + cells, 0u);
+      *stepped = 1;
       return;
     }
+    *stepped = 0;
     reserve_step(p, k, nsub);
+    float* const cent = p->centroids(p->lcur);
     hipLaunchKernelGGL(centroid_prep_kernel, dim3(static_cast<unsigned>(ceil_div(k, 256)), nsub), dim3(256), 0, nullptr,
-                       p->lcent.as<float>(), k, dsub, p->ct.as<float>(), p->norms.as<float>());
+                       cent, k, dsub, p->ct.as<float>(), p->norms.as<float>());
     NearestArgs na{};
     na.x = p->x.as<float>();
     na.n = p->n;
@@ -4162,23 +4172,42 @@ qvh_status qvh_points_step(qvh_points* p, uint32_t* counts) {
     na.k = k;
     na.out32 = p->out.as<uint32_t>();
     if (nsub == 1) {
-      prepare_assign_table(p->asg, p->lcent.as<float>(), p->norms.as<float>(), k, dsub, 0, nullptr);
+      prepare_assign_table(p->asg, cent, p->norms.as<float>(), k, dsub, 0, nullptr);
       launch_assign(na, p->asg, p->fb, nullptr);
     } else {
       launch_nearest(false, na, nsub, nullptr);
     }
-    const unsigned waves = static_cast<unsigned>(ceil_div(k, 4));
-    if (dsub <= 64) {
-      hipLaunchKernelGGL(points_update_kernel<1>, dim3(waves, nsub), dim3(256), 0, nullptr, p->x.as<float>(), p->n,
-                         p->dim, dsub, p->out.as<uint32_t>(), k, p->lcent.as<float>(), p->lcounts.as<uint32_t>());
-    } else {
-      hipLaunchKernelGGL(points_update_kernel<2>, dim3(waves, nsub, static_cast<unsigned>(ceil_div(dsub, 128))),
-                         dim3(256), 0, nullptr, p->x.as<float>(), p->n, p->dim, dsub, p->out.as<uint32_t>(), k,
-                         p->lcent.as<float>(), p->lcounts.as<uint32_t>());
-    }
     QVH_HIP(hipGetLastError());
-    QVH_HIP(hipMemcpy(counts, p->lcounts.ptr, static_cast<size_t>(nsub) * k * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    if (limit != 0) {
+      const unsigned waves = static_cast<unsigned>(ceil_div(k, 4));
+      const bool narrow = dsub <= 64;
+      hipLaunchKernelGGL(narrow ? points_update_kernel<1> : points_update_kernel<2>,
+                         dim3(waves, nsub, narrow ? 1u : static_cast<unsigned>(ceil_div(dsub, 128))), dim3(256), 0,
+                         nullptr, p->x.as<float>(), p->n, p->dim, dsub, p->out.as<uint32_t>(), k, limit,
+                         cent, p->centroids(p->lcur ^ 1u), p->lcounts.as<uint32_t>());
+      QVH_HIP(hipGetLastError());
+      QVH_HIP(hipMemcpy(counts, p->lcounts.ptr, cells * sizeof(uint32_t), hipMemcpyDeviceToHost));
+      if (*std::max_element(counts, counts + cells) <= limit) {
+        p->lcur ^= 1u;
+        *stepped = 1;
+      }
+    }
   });
+}
+
+qvh_status qvh_points_assigned(qvh_points* p, uint32_t* assign) {
+  return guarded([&] {
+    QVH_REQUIRE(p && assign, "qvh_points_assigned: null argument");
+    std::lock_guard<std::mutex> lock(p->mu);
+    QVH_REQUIRE(p->lk != 0 && p->out.bytes >= p->n * p->nsub * sizeof(uint32_t), "qvh_points_assigned: no step");
+    QVH_HIP(hipSetDevice(p->device));
+    if (p->n) QVH_HIP(hipMemcpy(assign, p->out.ptr, p->n * p->nsub * sizeof(uint32_t), hipMemcpyDeviceToHost));
+  });
+}
+
+qvh_status qvh_points_step(qvh_points* p, uint32_t* counts) {
+  int stepped = 0;
+  return qvh_points_step_within(p, 0xFFFFFFFFu, counts, &stepped);
 }
 
 qvh_status qvh_points_get_centroids(qvh_points* p, float* centroids) {
@@ -4187,7 +4216,7 @@ qvh_status qvh_points_get_centroids(qvh_points* p, float* centroids) {
     std::lock_guard<std::mutex> lock(p->mu);
     QVH_REQUIRE(p->lk != 0, "qvh_points_get_centroids: no centroids");
     QVH_HIP(hipSetDevice(p->device));
-    QVH_HIP(hipMemcpy(centroids, p->lcent.ptr, static_cast<size_t>(p->lk) * p->dim * sizeof(float),
+    QVH_HIP(hipMemcpy(centroids, p->centroids(p->lcur), static_cast<size_t>(p->lk) * p->dim * sizeof(float),
                       hipMemcpyDeviceToHost));
   });
 }

@@ -52,6 +52,6 @@ std::vector<std::uint64_t> filter_bitmap(const Filter& filter, std::size_t n, La
 /// [j * dim / nsub, (j + 1) * dim / nsub), seeded params.seed + j), each as quiver::kmeans runs it on
 /// those columns alone: nsub x k x (dim / nsub) centroids. n <= k * max_points_per_centroid.
 std::vector<float> kmeans_subspaces(const float* vectors, std::size_t n, std::size_t dim, std::size_t nsub,
-                                    const KMeansParams& params);
+                                    const KMeansParams& params, ThreadPool* pool);
 
 }  // namespace quiver::internal

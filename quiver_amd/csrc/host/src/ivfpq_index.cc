@@ -151,7 +151,7 @@ struct IvfPqIndex::Impl {
     sp.k = kSubCentroids;
     sp.iterations = params.train_iterations;
     sp.seed = params.seed + 1;  // sub-space j: seed + 1 + j
-    std::vector<float> cb = internal::kmeans_subspaces(residuals.data(), pq_n, d, m, sp);
+    std::vector<float> cb = internal::kmeans_subspaces(residuals.data(), pq_n, d, m, sp, pool);
     std::unique_lock lock(mu);
     QUIVER_CHECK(!trained, "index is already trained");
     commit(std::move(cent), std::move(cb));

@@ -3,6 +3,7 @@
 #include <memory>
 #include <numeric>
 #include <random>
+#include <type_traits>
 
 #include "device_util.h"
 #include "quiver/quantizer.h"
@@ -39,34 +40,125 @@ void split_empty_clusters(float* cent, Count* counts, std::size_t k, std::size_t
   }
 }
 
-/// Lloyd iterations with the assignment and the means on the device, for nsub sub-spaces at once
-/// (each with its own centroids in cent [nsub][k][dim / nsub] and its own draws). The host sees the
-/// counts of each iteration, and the centroids when some cluster is empty.
-void lloyd_on_device(const float* x, std::size_t n, std::size_t dim, std::size_t nsub, std::size_t k,
-                     std::size_t iterations, std::vector<std::mt19937_64>& rng, std::vector<float>& cent) {
+/// Points in one cluster up to which an iteration takes its means on the device. There one wave adds a
+/// cluster's points one after another, 45 ns a point (78 past 64 dims), so the largest cluster decides;
+/// the host adds every point once, one thread per 8 dims and sub-space. The bits are the same.
+/// Nanoseconds a point and iteration, assignment included (four iterations of random points, host and
+/// device at k = 4, 16, 64, 256):
+///   65,536 points     4 dims  3.2, 12.7   2.9, 6.0   2.8, 3.4   3.2, 2.9
+///                    16 dims  5.4, 18.2   4.9, 7.6   5.0, 4.5   6.6, 4.1
+///                    64 dims  8.6, 22.0   7.9, 9.4    10, 6.5   8.9, 5.6
+///                   128 dims   19, 32      19, 16     20, 12     20, 9.3
+///   500,000          16 dims  4.2, 15     3.9, 7.0   4.0, 3.9   5.1, 2.8
+///                    64 dims   26, 19      23, 8.8    22, 5.8    22, 5.4
+/// (1 dim is the host's at every k up to 256, 2 dims up to 512; with points past the host's caches
+/// its sums wait for memory.) Past 256 centroids a dimension the device's reads of every assignment
+/// per centroid are left to the host's sums too.
+std::size_t device_means_limit(std::size_t n, std::size_t nsub, std::size_t dsub, std::size_t k) {
+  if (k > 256 * dsub || n >= 0xFFFFFFFFull) return 0;
+  const double points = static_cast<double>(n), dims = static_cast<double>(dsub);
+  const bool cached = points * dims * static_cast<double>(nsub) * sizeof(float) <= 48e6;
+  const double host_ns = dsub <= 8 ? 1.2 + 0.35 * dims : cached ? 3.5 + 0.12 * dims : 18.0 + 0.08 * dims;
+  const double device_ns = 1.7 + (dsub <= 8 ? 0.0 : 0.06 * dims);
+  const double even = (static_cast<double>(nsub) * host_ns - device_ns) / (dsub <= 64 ? 45.0 : 78.0);
+  // Past 8 dims more than the break-even: a first iteration's clusters are the least even ones, and the
+  // host loses the more the fewer its threads and the more the points.
+  const double lenient = dsub <= 8 ? 1.0 : dsub <= 16 ? 2.0 : 3.0;
+  const auto limit = static_cast<std::size_t>(std::clamp(lenient * even, 0.0, 1.0) * points);
+  // Some cluster holds at least n / k points, and of many the largest about three times that.
+  return points * (dsub <= 8 ? 3.0 : 1.0) > static_cast<double>(limit) * static_cast<double>(k) ? 0 : limit;
+}
+
+/// The means of the clusters with points of every sub-space into cent, counts[nsub][k] the points: each
+/// (cluster, dimension) adds its points in index order, in double. `sums` is scratch.
+void host_means(const float* x, std::size_t n, std::size_t dim, std::size_t nsub, std::size_t k,
+                const std::uint32_t* assign, std::vector<std::size_t>& counts, std::vector<double>& sums,
+                std::vector<float>& cent, ThreadPool& tp) {
+  const std::size_t dsub = dim / nsub, chunks = (dsub + 7) / 8;
+  std::fill(counts.begin(), counts.end(), std::size_t{0});
+  for (std::size_t s = 0; s < nsub; ++s) {
+    for (std::size_t i = 0; i < n; ++i) ++counts[s * k + assign[s * n + i]];
+  }
+  const std::size_t stride = k * 8 + 8;  // by chunk and a line apart: no thread writes to another's cache lines
+  sums.resize(nsub * chunks * stride);
+  tp.parallel_for(nsub * chunks, 1, [&](std::size_t begin, std::size_t end) {
+    for (std::size_t chunk = begin; chunk < end; ++chunk) {
+      const std::size_t s = chunk / chunks, jb = chunk % chunks * 8, je = std::min(dsub, jb + 8);
+      double* const sum = sums.data() + chunk * stride;
+      std::fill(sum, sum + k * 8, 0.0);
+      for (std::size_t i = 0; i < n; ++i) {
+        const float* const v = x + i * dim + s * dsub;
+        double* const to = sum + static_cast<std::size_t>(assign[s * n + i]) * 8;
+        for (std::size_t j = jb; j < je; ++j) to[j - jb] += static_cast<double>(v[j]);
+      }
+      for (std::size_t c = 0; c < k; ++c) {
+        const std::size_t count = counts[s * k + c];
+        if (count == 0) continue;
+        float* const mean = cent.data() + (s * k + c) * dsub;
+        for (std::size_t j = jb; j < je; ++j) mean[j] = static_cast<float>(sum[c * 8 + j - jb] / static_cast<double>(count));
+      }
+    }
+  });
+}
+
+/// Lloyd iterations for nsub sub-spaces at once, each with its own centroids in cent
+/// [nsub][k][dim / nsub] and its own draws: assignment on the device, means there or on the host
+/// (device_means_limit; an iteration that meets a larger cluster ends on the host, and so do the next
+/// ones while it stays so).
+void lloyd(const float* x, std::size_t n, std::size_t dim, std::size_t nsub, std::size_t k, std::size_t iterations,
+           std::vector<std::mt19937_64>& rng, std::vector<float>& cent, ThreadPool& tp) {
   if (iterations == 0) return;
   qvh_points* raw = nullptr;
   internal::qvh_check(qvh_points_create(x, n, static_cast<std::uint32_t>(dim), &raw), "kmeans");
   std::unique_ptr<qvh_points, PointsDeleter> points(raw);
   const std::size_t dsub = dim / nsub;
+  const std::size_t most = device_means_limit(n, nsub, dsub, k);
+  std::size_t limit = most;
   const auto install = [&] {
     internal::qvh_check(qvh_points_set_centroids(points.get(), cent.data(), static_cast<std::uint32_t>(k),
                                                  static_cast<std::uint32_t>(nsub)),
                         "kmeans centroids");
   };
+  const auto fetch = [&] { internal::qvh_check(qvh_points_get_centroids(points.get(), cent.data()), "kmeans centroids"); };
   install();
-  std::vector<std::uint32_t> counts(nsub * k);
+  bool fetched = true;  // cent holds the installed centroids
+  std::vector<std::uint32_t> device_counts(nsub * k), assign;
+  std::vector<std::size_t> host_counts;
+  std::vector<double> sums;
   for (std::size_t iter = 0; iter < iterations; ++iter) {
-    internal::qvh_check(qvh_points_step(points.get(), counts.data()), "kmeans step");
     const bool last = iter + 1 == iterations;
-    const bool empty = std::find(counts.begin(), counts.end(), 0u) != counts.end();
-    if (!last && !empty) continue;
-    internal::qvh_check(qvh_points_get_centroids(points.get(), cent.data()), "kmeans centroids");
-    if (!empty) continue;
-    for (std::size_t s = 0; s < nsub; ++s) {
-      split_empty_clusters(cent.data() + s * k * dsub, counts.data() + s * k, k, dsub, n, rng[s]);
+    int stepped = 0;
+    internal::qvh_check(qvh_points_step_within(points.get(), static_cast<std::uint32_t>(limit), device_counts.data(),
+                                               &stepped),
+                        "kmeans step");
+    // Splits the empty clusters of an iteration and installs what the host has changed.
+    const auto finish = [&](auto& counts, bool changed) {
+      using Count = typename std::decay_t<decltype(counts)>::value_type;
+      const bool empty = std::find(counts.begin(), counts.end(), Count{0}) != counts.end();
+      if (!fetched && (last || empty)) {
+        fetch();
+        fetched = true;
+      }
+      if (empty) {
+        for (std::size_t s = 0; s < nsub; ++s) {
+          split_empty_clusters(cent.data() + s * k * dsub, counts.data() + s * k, k, dsub, n, rng[s]);
+        }
+      }
+      if (!last && (changed || empty)) install();
+    };
+    if (stepped != 0) {
+      fetched = false;
+      finish(device_counts, false);
+    } else {
+      if (!fetched) fetch();
+      fetched = true;
+      assign.resize(nsub * n);
+      host_counts.resize(nsub * k);
+      internal::qvh_check(qvh_points_assigned(points.get(), assign.data()), "kmeans assignment");
+      host_means(x, n, dim, nsub, k, assign.data(), host_counts, sums, cent, tp);
+      limit = *std::max_element(host_counts.begin(), host_counts.end()) > most ? 0 : most;
+      finish(host_counts, true);
     }
-    if (!last) install();
   }
 }
 
@@ -84,16 +176,12 @@ void draw_initial(const float* x, std::size_t dim, std::size_t off, std::size_t 
   for (std::size_t i = k; i-- > 0;) std::swap(order[i], order[touched[i]]);
 }
 
-/// The device reads every assignment once per centroid, the host adds dim values per point: past 256
-/// centroids a dimension the host's sums are the cheaper ones (by the memory rates of both sides;
-/// every product-quantizer sub-space, with 256 centroids, is on the device's side).
-bool means_on_device(std::size_t k, std::size_t dim) { return k <= 256 * dim; }
 }  // namespace
 
 namespace internal {
 
 std::vector<float> kmeans_subspaces(const float* vectors, std::size_t n, std::size_t dim, std::size_t nsub,
-                                    const KMeansParams& params) {
+                                    const KMeansParams& params, ThreadPool* pool) {
   const std::size_t k = params.k, dsub = dim / nsub;
   std::vector<float> cent(nsub * k * dsub);
   std::vector<std::mt19937_64> rng;
@@ -103,7 +191,7 @@ std::vector<float> kmeans_subspaces(const float* vectors, std::size_t n, std::si
     rng.emplace_back(params.seed + s);
     draw_initial(vectors, dim, s * dsub, dsub, k, order, rng.back(), cent.data() + s * k * dsub);
   }
-  lloyd_on_device(vectors, n, dim, nsub, k, params.iterations, rng, cent);
+  lloyd(vectors, n, dim, nsub, k, params.iterations, rng, cent, pool ? *pool : ThreadPool::global());
   return cent;
 }
 
@@ -121,7 +209,6 @@ std::vector<float> kmeans(const float* vectors, std::size_t n, std::size_t dim,
   QUIVER_CHECK(n >= k, "kmeans: need at least k=" + std::to_string(k) + " training points, got " +
                            std::to_string(n));
   QUIVER_CHECK(k <= 0xFFFFFFFFull && dim <= 0xFFFFFFFFull, "kmeans: k or dim too large");
-  ThreadPool& tp = pool ? *pool : ThreadPool::global();
   std::mt19937_64 rng(params.seed);
 
   const float* x = vectors;
@@ -145,42 +232,8 @@ std::vector<float> kmeans(const float* vectors, std::size_t n, std::size_t dim,
     std::iota(order.begin(), order.end(), std::size_t{0});
     draw_initial(x, dim, 0, dim, k, order, rng, cent.data());
   }
-  if (means_on_device(k, dim) && n < 0xFFFFFFFFull) {
-    std::vector<std::mt19937_64> one{rng};
-    lloyd_on_device(x, n, dim, 1, k, params.iterations, one, cent);
-    return cent;
-  }
-
-  qvh_points* raw = nullptr;
-  internal::qvh_check(qvh_points_create(x, n, static_cast<std::uint32_t>(dim), &raw), "kmeans");
-  std::unique_ptr<qvh_points, PointsDeleter> points(raw);
-
-  std::vector<std::uint32_t> assign(n);
-  std::vector<double> sums(k * dim);
-  std::vector<std::size_t> counts(k);
-  for (std::size_t iter = 0; iter < params.iterations; ++iter) {
-    internal::qvh_check(qvh_points_nearest(points.get(), cent.data(), static_cast<std::uint32_t>(k), 0,
-                                           assign.data()),
-                        "kmeans assignment");
-    std::fill(counts.begin(), counts.end(), std::size_t{0});
-    for (std::size_t i = 0; i < n; ++i) ++counts[assign[i]];
-    // Per (cluster, dimension) the points are added in index order; chunks split dimensions.
-    tp.parallel_for(dim, 8, [&](std::size_t jb, std::size_t je) {
-      for (std::size_t c = 0; c < k; ++c)
-        for (std::size_t j = jb; j < je; ++j) sums[c * dim + j] = 0.0;
-      for (std::size_t i = 0; i < n; ++i) {
-        const std::size_t c = assign[i];
-        for (std::size_t j = jb; j < je; ++j) sums[c * dim + j] += static_cast<double>(x[i * dim + j]);
-      }
-    });
-    for (std::size_t c = 0; c < k; ++c) {
-      if (counts[c] == 0) continue;
-      for (std::size_t j = 0; j < dim; ++j) {
-        cent[c * dim + j] = static_cast<float>(sums[c * dim + j] / static_cast<double>(counts[c]));
-      }
-    }
-    split_empty_clusters(cent.data(), counts.data(), k, dim, n, rng);
-  }
+  std::vector<std::mt19937_64> one{rng};
+  lloyd(x, n, dim, 1, k, params.iterations, one, cent, pool ? *pool : ThreadPool::global());
   return cent;
 }
 

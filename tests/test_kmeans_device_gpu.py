@@ -59,3 +59,28 @@ def test_sub_spaces_together(oracle, dim, m):
     cent, cb, _ = oracle.ivfpq_train(x, "l2", 8, m, 5, 1234)
     assert np.array_equal(idx.centroids.view(np.uint32), cent.view(np.uint32))
     assert np.array_equal(idx.codebook.view(np.uint32), cb.view(np.uint32))
+
+
+@pytest.mark.parametrize("dim,k", [(2, 64), (4, 256), (8, 64), (16, 40), (40, 8), (64, 8), (128, 3)])
+@pytest.mark.parametrize("share", [0.0, 0.5, 0.97])
+def test_dominating_clusters(oracle, dim, k, share):
+    """One cluster that holds a share of the points: the means are taken on the device, on the host, or on
+    the host from the first iteration that meets too large a cluster."""
+    rng = np.random.default_rng(dim + k)
+    x = rng.standard_normal((6_000, dim)).astype(np.float32)
+    x[: int(share * 6_000)] = 50.0 + 0.01 * x[: int(share * 6_000)]
+    x = x[rng.permutation(6_000)]
+    _same(oracle, x, k, 6, max_points_per_centroid=10_000)
+
+
+@pytest.mark.parametrize("m", [2, 8, 16])
+def test_dominating_clusters_in_sub_spaces(oracle, m):
+    x = np.random.default_rng(m).standard_normal((1_500, 4 * m)).astype(np.float32)
+    x[:1_200, :4] = 7.0
+    x[:700, 4:8] = -3.0
+    idx = quiver.IvfPqIndex(4 * m, "l2", nlist=4, m=m, train_iterations=5)
+    print(f"case: train {m}", flush=True)
+    idx.train(x)
+    cent, cb, _ = oracle.ivfpq_train(x, "l2", 4, m, 5, 1234)
+    assert np.array_equal(idx.centroids.view(np.uint32), cent.view(np.uint32))
+    assert np.array_equal(idx.codebook.view(np.uint32), cb.view(np.uint32))
