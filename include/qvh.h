@@ -75,6 +75,10 @@ qvh_status qvh_device_info(char* name, size_t name_len, char* arch, size_t arch_
  * legacy null stream here) and waits for it. */
 qvh_status qvh_device_finite(const float* d_x, uint64_t count, void* stream, int* finite);
 
+/* Copies `bytes` of host memory to the device on `stream` (NULL = the legacy null stream here) and waits
+ * for it. */
+qvh_status qvh_upload(void* d_dst, const void* src, uint64_t bytes, void* stream);
+
 /* Result rows to labels on the device, enqueued on `stream` (not NULL): out[i] = table[rows[i]], or -1
  * for QVH_EMPTY_ROW; `table` holds n labels by row. */
 qvh_status qvh_map_rows_device(const uint32_t* d_rows, uint64_t count, const uint64_t* d_table,

@@ -378,7 +378,9 @@ class FlatIndex:
 
         cached = getattr(self, "_dev_labels", None)
         if cached is None or cached[0] != (n, device):
-            cached = ((n, device), torch.from_numpy(self._index._labels().view(np.int64)).to(device))
+            table = torch.empty(n, dtype=torch.int64, device=device)
+            self._index._upload_labels(table.data_ptr(), n, torch.cuda.current_stream(device).cuda_stream)
+            cached = ((n, device), table)
             self._dev_labels = cached
         return cached[1]
 

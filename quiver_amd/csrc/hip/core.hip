@@ -228,6 +228,17 @@ qvh_status qvh_device_finite(const float* d_x, uint64_t count, void* stream, int
   });
 }
 
+qvh_status qvh_upload(void* d_dst, const void* src, uint64_t bytes, void* stream) {
+  return qvh::guarded([&] {
+    if (bytes == 0) return;
+    QVH_REQUIRE(d_dst && src, "qvh_upload: null buffer");
+    qvh::current_device();
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    QVH_HIP(hipMemcpyAsync(d_dst, src, bytes, hipMemcpyHostToDevice, s));
+    QVH_HIP(hipStreamSynchronize(s));
+  });
+}
+
 qvh_status qvh_map_rows_device(const uint32_t* d_rows, uint64_t count, const uint64_t* d_table, uint64_t n,
                                int64_t* d_labels, void* stream) {
   return qvh::guarded([&] {

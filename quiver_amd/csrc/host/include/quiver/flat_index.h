@@ -73,6 +73,9 @@ class FlatIndex {
   /// Labels by row.
   std::vector<Label> labels() const;
 
+  /// Copies the first n labels into a device buffer, on `stream` (null: the null stream), and waits.
+  void upload_labels(std::uint64_t* device, std::size_t n, void* stream) const;
+
  private:
   void search_rows(const float* queries, std::size_t nq, std::size_t k, const Filter* filter,
                    ThreadPool* pool, Label* labels, float* distances) const;

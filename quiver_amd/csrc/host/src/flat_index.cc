@@ -156,6 +156,13 @@ std::vector<std::uint64_t> FlatIndex::row_bitmap(const Filter& filter) const {
                                  ThreadPool::global());
 }
 
+void FlatIndex::upload_labels(std::uint64_t* device, std::size_t n, void* stream) const {
+  std::shared_lock lock(*mu_);
+  QUIVER_CHECK(n <= labels_.size(), "upload_labels: more labels than rows");
+  static_assert(sizeof(Label) == sizeof(std::uint64_t));
+  internal::qvh_check(qvh_upload(device, labels_.data(), n * sizeof(Label), stream), "labels");
+}
+
 std::vector<Label> FlatIndex::labels() const {
   std::shared_lock lock(*mu_);
   return labels_;

@@ -268,6 +268,11 @@ PYBIND11_MODULE(_quiver, m) {
              }
              return py::array_t<std::uint64_t>(static_cast<py::ssize_t>(bits.size()), bits.data());
            })
+      .def("_upload_labels",
+           [](const quiver::FlatIndex& self, std::uintptr_t device, std::size_t n, std::uintptr_t stream) {
+             py::gil_scoped_release release;
+             self.upload_labels(reinterpret_cast<std::uint64_t*>(device), n, reinterpret_cast<void*>(stream));
+           })
       .def("_labels",
            [](const quiver::FlatIndex& self) {
              const auto l = self.labels();

@@ -195,3 +195,50 @@ def test_calls_on_two_streams_share_the_handle_safely(kind):
     _same(want_a, got_a)
     _same(want_b, got_b)
     assert np.array_equal(want_a[0], again_a[0])
+
+
+@pytest.mark.parametrize("kind", ["flat", "ivfpq"])
+@pytest.mark.parametrize("nq", [1, 40])
+@pytest.mark.parametrize("admitted", [0, 1, 4])
+def test_device_filters_that_admit_fewer_than_k(kind, nq, admitted):
+    """Every slot of the results is written: -1 and +inf behind the admitted rows, in memory that held
+    other values before."""
+    import torch
+
+    rng = np.random.default_rng(admitted)
+    n, k = 5_000, 10
+    base, q = rng.standard_normal((n, 32)).astype(np.float32), rng.standard_normal((nq, 32)).astype(np.float32)
+    allowed = np.sort(rng.choice(n, admitted, replace=False)).astype(np.uint64)
+    if kind == "flat":
+        idx = quiver.FlatIndex(32)
+        options = {}
+    else:
+        idx = quiver.IvfPqIndex(32, nlist=16, m=8, train_iterations=3)
+        idx.train(base)
+        options = {"nprobe": 16}
+    idx.add(base)
+    dq = torch.from_numpy(q).to("cuda:0")
+    held = [torch.full((nq, k), 77, dtype=dt, device="cuda:0") for dt in (torch.int64, torch.float32, torch.int32)]
+    del held
+    print(f"case: {kind} nq={nq} admitted={admitted}", flush=True)
+    labels, dist = idx.search(dq, k, filter=allowed, **options)
+    host_labels, host_dist = idx.search(q, k, filter=allowed, **options)
+    assert np.array_equal(labels.cpu().numpy(), host_labels)
+    assert np.array_equal(dist.cpu().numpy().view(np.uint32), host_dist.view(np.uint32))
+    assert (host_labels[:, admitted:] == -1).all() and np.isinf(host_dist[:, admitted:]).all()
+    assert (np.sort(host_labels[:, :admitted], axis=1) == allowed.astype(np.int64)).all()
+
+
+def test_flat_device_labels_of_one_index_after_another():
+    """Labels of the caller's choice, of an index that grows, and of one made after another is gone."""
+    import torch
+
+    rng = np.random.default_rng(5)
+    for n in (1_000, 3_000):
+        base = rng.standard_normal((n, 16)).astype(np.float32)
+        own = rng.permutation(10 * n)[:n].astype(np.uint64)
+        idx = quiver.FlatIndex(16)
+        for part in (slice(0, n // 3), slice(n // 3, n)):
+            idx.add(base[part], own[part])
+            labels, _ = idx.search(torch.from_numpy(base[part]).to("cuda:0"), 1)
+            assert np.array_equal(labels.cpu().numpy()[:, 0], own[part].astype(np.int64))
