@@ -153,3 +153,29 @@ def test_noalloc_calls_on_two_handles_and_streams_take_the_array_in_turn():
         for h in handles:
             L.qvh_flat_destroy(h)
         dev.free()
+
+
+@pytest.mark.parametrize("dim,nq,k,integers", [(768, 300, 10, False), (768, 300, 30, False), (2_048, 5_000, 10, False),
+                                               (2_048, 5_000, 10, True), (1_024, 8_000, 15, False)])
+def test_noalloc_search_of_wide_rows(dim, nq, k, integers):
+    """Rows wider than 128 dims on both sides of the fixed array's size: with the split queries of the
+    16-bit scan in it, and where only the fp32 scan's workspace fits."""
+    L, dev = _lib(), Dev()
+    rng = np.random.default_rng(dim + k)
+    make = (lambda *s: rng.integers(-3, 4, s).astype(np.float32)) if integers else \
+        (lambda *s: rng.standard_normal(s).astype(np.float32))
+    base, q = make(1_500, dim), make(nq, dim)
+    h = _vp()
+    assert L.qvh_flat_create(dim, 0, C.byref(h)) == 0, L.qvh_last_error().decode()
+    try:
+        assert L.qvh_flat_append(h, base.ctypes.data_as(_vp), base.shape[0], None) == 0
+        d_q = dev.put(q)
+        print(f"case: noalloc dim={dim} nq={nq} k={k}", flush=True)
+        want = _search(L, dev, L.qvh_flat_search_device, h, d_q, nq, k)
+        allocs = _allocations(L)
+        got = _search(L, dev, L.qvh_flat_search_device_noalloc, h, d_q, nq, k)
+        assert _allocations(L) == allocs, "the no-allocation entry point allocated device memory"
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1].view(np.uint32), want[1].view(np.uint32))
+    finally:
+        L.qvh_flat_destroy(h)
+        dev.free()
