@@ -6,6 +6,7 @@
 * ``quiver_amd/lib/libquiver_amd.so`` - the C++ API (quiver::FlatIndex, ...) over the C-ABI
 * ``quiver_amd/_quiver*.so``          - the pybind11 module under quiver_amd/__init__.py
 * ``tests/cpp/test_cpp_api``          - the C++ API test program (run by tests/test_cpp_api_gpu.py)
+* ``tests/cpp/libhalf_scan_probe.so`` - matrix steps and scan minima (tests/test_flat_half_bound_gpu.py)
 
 Every HIP source is compiled with -ffp-contract=off (fused multiply-adds only where the source
 writes fmaf(), as the bit-exact paths require) and without packed-FP32 instructions.
@@ -106,6 +107,11 @@ def build_cpp_tests() -> str:
     _run(["g++", *CXX_FLAGS, src, f"-L{LIB}", "-lquiver_amd", "-lqvh", f"-Wl,-rpath,{LIB}",
           "-Wl,-rpath,$ORIGIN/../../quiver_amd/lib", "-o", out + ".tmp"])
     os.replace(out + ".tmp", out)
+    src = os.path.join(ROOT, "tests", "cpp", "half_scan_probe.hip")
+    probe = os.path.join(ROOT, "tests", "cpp", "libhalf_scan_probe.so")
+    _run([_hipcc(), *HIPCC_FLAGS, "-shared", src, f"-L{LIB}", "-lqvh", f"-Wl,-rpath,{LIB}",
+          "-Wl,-rpath,$ORIGIN/../../quiver_amd/lib", "-o", probe + ".tmp"])
+    os.replace(probe + ".tmp", probe)
     return out
 
 

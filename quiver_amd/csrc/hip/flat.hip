@@ -1587,21 +1587,26 @@ __global__ void __launch_bounds__(256) row_norms_kernel(const float* __restrict_
 ///
 /// With `half` (the scan on the 16-bit matrix unit, flat_half.hip; thr is then set), also the query's
 /// scale into word kHalfScaleWord of its thr words, and a bound of that scan's own. Its value of a
-/// row differs from the true distance by at most, in units of u (P + R)^2 (L2; u (1 + P R) for the
-/// inner product):
-///   2 + 6      the norms (summed in double, rounded once) and the split operands: |lo| <= 2^-11 |x|,
-///              so dropping lo.lo and rounding lo cost 3 x 2^-22 sum |q_i x_i| = 12 u P R, at most
-///              6 u (P + R)^2 doubled; halves below the fp16 range add less than 2;
+/// row differs from the true distance by at most, in units of u (P + R)^2 for L2 and of u (1 + P R) for
+/// the inner product:
+///   split      |lo| <= 2^-11 |x|, so dropping lo.lo and rounding lo cost 3 x 2^-22 sum |q_i x_i| =
+///              12 u P R: 12 of the inner product, and doubled at most 6 of L2 (P R <= (P + R)^2 / 4);
+///              halves below the fp16 range add less than 2;
+///   norms      L2: 2 (summed in double, rounded once);
 ///   n/16 + 1   matrix steps on the sum proper, each within 18 u of the sum of its magnitudes (17
 ///              addends each truncated at 2^-24 of the largest, one rounding; the steps of the small
-///              products come first and count 2^-10 of that): 1.125 n + 18;
+///              products come first and count 2^-10 of that): 1.125 n + 18. A half below fp16's
+///              normal range counts as 2^-14 there (the unit aligns by exponents), which beside the
+///              scaled norms of 2^10 adds at most 2^-15 of it (n = 4,096);
 ///   2          the value's way back to a distance;
 /// and the reference's own sum, which adds every term through at most n/32 + 15 roundings
-/// (src/simd/kernels_avx2.cc:35-83: four 8-lane chains, a tree, a tail of up to 7), two of them in
-/// the difference: n/32 + 18. Together below 1.16 n + 50; delta uses 1.25 n + 64. The form for wide rows
-/// (half = 2) takes its three products step by step, so all 3 n/16 of its steps count in full
-/// (3.375 n): 3.5 n + 64. delta is 0 under the condition above if also no stored or query value exceeds 2048 in magnitude: hi then holds every
-/// value, lo is 0, and the sums are exact.
+/// (src/simd/kernels_avx2.cc:35-83: four 8-lane chains, a tree, a tail of up to 7), for L2 two more in
+/// the difference, for the inner product one: n/32 + 17. Together 1.16 n + 47 (L2) and 1.16 n + 50;
+/// delta uses 1.25 n + 64. The form for wide rows (half = 2) takes its three products step by step, so
+/// all 3 n/16 of its steps count in full (3.375 n): 3.5 n + 64. delta is 0 under the condition above if
+/// also no stored or query value exceeds 2048 in magnitude: hi then holds every value, lo is 0, and
+/// the sums are exact. tests/test_flat_half_bound_gpu.py measures the matrix step and the scans'
+/// minima against 64-bit values.
 __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restrict__ src, float* __restrict__ qp,
                                                            uint64_t nq, uint32_t dim, uint32_t dp,
                                                            float* __restrict__ qn, const uint32_t* __restrict__ meta,
@@ -1642,22 +1647,14 @@ __global__ void __launch_bounds__(256) prep_queries_kernel(const float* __restri
   const double P = n2 < __builtin_huge_valf() ? sqrt(s) : __builtin_huge_val();
   const double R = stored_norm(meta, dp);
   if (half) {
-    // L2: the norm step's weight 2^8 s_q / s_x stays within fp16 (a zero query takes its upper end:
-    // at 1 the weight would be 0 for rows of norms below 2^-22, and nothing could be certified).
-    const float sx = half_scale(R), sq = half_scale(P);
-    thr[q * thr_stride + kHalfScaleWord] =
-        __float_as_uint(l2 && (P == 0.0 || sq > 128.0f * sx) ? 128.0f * sx : sq);
+    thr[q * thr_stride + kHalfScaleWord] = __float_as_uint(half_query_scale(P, R, l2 != 0));
   }
-  const double u = 1.0 / 16777216.0;
-  const double coef = (half == 2 ? 3.5 * dp + 64.0 : half == 1 ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;
   double d;
   if (integral && meta[1] == 0 && (P + R) * (P + R) * (1.0 + 1e-12) <= 16777216.0 &&
       (!half || (largest <= 2048.0f && __uint_as_float(meta[2]) <= 2048.0f))) {
     d = 0.0;
-  } else if (l2) {
-    d = coef * (P + R) * (P + R) + (dp + 32.0) * 0x1p-149;
   } else {
-    d = coef * (1.0 + P * R);
+    d = scan_bound(half, dp, l2 != 0, P, R);
   }
   const float df = static_cast<float>(d);
   delta[q] = static_cast<double>(df) < d ? __uint_as_float(__float_as_uint(df) + 1u) : df;

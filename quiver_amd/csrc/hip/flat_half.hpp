@@ -47,11 +47,28 @@ __device__ __forceinline__ float half_scale(double norm) {
   return ldexpf(1.0f, e < -100 ? -100 : e > 100 ? 100 : e);
 }
 
+/// The scale of a query of norm P against a store of largest norm R. L2: the norm step's weight
+/// 2^8 s_q / s_x stays within fp16 (a zero query takes its upper end: at 1 the weight would be 0 for rows
+/// of norms below 2^-22, and nothing could be certified).
+__device__ __forceinline__ float half_query_scale(double P, double R, bool l2) {
+  const float sx = half_scale(R), sq = half_scale(P);
+  return l2 && (P == 0.0 || sq > 128.0f * sx) ? 128.0f * sx : sq;
+}
+
+/// The bound on |scan's distance - reference's| for a query of norm P over rows of norms up to R, unless
+/// every sum is exact: form 0 is the fp32 scans', 1 and 2 the 16-bit scans' up to kHalfMaxDp and above.
+/// prep_queries_kernel derives it.
+__device__ __forceinline__ double scan_bound(int form, uint32_t dp, bool l2, double P, double R) {
+  const double u = 1.0 / 16777216.0;
+  const double coef = (form == 2 ? 3.5 * dp + 64.0 : form == 1 ? 1.25 * dp + 64.0 : 4.0 * dp + 16.0) * u;
+  return l2 ? coef * (P + R) * (P + R) + (dp + 32.0) * 0x1p-149 : coef * (1.0 + P * R);
+}
+
 struct HalfScanArgs {
   const float* X;          // [rows][dp] rows as stored (or the contiguous copy of listed rows)
   const float* xnorm;      // [rows] ||x||^2 (L2)
   uint64_t n;              // rows scanned
-  uint32_t dp;             // row width, a multiple of 8 in [16, 128]
+  uint32_t dp;             // row width: a multiple of 8 in [16, 128], for the wide form of 16 up to kHalfWideMaxDp
   const float* Q;          // [nq][dp] prepared queries
   const float* qnorm;      // [nq] ||q||^2
   uint32_t nq;
@@ -69,7 +86,8 @@ struct HalfScanArgs {
   int share;            // 0: every list keeps its own KL best
   uint32_t share_rank;  // nonzero: the shared bound is the larger of the lane pair's entries of this rank
   const uint32_t* meta;  // the store's meta words (stored_norm)
-  const uint32_t* gate;  // the launch runs when (*gate != 0) == (gate_want != 0); null: always
+  // The launch runs when (*gate != 0) == (gate_want != 0); null: always (the wide form takes none).
+  const uint32_t* gate;
   uint32_t gate_want;
   const void* qfrag;  // wide rows: the split queries (launch_half_query_frags)
 };
