@@ -206,7 +206,8 @@ class IvfPqIndex:
         store_vectors: keep float32 copies to enable exact re-ranking (``refine_factor``).
 
     Call :meth:`train` on a representative sample before :meth:`add`. Encoding and search run on
-    the GPU; training runs the reference's k-means with its assignment steps on the GPU.
+    the GPU; training runs the reference's k-means with its assignments, and
+    its means where clusters are many or wide, on the GPU.
     """
 
     def __init__(self, dim: int, metric: str = "l2", nlist: int = 1024, m: int = 16,
@@ -326,7 +327,8 @@ def kmeans(vectors: ArrayLike, k: int, iterations: int = 25, max_points_per_cent
 
 
 class FlatIndex:
-    """Exact brute-force index; the scan is a fused FP32-MFMA GEMM + top-k kernel on the GPU."""
+    """Exact brute-force index; the scan is a fused matrix-unit GEMM + top-k kernel on the GPU
+    (fp16 halves of the fp32 values for k up to 43, fp32 above), re-scored in fp32."""
 
     def __init__(self, dim: int, metric: str = "l2", *, _native=None):
         self._index = _native if _native is not None else _quiver.FlatIndex(dim, metric)

@@ -69,8 +69,9 @@ struct ScanArgs {
   int share;                // 0: every lane list keeps its own KL best (k > KL: no shared bound)
   uint32_t dp;              // row width (the chunked scan; the register scan has it as DP)
   int rowsplit;             // register scan, unfiltered, at most 128 queries: two waves per query group
-  // Launch gate: when set, the launch does nothing unless (*gate != 0) == (gate_want != 0), read
-  // once at the start. Two list lengths are launched back to back and the device picks one.
+  // Launch gate of the chunked scan: when set, the launch does nothing unless (*gate != 0) ==
+  // (gate_want != 0), read once at the start. Two list lengths are launched back to back and the device
+  // picks one.
   const uint32_t* gate;
   uint32_t gate_want;
 };
@@ -774,7 +775,6 @@ __global__ void __launch_bounds__(kRingThreads) flat_ring_kernel(ScanArgs a) {
   static_assert(DP % 32 == 0 && DP <= kMaxDp, "the ring scan takes whole 32-dim quarters");
   static_assert(kRingWaves / 2 * KL * 64 * 2 <= kRingWaves * kRingSlots * kRingSlotFloats, "list hand-off fits the rings");
   static_assert((kRingWaves & (kRingWaves - 1)) == 0 && kRingWaves >= 2, "the hand-off halves the waves");
-  if (gate_closed(a.gate, a.gate_want)) return;  // the same for every thread of the grid
   constexpr int NQ = DP / 32;  // quarters per block
   constexpr int R = kRingSlots;
   constexpr int SLOT_BYTES = kRingSlotFloats * 4;
@@ -2451,8 +2451,8 @@ uint32_t wide_selection(uint32_t k) { return k + std::max<uint32_t>(16, k / 2); 
 
 /// List length for a batch whose GEMM-form distances are all exact (every query's delta is 0:
 /// small-integer queries against a store of small integers), which needs no margin over k; 0 when
-/// none applies. 1M x 128 integer mixture, k = 10: scan 22.30 -> 21.53 ms, merge 82 -> 65 us (12
-/// entries: 21.79 ms).
+/// none applies. On the 16-bit unit such a batch also takes one product of halves instead of three
+/// (1M x 128 integer mixture, 10,000 queries: 2.9 ms of scan; 1.18M x 100 of real values 7.3 ms).
 int exact_list_length(uint32_t k) { return k <= 10 ? 10 : 0; }
 
 template <int DP>
@@ -2709,6 +2709,10 @@ uint64_t choose_splits(uint64_t qblocks, uint64_t tiles, uint64_t max_splits, in
   return pick;
 }
 
+static_assert(kQueriesPerBlock == static_cast<int>(kHalfWideQueries) && 2 * kMaxSplits <= kHalfMaxLists &&
+                  kMaxChunkedDp == kHalfWideMaxDp,
+              "the wide form of the 16-bit scan takes the chunked scan's query blocks and splits");
+
 /// Whether rows wider than kHalfMaxDp are searched faster by the fp32 scan, whose merge scores single
 /// rows where the 16-bit scan's scores the about 16 k rows of k groups: over few rows the groups cost
 /// more than the scan saves. Both sides in rows of a work-group's share of the fp32 scan, from the
@@ -2749,11 +2753,12 @@ FlatPlan plan_flat_search(const qvh_flat* f, uint64_t nq, uint32_t k, bool index
   }
   // At most kFewMaxBatch queries with 32 <= dim <= kFewMaxDim and k <= kFewMaxK: the few-query
   // scan, kFewMaxQ queries per launch;
-  // other batches of at most kSplitMaxQueries: the exact kernel over row splits. Otherwise k with a
-  // margin in a shared-bound list (shared_list_length): the MFMA scan with per-lane lists of KL = 16
-  // or 32 and a shared bound; larger k up to kWideMaxK: the same scan without the shared bound and
-  // the wide merge (its rare fallback queries on the exact kernel); larger k or dim: the exact kernel.
-  // Rows wider than kMaxDp (up to kMaxChunkedDp) take the chunked form of the MFMA scan.
+  // other batches of at most kSplitMaxQueries: the exact kernel over row splits. Otherwise the matrix
+  // scans. k up to 43: the 16-bit unit, k with a margin in lists of 16 or 32 groups (shared_list_length)
+  // under a shared bound, from 22 on lists of 32 of which the merge takes up to 64 groups; rows wider
+  // than kMaxDp take its wide form, or the chunked fp32 scan over few rows (fp32_wide_scan_faster)
+  // and where the split queries do not fit. k from 44 to kWideMaxK: the fp32 scan (chunked above
+  // kMaxDp) without a shared bound and the wide merge. Larger k or dim: the exact kernel.
   // kRingMinQueries to kRingMaxQueries unfiltered queries whose rows are whole 32-dim quarters,
   // with k in the shared-bound lists: the ring scan (its lists go to the same merge as the MFMA
   // scan's); fewer queries too when the rows are too few to split for the few-query kernel.

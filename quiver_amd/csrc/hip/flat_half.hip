@@ -1124,6 +1124,7 @@ void launch_half_query_frags(const float* Q, uint32_t nq, uint32_t dp, const uin
 }
 
 void launch_half_wide_scan(int kl, dim3 grid, const HalfScanArgs& a, hipStream_t s) {
+  if (a.gate != nullptr) throw Failure(QVH_EUNSUPPORTED, "half scan: the wide form takes no gate");
   if (kl == 16) {
     hipLaunchKernelGGL(flat_half_wide_kernel<16>, grid, dim3(kThreads), 0, s, a);
   } else {

@@ -1,10 +1,10 @@
 // k-means, nearest_centroid and the product quantizer, with the reference's interface
 // (include/quiver/quantizer.h:47-114).
 //
-// k-means runs its control flow (subsample, random initialization, double-precision centroid sums,
-// empty-cluster splitting) on the host with the reference's random engine; every assignment step is
-// one call of the device's exact nearest-centroid kernel (qvh_points_nearest), so the centroids
-// come out bit-identical to the reference's. The reference's per-vector methods (nearest_centroid,
+// k-means runs its control flow (subsample, random initialization, empty-cluster splitting) on the host
+// with the reference's random engine; the assignments run on the device (qvh_points_step_within), and the
+// double-precision means there or on the host, whichever is less work, in the same order, so the
+// centroids come out bit-identical to the reference's. The reference's per-vector methods (nearest_centroid,
 // ProductQuantizer::encode / decode / compute_*_table / adc / adc_batch) run on the host in the
 // reference's float order and cannot fail, as the reference's noexcept versions cannot; the
 // *_batch methods (no reference counterpart) run many vectors per device call (qvh_nearest_centroid,

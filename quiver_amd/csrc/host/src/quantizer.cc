@@ -138,8 +138,8 @@ ProductQuantizer::ProductQuantizer(std::size_t dim, std::size_t m) : dim_(dim), 
 }
 
 // ProductQuantizer::train of the reference (src/product_quantizer.cc:126-153): one 256-way k-means
-// per sub-space over that sub-space's columns, seeded seed + j, whose assignment steps run on the
-// device. The draws and sums must follow the reference's for a bit-identical codebook.
+// per sub-space over that sub-space's columns, seeded seed + j (kmeans.cc: what runs on the
+// device). The draws and sums must follow the reference's for a bit-identical codebook.
 void ProductQuantizer::train(const float* vectors, std::size_t n, ThreadPool* pool, std::size_t iterations,
                              std::uint64_t seed) {
   QUIVER_CHECK(m_ > 0, "PQ is not configured");

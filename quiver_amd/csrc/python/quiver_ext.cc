@@ -480,5 +480,5 @@ PYBIND11_MODULE(_quiver, m) {
       },
       py::arg("vectors"), py::arg("k"), py::arg("iterations") = 25, py::arg("max_points_per_centroid") = 256,
       py::arg("seed") = 1234, py::arg("num_threads") = 0,
-      "Lloyd's k-means (the reference's kmeans), assignment steps on the GPU.");
+      "Lloyd's k-means (the reference's kmeans), assignments and, where clusters are many or wide, means on the GPU.");
 }
