@@ -58,12 +58,15 @@ std::size_t device_means_limit(std::size_t n, std::size_t nsub, std::size_t dsub
   if (k > 256 * dsub || n >= 0xFFFFFFFFull) return 0;
   const double points = static_cast<double>(n), dims = static_cast<double>(dsub);
   const bool cached = points * dims * static_cast<double>(nsub) * sizeof(float) <= 48e6;
-  const double host_ns = dsub <= 8 ? 1.2 + 0.35 * dims : cached ? 3.5 + 0.12 * dims : 18.0 + 0.08 * dims;
+  // 40 us an iteration for the copy down and the threads' start (2,000 x 16, k = 8, 20 iterations: 1.0 ms on
+  // the device, 1.9 on the host).
+  const double each = dsub <= 8 ? 1.2 + 0.35 * dims : cached ? 3.5 + 0.12 * dims : 18.0 + 0.08 * dims;
+  const double host_ns = static_cast<double>(nsub) * each + 40e3 / points;
   const double device_ns = 1.7 + (dsub <= 8 ? 0.0 : 0.06 * dims);
-  const double even = (static_cast<double>(nsub) * host_ns - device_ns) / (dsub <= 64 ? 45.0 : 78.0);
+  const double even = (host_ns - device_ns) / (dsub <= 64 ? 45.0 : 78.0);
   // Past 8 dims more than the break-even: a first iteration's clusters are the least even ones, and the
-  // host loses the more the fewer its threads and the more the points.
-  const double lenient = dsub <= 8 ? 1.0 : dsub <= 16 ? 2.0 : 3.0;
+  // host loses the more the fewer its threads.
+  const double lenient = dsub <= 8 ? 1.0 : !cached ? 1.5 : dsub <= 16 || dsub > 64 ? 2.0 : 3.0;
   const auto limit = static_cast<std::size_t>(std::clamp(lenient * even, 0.0, 1.0) * points);
   // Some cluster holds at least n / k points, and of many the largest about three times that.
   return points * (dsub <= 8 ? 3.0 : 1.0) > static_cast<double>(limit) * static_cast<double>(k) ? 0 : limit;
