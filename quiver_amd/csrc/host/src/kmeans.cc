@@ -51,8 +51,8 @@ void split_empty_clusters(float* cent, Count* counts, std::size_t k, std::size_t
 ///                   128 dims   19, 32      19, 16     20, 12     20, 9.3
 ///   500,000          16 dims  4.2, 15     3.9, 7.0   4.0, 3.9   5.1, 2.8
 ///                    64 dims   26, 19      23, 8.8    22, 5.8    22, 5.4
-/// (1 dim is the host's at every k up to 256, 2 dims up to 512; with points past the host's caches
-/// its sums wait for memory.) Past 256 centroids a dimension the device's reads of every assignment
+/// (At these sizes 1 dim is the host's at every k up to 256, 2 dims up to 512; with points past the
+/// host's caches its sums wait for memory.) Past 256 centroids a dimension the device's reads of every assignment
 /// per centroid are left to the host's sums too.
 std::size_t device_means_limit(std::size_t n, std::size_t nsub, std::size_t dsub, std::size_t k) {
   if (k > 256 * dsub || n >= 0xFFFFFFFFull) return 0;
